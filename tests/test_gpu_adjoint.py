@@ -78,6 +78,39 @@ def test_adjoint_step_matches_oracle(case, storage, tol):
         assert rel_max(gg.cpu().numpy().reshape(3, Z, Y), gh) < tol
 
 
+@pytest.mark.parametrize("shape", [(1, 6, 5), (2, 5, 6), (3, 66, 4), (5, 1, 7), (4, 2, 3), (3, 97, 5), (4, 256, 3)])
+@pytest.mark.parametrize("storage,tol", [("f64", 1e-12), ("f32", 2e-5)])
+def test_adjoint_step_at_the_edges_of_its_shapes(shape, storage, tol):
+    """Extents of one and two sites (where the wrap and the clamp of a pull meet),
+    rows that end inside a wave and rows of whole blocks, from the state and
+    from a recording, against the oracle's adjoint."""
+    import ctypes as C
+
+    from pytnl_lbm.adjoint import tape_elements
+    from pytnl_lbm.lattice import _ptr, _stream_ptr
+    X, Y, Z = shape
+    g, h, w = setup("outflow_right", storage, X, Y, Z)
+    wq = from_dev(to_dev(w, TORCH[storage]), X, Y, Z)
+    gh = np.zeros((3, Z, Y))
+    ref = h.adjoint_step(wq, grad=gh, which=0)
+    ln = to_dev(wq, TORCH[storage])
+    tape = torch.zeros(tape_elements(g.d.XYZ), dtype=TORCH[storage], device="cuda")
+    g.d.even_iter = 1
+    g._check(g.lib.tnl_lbm_d3q27_step_record(C.byref(g.cfg), C.byref(g.d), _ptr(tape), int(storage == "f64"), _stream_ptr()))
+    for recorded in (False, True):
+        lam = torch.empty(27 * g.d.XYZ, dtype=TORCH[storage], device="cuda")
+        gg = torch.zeros(3 * Y * Z, dtype=torch.float64, device="cuda")
+        if recorded:
+            g._check(g.lib.tnl_lbm_d3q27_adjoint_step_recorded(C.byref(g.cfg), C.byref(g.d), _ptr(tape), int(storage == "f64"),
+                                                               _ptr(ln), _ptr(lam), _ptr(gg), _stream_ptr()))
+        else:
+            g.adjoint_step(ln, lam, gg, which=0)
+        torch.cuda.synchronize()
+        assert rel_max(from_dev(lam, X, Y, Z), ref) < tol, (recorded, rel_max(from_dev(lam, X, Y, Z), ref))
+        if np.abs(gh).max() > 0:
+            assert rel_max(gg.cpu().numpy().reshape(3, Z, Y), gh) < tol
+
+
 def test_adjoint_rejects_unsupported_configurations():
     g = D3Q27Lattice(4, 4, 4, pattern="AA", nu=0.02)
     lam = torch.zeros(27 * g.d.XYZ, dtype=torch.float64, device="cuda")

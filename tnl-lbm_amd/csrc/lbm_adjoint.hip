@@ -12,17 +12,8 @@ int adjoint_for(const StepArgs& A0, const AdjPtrs& P, unsigned threads, unsigned
 {
 	StepArgs A = A0;
 	linearize(A, threads, grid);
-	// FP64: 32-bit slot offsets where every population array (state, lambda
-	// in and out) holds at most 4 GiB: 2 spilled registers instead of 4 and
-	// -68 VALU, ~2% faster on the C4 duct; FP32 measured ~2% slower with them
-	constexpr bool F64MATH = std::is_same<typename Storage<ST>::real, double>::value;
-	bool o32 = false;
-	if constexpr (F64MATH)
-		o32 = narrow_slots(A.XYZ, sizeof(typename Storage<ST>::elem));
-	if (o32) {
-		if constexpr (F64MATH)
-			hipLaunchKernelGGL((k_adjoint_ab<ST, false, TAPE, true>), dim3(grid), dim3(threads), 0, st, A, P);
-	}
+	if (narrow_planes(A, sizeof(typename Storage<ST>::elem)))
+		hipLaunchKernelGGL((k_adjoint_ab<ST, false, TAPE, true>), dim3(grid), dim3(threads), 0, st, A, P);
 	else
 		hipLaunchKernelGGL((k_adjoint_ab<ST, false, TAPE>), dim3(grid), dim3(threads), 0, st, A, P);
 	if (int rc = hip_check(hipGetLastError(), "adjoint launch"))

@@ -25,127 +25,112 @@ struct AdjCum
 	static constexpr int NMOM = 10;
 	static LBM_DEV void raw_moments(const real* f, real* m) { raw_moments10(f, m); }
 
-	// forward backward-pass of one column, absolute form:
-	//   fz = k0 (1 - v^2) - 2 v k1 - k2,  f-+ = (k0 (v^2 -+ v) + k1 (2 v -+ 1) + k2) / 2
-	static LBM_DEV void bwd(real k0, real k1, real k2, real v, real& fm, real& fz, real& fp)
+	// The backward central-moment transform of one column (k0, k1, k2) along an
+	// axis of velocity v is f = V^-1 S(v) k: the shift of the central moments to
+	// raw ones, m = S(v) k with
+	//   m0 = k0,  m1 = k1 + v k0,  m2 = k2 + 2 v k1 + v^2 k0,
+	// then f_-+ = (m2 -+ m1) / 2, f_0 = m0 - m2.  Its transpose takes
+	// (lm, lz, lp) to (l0, l1, l2).
+	static LBM_DEV void bwd_adj(real v, real lm, real lz, real lp, real& l0, real& l1, real& l2)
 	{
-		const real v2 = v * v;
-		fz = k0 * ((real) 1 - v2) - (real) 2 * v * k1 - k2;
-		fm = (k0 * (v2 - v) + k1 * ((real) 2 * v - (real) 1) + k2) * (real) 0.5;
-		fp = (k0 * (v2 + v) + k1 * ((real) 2 * v + (real) 1) + k2) * (real) 0.5;
-	}
-	// its adjoint: (lm, lz, lp) -> (l0, l1, l2), and d/dv accumulated into lv
-	static LBM_DEV void bwd_adj(real k0, real k1, real v, real lm, real lz, real lp, real& l0, real& l1, real& l2, real& lv)
-	{
-		const real S = (real) 0.5 * (lm + lp);
 		const real d = (real) 0.5 * (lp - lm);
-		l2 = S - lz;
-		l1 = (real) 2 * v * l2 + d;
-		l0 = v * (v * l2 + d) + lz;
-		lv += k0 * l1 + (real) 2 * k1 * l2;
+		l2 = (real) 0.5 * (lp + lm) - lz;
+		const real t = v * l2 + d;
+		l0 = v * t + lz;
+		l1 = v * l2 + t;
 	}
 
-	// mu = (d f_out / d f_in)^T lam for the collision at the pre-collision
-	// populations f.  rho_fixed: the caller has replaced rho by 1 before the
-	// collision (OUTFLOW_RIGHT, bc.h:191-194): the 4th/6th-order products then
-	// divide by 1 while u and the trace keep the actual mass.
-	template <typename L, typename Mu>
-	static LBM_DEV void vjp(const real* f, const L* lam, real Fx, real Fy, real Fz, real omega1, bool rho_fixed, Mu* mu)
+	// (d f_out / d f_in)^T lam for the collision, from the raw moments of the
+	// pre-collision populations, which are all the Jacobian of the default
+	// cumulant depends on.  The result is mu = M^T l: `l` holds the ten
+	// cotangents of the raw moments in the order of raw_moments10, and
+	// for_each_mu spreads them over the populations.  rho_fixed: the caller
+	// has replaced rho by 1 before the collision (OUTFLOW_RIGHT,
+	// bc.h:191-194): the 4th/6th-order products then divide by 1 while u and
+	// the trace keep the actual mass.  lam may be held in a narrower type than
+	// the arithmetic (float fields, double sweep).
+	//
+	// The velocity's cotangent needs no forward recomputation of the chain:
+	// S(v) = exp(v N) with N k = (0, k0, 2 k1), so d/dv of a column's output is
+	// the transform applied to N k, the transforms along different axes
+	// commute, and
+	//   d/dv_a <lam, f_out> = <lK, N_a K>
+	// with K the post-collision central moments and lK = lam pulled back
+	// through all three passes.  That leaves one array of 27 values live (the
+	// recomputed intermediate populations of the two earlier passes, 54
+	// doubles, set the register count before) and half the operations.
+	template <typename L>
+	static LBM_DEV void vjp_m(const real* m, const L* lam, real Fx, real Fy, real Fz, real omega1, bool rho_fixed, real* l)
 	{
-		real m[NMOM];
-		raw_moments(f, m);
-		vjp_m(m, lam, Fx, Fy, Fz, omega1, rho_fixed, mu);
-	}
-
-	// the same from the raw moments of the pre-collision populations, which
-	// are all the Jacobian of the default cumulant depends on.  lam and mu may
-	// be held in a narrower type than the arithmetic (float fields, double
-	// sweep): each value is widened where it is read and rounded once where
-	// it is written.
-	template <typename L, typename Mu>
-	static LBM_DEV void vjp_m(const real* m, const L* lam, real Fx, real Fy, real Fz, real omega1, bool rho_fixed, Mu* mu)
-	{
-		// ---- forward recomputation ---------------------------------------
-		const real m0 = m[0], jx = m[1], jy = m[2], jz = m[3], Pxx = m[4], Pyy = m[5], Pzz = m[6], Pxy = m[7], Pxz = m[8],
-				   Pyz = m[9];
 		const real hx = (real) 0.5 * Fx, hy = (real) 0.5 * Fy, hz = (real) 0.5 * Fz;
+		const real m0 = m[0];
 		const real rv = (real) 1 / m0;
-		const real vx = (jx + hx) * rv, vy = (jy + hy) * rv, vz = (jz + hz) * rv;
+		const real vx = (m[1] + hx) * rv, vy = (m[2] + hy) * rv, vz = (m[3] + hz) * rv;
+		// ---- the collision's central moments (m0 u - j = F/2 throughout) --------
 		const real rk = rho_fixed ? (real) 1 : rv;
-		const real k200 = Pxx - vx * ((real) 2 * jx - m0 * vx);
-		const real k020 = Pyy - vy * ((real) 2 * jy - m0 * vy);
-		const real k002 = Pzz - vz * ((real) 2 * jz - m0 * vz);
-		const real k110 = Pxy - vx * jy - vy * (jx - m0 * vx);
-		const real k101 = Pxz - vx * jz - vz * (jx - m0 * vx);
-		const real k011 = Pyz - vy * jz - vz * (jy - m0 * vy);
 		const real om = (real) 1 - omega1;
 		const real third = (real) (1.0 / 3.0);
-		const real E33 = om * (k200 - k020), E34 = om * (k200 - k002), E35 = m0;
-		const real a = third * (E33 + E34 + E35);
-		const real b = third * (-(real) 2 * E33 + E34 + E35);
-		const real c = third * (E33 - (real) 2 * E34 + E35);
-		const real s = om * k110, p = om * k101, qq = om * k011;
-		const real X211 = a * qq + (real) 2 * p * s, X121 = b * p + (real) 2 * s * qq, X112 = c * s + (real) 2 * qq * p;
-		const real X220 = b * a + (real) 2 * s * s, X022 = c * b + (real) 2 * qq * qq, X202 = a * c + (real) 2 * p * p;
-		const real ks211 = X211 * rk, ks121 = X121 * rk, ks112 = X112 * rk;
-		const real ks220 = X220 * rk, ks022 = X022 * rk, ks202 = X202 * rk;
-		const real Y1 = a * ks022 + b * ks202 + c * ks220 + (real) 4 * (qq * ks211 + p * ks121 + s * ks112);
-		const real Y2 = (real) 16 * s * p * qq + (real) 4 * (p * p * b + qq * qq * a + s * s * c) + (real) 2 * a * b * c;
-		const real ks222 = Y1 * rk - Y2 * rk * rk;
-		// x-pass column inputs K[j][k][m] (moment m along x; j, k along y, z)
-		real K[3][3][3];
-		K[0][0][0] = m0;    K[0][0][1] = hx;    K[0][0][2] = a;
-		K[1][0][0] = hy;    K[1][0][1] = s;     K[1][0][2] = 0;
-		K[2][0][0] = b;     K[2][0][1] = 0;     K[2][0][2] = ks220;
-		K[0][1][0] = hz;    K[0][1][1] = p;     K[0][1][2] = 0;
-		K[1][1][0] = qq;    K[1][1][1] = 0;     K[1][1][2] = ks211;
-		K[2][1][0] = 0;     K[2][1][1] = ks121; K[2][1][2] = 0;
-		K[0][2][0] = c;     K[0][2][1] = 0;     K[0][2][2] = ks202;
-		K[1][2][0] = 0;     K[1][2][1] = ks112; K[1][2][2] = 0;
-		K[2][2][0] = ks022; K[2][2][1] = 0;     K[2][2][2] = ks222;
-		real U[3][3][3], T[3][3][3];  // U[i][j][k]: x position i; T[i][j][k]: x, y positions i, j
-#pragma unroll
-		for (int j = 0; j < 3; j++)
-#pragma unroll
-			for (int k = 0; k < 3; k++)
-				bwd(K[j][k][0], K[j][k][1], K[j][k][2], vx, U[0][j][k], U[1][j][k], U[2][j][k]);
-#pragma unroll
-		for (int i = 0; i < 3; i++)
-#pragma unroll
-			for (int k = 0; k < 3; k++)
-				bwd(U[i][0][k], U[i][1][k], U[i][2][k], vy, T[i][0][k], T[i][1][k], T[i][2][k]);
-
-		// ---- reverse sweep ---------------------------------------------------
-		real lvx = 0, lvy = 0, lvz = 0;
-		real lT[3][3][3], lU[3][3][3], lK[3][3][3];
+		real a, b, c, s, p, qq;
+		{
+			const real k200 = m[4] - vx * (m[1] - hx), k020 = m[5] - vy * (m[2] - hy), k002 = m[6] - vz * (m[3] - hz);
+			const real E33 = om * (k200 - k020), E34 = om * (k200 - k002);
+			a = third * (E33 + E34 + m0);
+			b = third * (-(real) 2 * E33 + E34 + m0);
+			c = third * (E33 - (real) 2 * E34 + m0);
+			s = om * (m[7] - vx * m[2] + vy * hx);
+			p = om * (m[8] - vx * m[3] + vz * hx);
+			qq = om * (m[9] - vy * m[3] + vz * hy);
+		}
+		const real ks211 = (a * qq + (real) 2 * p * s) * rk, ks121 = (b * p + (real) 2 * s * qq) * rk,
+				   ks112 = (c * s + (real) 2 * qq * p) * rk;
+		const real ks220 = (b * a + (real) 2 * s * s) * rk, ks022 = (c * b + (real) 2 * qq * qq) * rk,
+				   ks202 = (a * c + (real) 2 * p * p) * rk;
+		// the schedule keeps these three phases apart (moments, the passes over
+		// lam, the products' reverse): mixed, their live values spill
+		__builtin_amdgcn_sched_barrier(0);
+		// ---- lam through the three passes, z first: cotangents lK[i][j][k] of K ---
+		real lK[3][3][3];
 #pragma unroll
 		for (int i = 0; i < 3; i++)
 #pragma unroll
 			for (int j = 0; j < 3; j++)
-				bwd_adj(T[i][j][0], T[i][j][1], vz, lam[qidx(i, j, 0)], lam[qidx(i, j, 1)], lam[qidx(i, j, 2)], lT[i][j][0],
-						lT[i][j][1], lT[i][j][2], lvz);
+				bwd_adj(vz, (real) lam[qidx(i, j, 0)], (real) lam[qidx(i, j, 1)], (real) lam[qidx(i, j, 2)], lK[i][j][0], lK[i][j][1],
+						lK[i][j][2]);
 #pragma unroll
 		for (int i = 0; i < 3; i++)
 #pragma unroll
 			for (int k = 0; k < 3; k++)
-				bwd_adj(U[i][0][k], U[i][1][k], vy, lT[i][0][k], lT[i][1][k], lT[i][2][k], lU[i][0][k], lU[i][1][k], lU[i][2][k], lvy);
+				bwd_adj(vy, lK[i][0][k], lK[i][1][k], lK[i][2][k], lK[i][0][k], lK[i][1][k], lK[i][2][k]);
 #pragma unroll
 		for (int j = 0; j < 3; j++)
 #pragma unroll
 			for (int k = 0; k < 3; k++)
-				bwd_adj(K[j][k][0], K[j][k][1], vx, lU[0][j][k], lU[1][j][k], lU[2][j][k], lK[j][k][0], lK[j][k][1], lK[j][k][2], lvx);
+				bwd_adj(vx, lK[0][j][k], lK[1][j][k], lK[2][j][k], lK[0][j][k], lK[1][j][k], lK[2][j][k]);
+		// d/dv_a: <lK, N_a K> over the columns whose K is not identically zero
+		real lvx = lK[1][0][0] * m0 + lK[1][1][0] * hy + lK[1][0][1] * hz + lK[1][2][0] * b + lK[1][1][1] * qq + lK[1][0][2] * c
+				 + lK[1][2][2] * ks022
+				 + (real) 2 * (lK[2][0][0] * hx + lK[2][1][0] * s + lK[2][0][1] * p + lK[2][2][1] * ks121 + lK[2][1][2] * ks112);
+		real lvy = lK[0][1][0] * m0 + lK[1][1][0] * hx + lK[0][1][1] * hz + lK[2][1][0] * a + lK[1][1][1] * p + lK[0][1][2] * c
+				 + lK[2][1][2] * ks202
+				 + (real) 2 * (lK[0][2][0] * hy + lK[1][2][0] * s + lK[0][2][1] * qq + lK[2][2][1] * ks211 + lK[1][2][2] * ks112);
+		real lvz = lK[0][0][1] * m0 + lK[1][0][1] * hx + lK[0][1][1] * hy + lK[2][0][1] * a + lK[1][1][1] * s + lK[0][2][1] * b
+				 + lK[2][2][1] * ks220
+				 + (real) 2 * (lK[0][0][2] * hz + lK[1][0][2] * p + lK[0][1][2] * qq + lK[2][1][2] * ks211 + lK[1][2][2] * ks121);
+		__builtin_amdgcn_sched_barrier(0);
+		// ---- the products' reverse sweep ---------------------------------------
 		// (the first-order inputs hx, hy, hz are constants: post-collision
 		// k_100 = -(j_x - m0 u_x) = F_x / 2 identically)
 		real lm0 = lK[0][0][0];
-		real la = lK[0][0][2], lb = lK[2][0][0], lc = lK[0][2][0];
-		real ls = lK[1][0][1], lp = lK[0][1][1], lqq = lK[1][1][0];
-		real lks220 = lK[2][0][2], lks211 = lK[1][1][2], lks121 = lK[2][1][1], lks202 = lK[0][2][2], lks112 = lK[1][2][1];
-		real lks022 = lK[2][2][0];
+		real la = lK[2][0][0], lb = lK[0][2][0], lc = lK[0][0][2];
+		real ls = lK[1][1][0], lp = lK[1][0][1], lqq = lK[0][1][1];
+		real lks220 = lK[2][2][0], lks211 = lK[2][1][1], lks121 = lK[1][2][1], lks202 = lK[2][0][2], lks112 = lK[1][1][2];
+		real lks022 = lK[0][2][2];
 		const real lks222 = lK[2][2][2];
-		real lrk = 0;
-		// ks222 = Y1 rk - Y2 rk^2
-		const real lY1 = lks222 * rk, lY2 = -lks222 * rk * rk;
-		lrk += lks222 * (Y1 - (real) 2 * Y2 * rk);
+		// ks222 = Y1 rk - Y2 rk^2; lr collects rk d/d(rk) of the products
+		const real Y1 = a * ks022 + b * ks202 + c * ks220 + (real) 4 * (qq * ks211 + p * ks121 + s * ks112);
+		const real Y2 = (real) 16 * s * p * qq + (real) 4 * (p * p * b + qq * qq * a + s * s * c) + (real) 2 * a * b * c;
+		const real lY1 = lks222 * rk, lY2 = -lY1 * rk;
+		real lr = lY1 * Y1 + (real) 2 * lY2 * Y2;
 		la += lY1 * ks022; lks022 += lY1 * a;
 		lb += lY1 * ks202; lks202 += lY1 * b;
 		lc += lY1 * ks220; lks220 += lY1 * c;
@@ -159,7 +144,7 @@ struct AdjCum
 		la += lY2 * ((real) 4 * qq * qq + (real) 2 * b * c);
 		lc += lY2 * ((real) 4 * s * s + (real) 2 * a * b);
 		// ks_xyz = X_xyz rk
-		lrk += lks211 * X211 + lks121 * X121 + lks112 * X112 + lks220 * X220 + lks022 * X022 + lks202 * X202;
+		lr += lks211 * ks211 + lks121 * ks121 + lks112 * ks112 + lks220 * ks220 + lks022 * ks022 + lks202 * ks202;
 		const real l211 = lks211 * rk, l121 = lks121 * rk, l112 = lks112 * rk;
 		const real l220 = lks220 * rk, l022 = lks022 * rk, l202 = lks202 * rk;
 		la += l211 * qq; lqq += l211 * a; lp += (real) 2 * l211 * s; ls += (real) 2 * l211 * p;
@@ -168,32 +153,55 @@ struct AdjCum
 		lb += l220 * a; la += l220 * b; ls += (real) 4 * l220 * s;
 		lc += l022 * b; lb += l022 * c; lqq += (real) 4 * l022 * qq;
 		la += l202 * c; lc += l202 * a; lp += (real) 4 * l202 * p;
-		// a, b, c <- E33, E34, E35 = m0
+		// a, b, c <- E33, E34, m0
 		const real lE33 = third * (la - (real) 2 * lb + lc);
 		const real lE34 = third * (la + lb - (real) 2 * lc);
 		lm0 += third * (la + lb + lc);
 		const real lk200 = om * (lE33 + lE34), lk020 = -om * lE33, lk002 = -om * lE34;
 		const real lk110 = om * ls, lk101 = om * lp, lk011 = om * lqq;
-		if (! rho_fixed)
-			lm0 -= lrk * rk * rk;
-		// central moments <- raw moments, velocity, mass
-		real ljx = 0, ljy = 0, ljz = 0;
-		lvx += lk200 * ((real) 2 * (m0 * vx - jx)); ljx -= (real) 2 * vx * lk200; lm0 += vx * vx * lk200;
-		lvy += lk020 * ((real) 2 * (m0 * vy - jy)); ljy -= (real) 2 * vy * lk020; lm0 += vy * vy * lk020;
-		lvz += lk002 * ((real) 2 * (m0 * vz - jz)); ljz -= (real) 2 * vz * lk002; lm0 += vz * vz * lk002;
-		lvx += lk110 * (m0 * vy - jy); lvy += lk110 * (m0 * vx - jx); ljy -= vx * lk110; ljx -= vy * lk110; lm0 += vx * vy * lk110;
-		lvx += lk101 * (m0 * vz - jz); lvz += lk101 * (m0 * vx - jx); ljz -= vx * lk101; ljx -= vz * lk101; lm0 += vx * vz * lk101;
-		lvy += lk011 * (m0 * vz - jz); lvz += lk011 * (m0 * vy - jy); ljz -= vy * lk011; ljy -= vz * lk011; lm0 += vy * vz * lk011;
+		// rk = 1 / m0 unless the caller fixed rho
+		lm0 -= rho_fixed ? (real) 0 : lr * rk;
+		// central moments <- raw moments, velocity, mass (m0 u - j = F/2)
+		lvx += (real) 2 * hx * lk200 + hy * lk110 + hz * lk101;
+		lvy += (real) 2 * hy * lk020 + hx * lk110 + hz * lk011;
+		lvz += (real) 2 * hz * lk002 + hx * lk101 + hy * lk011;
+		const real tx = vx * lk200, ty = vy * lk020, tz = vz * lk002;
+		lm0 += vx * (tx + vy * lk110 + vz * lk101) + vy * (ty + vz * lk011) + vz * tz;
 		// u = (j + F/2) / m0
-		ljx += lvx * rv; ljy += lvy * rv; ljz += lvz * rv;
-		lm0 -= (lvx * vx + lvy * vy + lvz * vz) * rv;
-		// raw moments are linear in f
+		const real ux = lvx * rv, uy = lvy * rv, uz = lvz * rv;
+		const real ljx = ux - (real) 2 * tx - vy * lk110 - vz * lk101;
+		const real ljy = uy - (real) 2 * ty - vx * lk110 - vz * lk011;
+		const real ljz = uz - (real) 2 * tz - vx * lk101 - vy * lk011;
+		lm0 -= ux * vx + uy * vy + uz * vz;
+		l[0] = lm0; l[1] = ljx; l[2] = ljy; l[3] = ljz; l[4] = lk200; l[5] = lk020; l[6] = lk002; l[7] = lk110; l[8] = lk101;
+		l[9] = lk011;
+	}
+
+	// mu = M^T l, the raw moments being linear in the populations: put(q, mu_q)
+	// for every q, by (c_x, c_y) columns of one base and one z-odd part.
+	template <typename Put>
+	static LBM_DEV void for_each_mu(const real* l, Put&& put)
+	{
 #pragma unroll
-		for (int q = 0; q < 27; q++) {
-			const real cx = (real) CX[q], cy = (real) CY[q], cz = (real) CZ[q];
-			mu[q] = (Mu) (lm0 + cx * ljx + cy * ljy + cz * ljz + (cx * cx) * lk200 + (cy * cy) * lk020 + (cz * cz) * lk002
-						  + (cx * cy) * lk110 + (cx * cz) * lk101 + (cy * cz) * lk011);
-		}
+		for (int i = 0; i < 3; i++)
+#pragma unroll
+			for (int j = 0; j < 3; j++) {
+				real e = l[0], o = l[3];
+				if (i != 1) {
+					e += i == 2 ? l[4] + l[1] : l[4] - l[1];
+					o += i == 2 ? l[8] : -l[8];
+				}
+				if (j != 1) {
+					e += j == 2 ? l[5] + l[2] : l[5] - l[2];
+					o += j == 2 ? l[9] : -l[9];
+				}
+				if (i != 1 && j != 1)
+					e += i == j ? l[7] : -l[7];
+				const real ez = e + l[6];
+				put(qidx(i, j, 0), ez - o);
+				put(qidx(i, j, 1), e);
+				put(qidx(i, j, 2), ez + o);
+			}
 	}
 
 	// gradient with respect to u of sum_q lam_q feq_q(1, u), feq = D3Q27_EQ_INV_CUM
@@ -294,21 +302,60 @@ LBM_DEV bool shell_coords(const StepArgs& A, int64_t& x, int64_t& z, int64_t& y)
 	return false;
 }
 
+// Whether the periodic-wrap slot of direction q differs from the slot the
+// site really pulls from, as a bit per direction.  Per axis a pull towards -1
+// or +1 is irregular where the wrap and the clamp differ (a non-periodic site
+// on that face of the box); OUTFLOW_RIGHT pulls c_x = 0 and -1 from x - 1.
+constexpr uint32_t dir_mask(int axis, int c)
+{
+	uint32_t m = 0;
+	for (int q = 0; q < 27; q++)
+		if ((axis == 0 ? CX[q] : axis == 1 ? CY[q] : CZ[q]) == c)
+			m |= 1u << q;
+	return m;
+}
+LBM_DEV uint32_t irregular_pulls(bool per, bool right, int32_t x, int32_t y, int32_t z, int32_t X, int32_t Y, int32_t Z)
+{
+	uint32_t m = 0;
+	if (! per) {
+		m |= x == 0 && X > 1 ? dir_mask(0, 1) : 0;
+		m |= x == X - 1 && X > 1 && ! right ? dir_mask(0, -1) : 0;
+		m |= y == 0 && Y > 1 ? dir_mask(1, 1) : 0;
+		m |= y == Y - 1 && Y > 1 ? dir_mask(1, -1) : 0;
+		m |= z == 0 && Z > 1 ? dir_mask(2, 1) : 0;
+		m |= z == Z - 1 && Z > 1 ? dir_mask(2, -1) : 0;
+	}
+	if (right) {
+		m |= x > 0 ? dir_mask(0, 0) : 0;
+		m |= X > 2 || x < X - 1 ? dir_mask(0, -1) : 0;
+	}
+	return m;
+}
+
 // SPECIAL = false: every site, plain stores to the slots it owns under the
 // periodic wrap (0 for slots whose true reader is elsewhere).  SPECIAL = true:
 // the face sites only, atomic adds of those contributions to their true
 // sources, after the first pass.
-// (256, 2): two waves per SIMD; the FP64 form then spills a few registers
-// instead of running one wave per SIMD at 264
-template <int ST, bool SPECIAL, int TAPE = 0, bool O32 = false>
-__global__ void __launch_bounds__(256, 2) k_adjoint_ab(const StepArgs A, const AdjPtrs P)
+//
+// P32: one x plane of a population array holds at most 4 GiB.  A block lies in
+// one x plane in every mapping, so the first pass addresses a slot as a
+// wave-uniform base (array, direction and x plane) plus a 32-bit per-lane
+// offset within the plane.
+//
+// Bound: HBM, then FP64 issue (about 500 FP64 instructions a site).  Four
+// waves per SIMD (at most 128 VGPRs; from an FP64 state, whose 27 pulled values
+// meet the 27 of lambda, three): 256x96x96 duct, float fields and recording,
+// 164 -> 145 us (4.2 TB/s) against the sweep that recomputed the chain's
+// intermediate populations at 256 VGPRs and two waves.
+template <int ST, bool SPECIAL, int TAPE = 0, bool P32 = false>
+__global__ void __launch_bounds__(256, (TAPE == 0 && ST == TNL_LBM_STORE_F64) ? 3 : 4) k_adjoint_ab(const StepArgs A, const AdjPtrs P)
 {
 	using S = Storage<ST>;
 	using real = typename S::real;
 	using elem = typename S::elem;
 	using D = AdjCum<real>;
-	// lambda in and mu out in the element type where it is narrower than the
-	// arithmetic (float fields with a double sweep): fewer registers
+	// lambda in the element type where it is narrower than the arithmetic
+	// (float fields with a double sweep): fewer registers
 	using lreal = std::conditional_t<(sizeof(elem) < sizeof(real)), elem, real>;
 	int64_t x, z, y;
 	if (SPECIAL ? ! shell_coords(A, x, z, y) : ! block_coords(A, x, z, y))
@@ -316,36 +363,32 @@ __global__ void __launch_bounds__(256, 2) k_adjoint_ab(const StepArgs A, const A
 	const int64_t s0 = (x * A.Zs + z) * A.Ys + y;
 	const int16_t gi = A.map ? A.map[s0] : (int16_t) GEO_PERIODIC;
 	const bool per = gi == GEO_PERIODIC;
-	const Nb NX = neighbours<false>(x, A.X, 0, false, per);
-	const Nb NY = neighbours<false>(y, A.Y, 0, false, per);
-	const Nb NZ = neighbours<false>(z, A.Z, 0, false, per);
-	Nb PX = NX;
-	if (gi == GEO_OUTFLOW_RIGHT)
-		PX.p = PX.o = NX.m;
-	const Nb WX = neighbours<false>(x, A.X, 0, false, true);
-	const Nb WY = neighbours<false>(y, A.Y, 0, false, true);
-	const Nb WZ = neighbours<false>(z, A.Z, 0, false, true);
-	auto sidx = [&](int64_t xs, int64_t ys, int64_t zs) { return (xs * A.Zs + zs) * A.Ys + ys; };
-	uint32_t irregular = 0;
-#pragma unroll
-	for (int q = 0; q < 27; q++) {
-		const bool same = PX[-CX[q]] == WX[-CX[q]] && NY[-CY[q]] == WY[-CY[q]] && NZ[-CZ[q]] == WZ[-CZ[q]];
-		if (gi == GEO_NOTHING || ! same)
-			irregular |= 1u << q;
-	}
+	const uint32_t irregular = gi == GEO_NOTHING ? (1u << 27) - 1
+												 : irregular_pulls(per, gi == GEO_OUTFLOW_RIGHT, (int32_t) x, (int32_t) y, (int32_t) z,
+																   (int32_t) A.X, (int32_t) A.Y, (int32_t) A.Z);
 	if (SPECIAL && (gi == GEO_NOTHING || irregular == 0))
 		return;
+	// the slot of direction q at (xs, ys, zs); xs is wave-uniform in the first
+	// pass except for the pulls
+	auto slot_at = [&](auto* base, int q, int64_t xs, int64_t ys, int64_t zs) {
+		if constexpr (P32 && ! SPECIAL)
+			return at(base + (q * A.XYZ + xs * A.Zs * A.Ys), (uint32_t) zs * (uint32_t) A.Ys + (uint32_t) ys);
+		else
+			return base + (q * A.XYZ + (xs * A.Zs + zs) * A.Ys + ys);
+	};
+	const elem* __restrict__ Ln = (const elem*) P.lam_next;
+	elem* __restrict__ L = (elem*) P.lam;
 	if (SPECIAL && (gi == GEO_WALL || gi == GEO_INFLOW)) {
 		// bounce-back: mu_q = lam_next[opp(q)], read only for the irregular directions
 		// (the face sites are one per cache line here); inflow: mu = 0
 		if (gi == GEO_WALL) {
-			const elem* Ln = (const elem*) P.lam_next;
-			elem* L = (elem*) P.lam;
+			const Nb NX = neighbours<false>(x, A.X, 0, false, false);
+			const Nb NY = neighbours<false>(y, A.Y, 0, false, false);
+			const Nb NZ = neighbours<false>(z, A.Z, 0, false, false);
 #pragma unroll
 			for (int q = 0; q < 27; q++)
 				if ((irregular >> q) & 1u)
-					atomicAdd(L + q * A.XYZ + sidx(PX[-CX[q]], NY[-CY[q]], NZ[-CZ[q]]),
-							  (elem) S::ld(Ln + opp(q) * A.XYZ + s0));
+					atomicAdd(slot_at(L, q, NX[-CX[q]], NY[-CY[q]], NZ[-CZ[q]]), (elem) S::ld(Ln + opp(q) * A.XYZ + s0));
 		}
 		return;
 	}
@@ -353,108 +396,96 @@ __global__ void __launch_bounds__(256, 2) k_adjoint_ab(const StepArgs A, const A
 	// an irregular pull away from the faces (OUTFLOW_RIGHT inside the box) has no fix-up: poison it
 	const bool unsupported = gi != GEO_NOTHING && irregular != 0 && ! on_shell;
 
-	lreal mu[27];
-	if (gi == GEO_NOTHING || unsupported) {
-		const lreal v = unsupported ? (lreal) __builtin_nan("") : (lreal) 0;
+	lreal lam[27];
+#pragma unroll
+	for (int q = 0; q < 27; q++)
+		lam[q] = (lreal) S::ld(slot_at(Ln, q, x, y, z));
+	// raw moments of the pulled populations: from the state, or recorded by the
+	// forward step (read at every site, used where the forward step wrote them)
+	Nb PX, NY, NZ;
+	if (SPECIAL || TAPE == 0) {
+		PX = neighbours<false>(x, A.X, 0, false, per);
+		NY = neighbours<false>(y, A.Y, 0, false, per);
+		NZ = neighbours<false>(z, A.Z, 0, false, per);
+		if (gi == GEO_OUTFLOW_RIGHT)
+			PX.p = PX.o = PX.m;
+	}
+	real m[D::NMOM];
+	if constexpr (TAPE == 0) {
+		const elem* F = (const elem*) A.df0;
+		real f[27];
 #pragma unroll
 		for (int q = 0; q < 27; q++)
-			mu[q] = v;
+			f[q] = S::ld(F + (q * A.XYZ + (PX[-CX[q]] * A.Zs + NZ[-CZ[q]]) * A.Ys + NY[-CY[q]]));
+		D::raw_moments(f, m);
 	}
 	else {
-		const elem* Ln = (const elem*) P.lam_next;
-		lreal lam[27];
-#pragma unroll
-		for (int q = 0; q < 27; q++)
-			lam[q] = (lreal) S::ld(slot0<O32, false>(Ln, q, A, s0));
-		// raw moments of the pulled populations: from the state, or recorded by the forward step
-		const bool needs_m = gi == GEO_FLUID || gi == GEO_PERIODIC || gi == GEO_OUTFLOW_RIGHT || gi == GEO_OUTFLOW_EQ;
-		real m[D::NMOM];
+		using TT = std::conditional_t<TAPE == 2, double, float>;
+		const TT* tp = (const TT*) P.tape;
 #pragma unroll
 		for (int k = 0; k < D::NMOM; k++)
-			m[k] = 0;
-		if (needs_m) {
-			if constexpr (TAPE == 0) {
-				const elem* F = (const elem*) A.df0;
-				real f[27];
-#pragma unroll
-				for (int q = 0; q < 27; q++)
-					f[q] = S::ld(slot<O32, false>(F, q, A, PX[-CX[q]], NY[-CY[q]], NZ[-CZ[q]]));
-				D::raw_moments(f, m);
-			}
-			else {
-				using TT = std::conditional_t<TAPE == 2, double, float>;
-				const TT* tp = (const TT*) P.tape;
-#pragma unroll
-				for (int k = 0; k < D::NMOM; k++)
-					m[k] = (real) tp[tape_index(k, s0)];
-			}
-		}
-		switch (gi) {
-			case GEO_FLUID:
-			case GEO_PERIODIC:
-			case GEO_OUTFLOW_RIGHT:
-				D::vjp_m(m, lam, (real) A.fx, (real) A.fy, (real) A.fz, (real) A.omega1, gi == GEO_OUTFLOW_RIGHT, mu);
-				break;
-			case GEO_WALL:
-#pragma unroll
-				for (int q = 0; q < 27; q++)
-					mu[q] = lam[opp(q)];
-				break;
-			case GEO_INFLOW:
-				{
-#pragma unroll
-					for (int q = 0; q < 27; q++)
-						mu[q] = 0;
-					if (! SPECIAL && P.grad) {
-						const int64_t iy = A.Y * z + y;
-						const real ux = (real) inflow_component(A, 0, iy);
-						const real uy = (real) inflow_component(A, 1, iy);
-						const real uz = (real) inflow_component(A, 2, iy);
-						real gx = 0, gy = 0, gz = 0;
-						D::eq_grad(lam, ux, uy, uz, gx, gy, gz);
-						const int64_t n = A.Y * A.Z;
-						atomicAdd(P.grad + iy, (double) gx);
-						atomicAdd(P.grad + n + iy, (double) gy);
-						atomicAdd(P.grad + 2 * n + iy, (double) gz);
-					}
-					break;
-				}
-			case GEO_OUTFLOW_EQ:
-				{
-					// f_out = feq(1, u(f_in)), u = (j + F/2) / m0
-					const real m0 = m[0], jx = m[1], jy = m[2], jz = m[3];
-					const real rv = (real) 1 / m0;
-					const real ux = (jx + (real) 0.5 * (real) A.fx) * rv, uy = (jy + (real) 0.5 * (real) A.fy) * rv,
-							   uz = (jz + (real) 0.5 * (real) A.fz) * rv;
-					real gx = 0, gy = 0, gz = 0;
-					D::eq_grad(lam, ux, uy, uz, gx, gy, gz);
-#pragma unroll
-					for (int q = 0; q < 27; q++)
-						mu[q] = (lreal) ((gx * ((real) CX[q] - ux) + gy * ((real) CY[q] - uy) + gz * ((real) CZ[q] - uz)) * rv);
-					break;
-				}
-			default:
-				// no adjoint for this geometry code: make the result unusable, visibly
-#pragma unroll
-				for (int q = 0; q < 27; q++)
-					mu[q] = (lreal) __builtin_nan("");
-				break;
-		}
+			m[k] = (real) tp[tape_index(k, s0)];
 	}
 
-	elem* L = (elem*) P.lam;
-	if (! SPECIAL) {
-#pragma unroll
-		for (int q = 0; q < 27; q++) {
-			const real v = (irregular >> q) & 1u && ! unsupported ? (real) 0 : mu[q];
-			S::st(slot<O32, false>(L, q, A, WX[-CX[q]], WY[-CY[q]], WZ[-CZ[q]]), v);
+	const Nb WX = neighbours<false>(x, A.X, 0, false, true);
+	const Nb WY = neighbours<false>(y, A.Y, 0, false, true);
+	const Nb WZ = neighbours<false>(z, A.Z, 0, false, true);
+	// mu_q of this site to its slot: a plain store in the first pass (0 where
+	// the true reader is elsewhere), an atomic add in the second
+	auto put = [&](int q, real v) {
+		const bool irr = (irregular >> q) & 1u;
+		if constexpr (SPECIAL) {
+			if (irr)
+				atomicAdd(slot_at(L, q, PX[-CX[q]], NY[-CY[q]], NZ[-CZ[q]]), (elem) v);
 		}
+		else
+			S::st(slot_at(L, q, WX[-CX[q]], WY[-CY[q]], WZ[-CZ[q]]), irr && ! unsupported ? (real) 0 : v);
+	};
+	if ((gi == GEO_FLUID || gi == GEO_PERIODIC || gi == GEO_OUTFLOW_RIGHT) && ! unsupported) {
+		real l[D::NMOM];
+		D::vjp_m(m, lam, (real) A.fx, (real) A.fy, (real) A.fz, (real) A.omega1, gi == GEO_OUTFLOW_RIGHT, l);
+		if (! SPECIAL && irregular == 0)
+			D::for_each_mu(l, [&](int q, real v) { S::st(slot_at(L, q, WX[-CX[q]], WY[-CY[q]], WZ[-CZ[q]]), v); });
+		else
+			D::for_each_mu(l, put);
 	}
-	else {
+	else if (gi == GEO_WALL && ! unsupported) {
 #pragma unroll
 		for (int q = 0; q < 27; q++)
-			if ((irregular >> q) & 1u)
-				atomicAdd(L + q * A.XYZ + sidx(PX[-CX[q]], NY[-CY[q]], NZ[-CZ[q]]), (elem) mu[q]);
+			put(q, (real) lam[opp(q)]);
+	}
+	else if (gi == GEO_OUTFLOW_EQ && ! unsupported) {
+		// f_out = feq(1, u(f_in)), u = (j + F/2) / m0
+		const real rv = (real) 1 / m[0];
+		const real ux = (m[1] + (real) 0.5 * (real) A.fx) * rv, uy = (m[2] + (real) 0.5 * (real) A.fy) * rv,
+				   uz = (m[3] + (real) 0.5 * (real) A.fz) * rv;
+		real gx = 0, gy = 0, gz = 0;
+		D::eq_grad(lam, ux, uy, uz, gx, gy, gz);
+#pragma unroll
+		for (int q = 0; q < 27; q++)
+			put(q, (gx * ((real) CX[q] - ux) + gy * ((real) CY[q] - uy) + gz * ((real) CZ[q] - uz)) * rv);
+	}
+	else {
+		if (gi == GEO_INFLOW && ! unsupported && ! SPECIAL && P.grad) {
+			const int64_t iy = A.Y * z + y;
+			const real ux = (real) inflow_component(A, 0, iy);
+			const real uy = (real) inflow_component(A, 1, iy);
+			const real uz = (real) inflow_component(A, 2, iy);
+			real gx = 0, gy = 0, gz = 0;
+			D::eq_grad(lam, ux, uy, uz, gx, gy, gz);
+			const int64_t n = A.Y * A.Z;
+			atomicAdd(P.grad + iy, (double) gx);
+			atomicAdd(P.grad + n + iy, (double) gy);
+			atomicAdd(P.grad + 2 * n + iy, (double) gz);
+		}
+		// inlet sites (f_out does not depend on the state) and NOTHING sites: 0;
+		// a geometry code without an adjoint, or an irregular pull without a
+		// fix-up, makes the result unusable, visibly
+		const bool none = gi == GEO_NOTHING || (gi == GEO_INFLOW && ! unsupported);
+		const real v = none ? (real) 0 : (real) __builtin_nan("");
+#pragma unroll
+		for (int q = 0; q < 27; q++)
+			put(q, v);
 	}
 }
 

@@ -76,6 +76,12 @@ struct StepArgs
 
 constexpr int NXCD = 8;
 
+// one x plane of a population array of `elem`-byte elements takes 32-bit offsets
+inline bool narrow_planes(const StepArgs& A, size_t elem)
+{
+	return narrow_slots_allowed() && (uint64_t) A.Ys * (uint64_t) A.Zs * elem <= (1ull << 32);
+}
+
 // per-site force of MACRO::computeForcing (kernels.h:103): added to the
 // homogeneous force of copyQuantities (macro.h:80-86) in the arithmetic of
 // the collision
