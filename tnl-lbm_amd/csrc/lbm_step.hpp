@@ -52,6 +52,9 @@ struct StepArgs
 	uint32_t nblocks;  // logical blocks
 	uint32_t per_xcd;  // padded blocks / 8
 	int32_t lin;       // linear y-z mapping (see linearize)
+	// the even A-A step over one contiguous range of stored sites (flat_range)
+	int32_t flat;
+	int64_t flat0, nflat;  // its first site and length
 	int32_t even;
 	int32_t out_macro;
 	int32_t macro_f64;
@@ -163,6 +166,28 @@ LBM_DEV bool block_coords(const StepArgs& A, int64_t& x, int64_t& z, int64_t& y)
 	z = A.offz + (int64_t) (t % (uint32_t) A.nz);
 	x = A.offx + (int64_t) (t / (uint32_t) A.nz);
 	y = A.offy + (int64_t) yb * blockDim.x + threadIdx.x;
+	return y < A.offy + A.ny;
+}
+
+// the box's sites with the mapping chosen at compile time
+template <bool LIN>
+LBM_DEV bool box_coords(const StepArgs& A, int64_t& x, int64_t& z, int64_t& y)
+{
+	const uint32_t b = blockIdx.x;
+	const uint32_t L = (b % NXCD) * A.per_xcd + b / NXCD;
+	if (L >= A.nblocks)
+		return false;
+	if constexpr (LIN) {
+		const uint32_t i = (L % A.nyb) * blockDim.x + threadIdx.x;
+		x = A.offx + (int64_t) (L / A.nyb);
+		z = A.offz + (int64_t) (i / (uint32_t) A.ny);
+		y = A.offy + (int64_t) (i % (uint32_t) A.ny);
+		return i < (uint32_t) A.ny * (uint32_t) A.nz;
+	}
+	const uint32_t t = L / A.nyb;
+	z = A.offz + (int64_t) (t % (uint32_t) A.nz);
+	x = A.offx + (int64_t) (t / (uint32_t) A.nz);
+	y = A.offy + (int64_t) (L % A.nyb) * blockDim.x + threadIdx.x;
 	return y < A.offy + A.ny;
 }
 
@@ -285,7 +310,8 @@ LBM_DEV char* after(char* p, const T& v)
 }
 
 // Build-time tuning knobs (defaults are the measured best on MI355X):
-//  LBM_NT_EVEN   bitmask over storage forms: nontemporal hints on the even step
+//  LBM_NT_EVEN   bitmask over storage forms: nontemporal hints on the even
+//                step, where every wave's access covers whole lines
 //  LBM_PIN_ADDR  bitmask over storage forms: scalar base pointers, even step
 //  LBM_NT_ODD    bitmask over storage forms: nontemporal hints on the odd
 //                step's accesses within the site's own y (c_y = 0); the +-1
@@ -313,12 +339,11 @@ LBM_DEV char* after(char* p, const T& v)
 #ifndef LBM_PIN_ODD
 #define LBM_PIN_ODD 0x3f
 #endif
-//  LBM_TPB_FP32  block size of the periodic kernel for the FP32-compute forms
-//                where the row length is a multiple of it (the paired 2-byte
-//                even step keeps its own shape): a 512-site row in one block
-//                keeps 7 of its 8 wave boundaries, whose +-1 shifted lines the
-//                neighbouring waves share on the odd step, on one CU
-//                (measured +0.6 to +1.2 points on both steps at 512^3)
+//  LBM_TPB_FP32  block size of the periodic odd step for the FP32-compute forms
+//                where the row length is a multiple of it: a 512-site row in
+//                one block keeps 7 of its 8 wave boundaries, whose +-1 shifted
+//                lines the neighbouring waves share, on one CU (measured +0.6
+//                to +1.2 points at 512^3); and of the even step's flat range
 #ifndef LBM_TPB_FP32
 #define LBM_TPB_FP32 512
 #endif
@@ -351,124 +376,189 @@ LBM_DEV char* sptr(char* p)
 	return p;
 }
 
-template <int ST, int COLL, bool EVEN>
+// Site of a lane of the even step: the stored offset of its block's row or
+// range (wave-uniform) and its own offset from there.  The even step moves
+// nothing between sites, so where the launch covers whole rows and columns of
+// a lattice without y and z overlaps, its sites are one contiguous range of
+// every population plane (A.flat): blocks take it in order, every wave is
+// full whatever the row length, and the planes' alignment alone decides
+// whether a wave's accesses cover whole lines.  `per` sites per lane.
+LBM_DEV bool even_site(const StepArgs& A, uint32_t per, uint64_t& row, uint32_t& yl)
+{
+	const uint32_t b = blockIdx.x;
+	const uint32_t L = (b % NXCD) * A.per_xcd + b / NXCD;
+	if (L >= A.nblocks)
+		return false;
+	if (A.flat) {
+		const uint64_t first = (uint64_t) L * (blockDim.x * per);
+		row = (uint64_t) A.flat0 + first;
+		yl = threadIdx.x * per;
+		return first + yl < (uint64_t) A.nflat;
+	}
+	const uint32_t t = L / A.nyb;
+	const int64_t z = A.offz + (int64_t) (t % (uint32_t) A.nz);
+	const int64_t x = A.offx + (int64_t) (t / (uint32_t) A.nz);
+	const uint32_t i = ((L % A.nyb) * blockDim.x + threadIdx.x) * per;
+	row = (uint64_t) (((x + A.ox) * A.Zs + (z + A.oz)) * A.Ys);
+	yl = (uint32_t) (A.offy + A.oy) + i;
+	return i < (uint32_t) A.ny;
+}
+
+// NTE: nontemporal hints, taken where every wave's accesses cover whole 128-byte
+// lines (even_launch).  A partial line written with the hint goes to memory by
+// itself instead of meeting its other half in L2: (301, 187, 129) F64 985 us
+// with the hints and 707 without, F32 (200, 100, 400) 578 and 303; with whole
+// lines they gain 2% (F64) to 10% (F16) at 512^3.
+template <int ST, int COLL, bool NTE>
 __global__ void __launch_bounds__(ST == TNL_LBM_STORE_F64 ? 256 : LBM_TPB_FP32)
 __attribute__((amdgpu_waves_per_eu(ST == TNL_LBM_STORE_F64 ? LBM_WAVES_F64 : 1, ST == TNL_LBM_STORE_F64 ? LBM_MAXWAVES_F64 : 8)))
-k_aa_periodic(const StepArgs A)
+k_aa_even(const StepArgs A)
 {
 	using S = Storage<ST>;
 	using real = typename S::real;
 	using elem = typename S::elem;
 	constexpr uint32_t E = sizeof(elem);
-	constexpr bool NT = (LBM_NT_EVEN >> ST) & 1;
+	constexpr bool NT = NTE && ((LBM_NT_EVEN >> ST) & 1);
 	constexpr bool PIN = (LBM_PIN_ADDR >> ST) & 1;
+	uint64_t first;
+	uint32_t yl;
+	if (! even_site(A, 1, first, yl))
+		return;
+	char* __restrict__ df = (char*) A.df0;
+	const uint64_t pb = A.plane_bytes;
+	real f[27];
+	const uint64_t row = first * E;
+	const uint32_t yb = yl * E;
+#pragma unroll
+	for (int q = 0; q < 27; q++) {
+		const elem* p = (const elem*) (sptr<PIN>(df + ((uint64_t) q * pb + row)) + yb);
+		const elem v = NT ? ld_nt(p) : *p;
+		f[q] = S::ld(&v, A.cls_sc[ncls(q)]);
+	}
+	real rho, vx, vy, vz;
+	collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
+	char* out = after<PIN>(df, f[26]);
+	if constexpr (S::fixed) {
+		// two populations per conversion
+#pragma unroll
+		for (int q = 0; q < 27; q += 2) {
+			const int q1 = q + 1 < 27 ? q + 1 : q;
+			const auto r = __builtin_amdgcn_cvt_pknorm_i16(f[q] * A.cls_inv[ncls(q)], f[q1] * A.cls_inv[ncls(q1)]);
+			elem* p0 = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q) * pb + row)) + yb);
+			NT ? st_nt(p0, (elem) r[0]) : (void) (*p0 = r[0]);
+			if (q + 1 < 27) {
+				elem* p1 = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q1) * pb + row)) + yb);
+				NT ? st_nt(p1, (elem) r[1]) : (void) (*p1 = r[1]);
+			}
+		}
+	}
+	else {
+#pragma unroll
+		for (int q = 0; q < 27; q++) {
+			elem v;
+			S::st(&v, f[q] * out_factor<ST, COLL>(q));
+			elem* p = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q) * pb + row)) + yb);
+			if (NT)
+				st_nt(p, v);
+			else
+				*p = v;
+		}
+	}
+	if (A.out_macro)
+		write_macro(A, (int64_t) (row / E) + yl, rho, vx, vy, vz);
+}
+
+// LIN: consecutive lanes walk the y-z plane of one x, row after row, so that a
+// row length that is not a multiple of the wave still fills every wave; x
+// stays wave-uniform, z becomes a per-lane row offset.  Otherwise a block is a
+// segment of one row and the row offsets are scalars.
+// NTO: nontemporal hints on the c_y = 0 accesses.
+template <int ST, int COLL, bool NTO, bool LIN>
+__global__ void __launch_bounds__(ST == TNL_LBM_STORE_F64 ? 256 : LBM_TPB_FP32)
+__attribute__((amdgpu_waves_per_eu(ST == TNL_LBM_STORE_F64 ? LBM_WAVES_F64 : 1, ST == TNL_LBM_STORE_F64 ? LBM_MAXWAVES_F64 : 8)))
+k_aa_odd(const StepArgs A)
+{
+	using S = Storage<ST>;
+	using real = typename S::real;
+	using elem = typename S::elem;
+	constexpr uint32_t E = sizeof(elem);
 	constexpr bool PIN_ODD = (LBM_PIN_ODD >> ST) & 1;
-	constexpr bool NT_ODD = (LBM_NT_ODD >> ST) & 1;
+	constexpr bool NT_ODD = NTO && ((LBM_NT_ODD >> ST) & 1);
 	int64_t x, z, y;
-	if (! block_coords<false>(A, x, z, y))
+	if (! box_coords<LIN>(A, x, z, y))
 		return;
 	char* __restrict__ df = (char*) A.df0;
 	const uint64_t pb = A.plane_bytes;
 	real f[27];
 	const uint32_t yl = (uint32_t) (y + A.oy);
-	if constexpr (EVEN) {
-		const uint64_t row = (uint64_t) (((x + A.ox) * A.Zs + (z + A.oz)) * A.Ys) * E;
-		const uint32_t yb = yl * E;
+	// periodic neighbours (kernelInitIndices, kernels.h:21-28)
+	const int64_t xp = (! A.dist_x && x == A.X - 1) ? 0 : x + 1;
+	const int64_t xm = (! A.dist_x && x == 0) ? A.X - 1 : x - 1;
+	const int64_t zp = (! A.dist_z && z == A.Z - 1) ? 0 : z + 1;
+	const int64_t zm = (! A.dist_z && z == 0) ? A.Z - 1 : z - 1;
+	const uint32_t ypl = (uint32_t) (((! A.dist_y && y == A.Y - 1) ? 0 : y + 1) + A.oy);
+	const uint32_t yml = (uint32_t) (((! A.dist_y && y == 0) ? A.Y - 1 : y - 1) + A.oy);
+	const int64_t xs[3] = {xm + A.ox, x + A.ox, xp + A.ox};
+	const int64_t zs[3] = {zm + A.oz, z + A.oz, zp + A.oz};
+	const uint32_t ys[3] = {yml * E, yl * E, ypl * E};
+	// scalar part and per-lane part of a slot's byte offset in its plane
+	// (LIN: one x plane holds at most 4 GiB, odd_launch)
+	uint64_t xrow[3];
+	uint32_t zrow[3];
 #pragma unroll
-		for (int q = 0; q < 27; q++) {
-			const elem* p = (const elem*) (sptr<PIN>(df + ((uint64_t) q * pb + row)) + yb);
-			const elem v = NT ? ld_nt(p) : *p;
+	for (int k = 0; k < 3; k++) {
+		xrow[k] = (uint64_t) (xs[k] * A.Zs * A.Ys) * E;
+		zrow[k] = (uint32_t) zs[k] * (uint32_t) A.Ys * E;
+	}
+	auto slot_of = [&](char* base, int q, int cx, int cy, int cz) {
+		if constexpr (LIN)
+			return (elem*) (sptr<PIN_ODD>(base + ((uint64_t) q * pb + xrow[1 + cx])) + (zrow[1 + cz] + ys[1 + cy]));
+		else {
+			const uint64_t row = (uint64_t) ((xs[1 + cx] * A.Zs + zs[1 + cz]) * A.Ys) * E;
+			return (elem*) (sptr<PIN_ODD>(base + ((uint64_t) q * pb + row)) + ys[1 + cy]);
+		}
+	};
+#pragma unroll
+	for (int q = 0; q < 27; q++) {
+		const elem* p = slot_of(df, opp(q), -CX[q], -CY[q], -CZ[q]);
+		if (NT_ODD && CY[q] == 0) {
+			const elem v = ld_nt(p);
 			f[q] = S::ld(&v, A.cls_sc[ncls(q)]);
 		}
-		real rho, vx, vy, vz;
-		collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
-		char* out = after<PIN>(df, f[26]);
-		if constexpr (S::fixed) {
-			// two populations per conversion
+		else
+			f[q] = S::ld(p, A.cls_sc[ncls(q)]);
+	}
+	real rho, vx, vy, vz;
+	collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
+	char* out = after<PIN_ODD>(df, f[26]);
+	auto dst = [&](int q) { return slot_of(out, q, CX[q], CY[q], CZ[q]); };
+	auto put = [&](int q, elem v) {
+		if (NT_ODD && CY[q] == 0)
+			st_nt(dst(q), v);
+		else
+			*dst(q) = v;
+	};
+	if constexpr (S::fixed) {
+		// two populations per conversion
 #pragma unroll
-			for (int q = 0; q < 27; q += 2) {
-				const int q1 = q + 1 < 27 ? q + 1 : q;
-				const auto r = __builtin_amdgcn_cvt_pknorm_i16(f[q] * A.cls_inv[ncls(q)], f[q1] * A.cls_inv[ncls(q1)]);
-				elem* p0 = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q) * pb + row)) + yb);
-				NT ? st_nt(p0, (elem) r[0]) : (void) (*p0 = r[0]);
-				if (q + 1 < 27) {
-					elem* p1 = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q1) * pb + row)) + yb);
-					NT ? st_nt(p1, (elem) r[1]) : (void) (*p1 = r[1]);
-				}
-			}
+		for (int q = 0; q < 27; q += 2) {
+			const int q1 = q + 1 < 27 ? q + 1 : q;
+			const auto r = __builtin_amdgcn_cvt_pknorm_i16(f[q] * A.cls_inv[ncls(q)], f[q1] * A.cls_inv[ncls(q1)]);
+			put(q, (elem) r[0]);
+			if (q + 1 < 27)
+				put(q1, (elem) r[1]);
 		}
-		else {
-#pragma unroll
-			for (int q = 0; q < 27; q++) {
-				elem v;
-				S::st(&v, f[q] * out_factor<ST, COLL>(q));
-				elem* p = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q) * pb + row)) + yb);
-				if (NT)
-					st_nt(p, v);
-				else
-					*p = v;
-			}
-		}
-		if (A.out_macro)
-			write_macro(A, (int64_t) (row / E) + yl, rho, vx, vy, vz);
 	}
 	else {
-		// periodic neighbours (kernelInitIndices, kernels.h:21-28)
-		const int64_t xp = (! A.dist_x && x == A.X - 1) ? 0 : x + 1;
-		const int64_t xm = (! A.dist_x && x == 0) ? A.X - 1 : x - 1;
-		const int64_t zp = (! A.dist_z && z == A.Z - 1) ? 0 : z + 1;
-		const int64_t zm = (! A.dist_z && z == 0) ? A.Z - 1 : z - 1;
-		const uint32_t ypl = (uint32_t) (((! A.dist_y && y == A.Y - 1) ? 0 : y + 1) + A.oy);
-		const uint32_t yml = (uint32_t) (((! A.dist_y && y == 0) ? A.Y - 1 : y - 1) + A.oy);
-		const int64_t xs[3] = {xm + A.ox, x + A.ox, xp + A.ox};
-		const int64_t zs[3] = {zm + A.oz, z + A.oz, zp + A.oz};
-		const uint32_t ys[3] = {yml * E, yl * E, ypl * E};
 #pragma unroll
 		for (int q = 0; q < 27; q++) {
-			const uint64_t row = (uint64_t) ((xs[1 - CX[q]] * A.Zs + zs[1 - CZ[q]]) * A.Ys) * E;
-			const elem* p = (const elem*) (sptr<PIN_ODD>(df + ((uint64_t) opp(q) * pb + row)) + ys[1 - CY[q]]);
-			if (NT_ODD && CY[q] == 0) {
-				const elem v = ld_nt(p);
-				f[q] = S::ld(&v, A.cls_sc[ncls(q)]);
-			}
-			else
-				f[q] = S::ld(p, A.cls_sc[ncls(q)]);
+			elem v;
+			S::st(&v, f[q] * out_factor<ST, COLL>(q));
+			put(q, v);
 		}
-		real rho, vx, vy, vz;
-		collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
-		char* out = after<PIN_ODD>(df, f[26]);
-		auto dst = [&](int q) {
-			const uint64_t row = (uint64_t) ((xs[1 + CX[q]] * A.Zs + zs[1 + CZ[q]]) * A.Ys) * E;
-			return (elem*) (sptr<PIN_ODD>(out + ((uint64_t) q * pb + row)) + ys[1 + CY[q]]);
-		};
-		auto put = [&](int q, elem v) {
-			if (NT_ODD && CY[q] == 0)
-				st_nt(dst(q), v);
-			else
-				*dst(q) = v;
-		};
-		if constexpr (S::fixed) {
-			// two populations per conversion
-#pragma unroll
-			for (int q = 0; q < 27; q += 2) {
-				const int q1 = q + 1 < 27 ? q + 1 : q;
-				const auto r = __builtin_amdgcn_cvt_pknorm_i16(f[q] * A.cls_inv[ncls(q)], f[q1] * A.cls_inv[ncls(q1)]);
-				put(q, (elem) r[0]);
-				if (q + 1 < 27)
-					put(q1, (elem) r[1]);
-			}
-		}
-		else {
-#pragma unroll
-			for (int q = 0; q < 27; q++) {
-				elem v;
-				S::st(&v, f[q] * out_factor<ST, COLL>(q));
-				put(q, v);
-			}
-		}
-		if (A.out_macro)
-			write_macro(A, (xs[1] * A.Zs + zs[1]) * A.Ys + yl, rho, vx, vy, vz);
 	}
+	if (A.out_macro)
+		write_macro(A, (xs[1] * A.Zs + zs[1]) * A.Ys + yl, rho, vx, vy, vz);
 }
 
 // ===========================================================================
@@ -579,25 +669,18 @@ LBM_DEV void collide_pair(uint32_t* w, const StepArgs& A, int64_t s)
 		w[q] = (w[q] & 0xffffu) | (C::put(f[q], q, A) << 16);
 }
 
-template <int ST, int COLL>
+template <int ST, int COLL, bool NTE>
 __global__ void __launch_bounds__(256) k_aa_even_pair(const StepArgs A)
 {
-	constexpr bool NT = (LBM_NT_EVEN >> ST) & 1;
+	constexpr bool NT = NTE && ((LBM_NT_EVEN >> ST) & 1);
 	constexpr bool PIN = (LBM_PIN_ADDR >> ST) & 1;
-	const uint32_t b = blockIdx.x;
-	const uint32_t L = (b % NXCD) * A.per_xcd + b / NXCD;
-	if (L >= A.nblocks)
+	uint64_t first;
+	uint32_t yl;  // sites yl, yl + 1 from `first` on
+	if (! even_site(A, 2, first, yl))
 		return;
-	const uint32_t t = L / A.nyb;
-	const int64_t z = A.offz + (int64_t) (t % (uint32_t) A.nz);
-	const int64_t x = A.offx + (int64_t) (t / (uint32_t) A.nz);
-	const uint32_t pair = (L % A.nyb) * blockDim.x + threadIdx.x;
-	if (2 * pair >= (uint32_t) A.ny)
-		return;
-	const uint32_t yl = (uint32_t) (A.offy + 2 * (int64_t) pair + A.oy);  // sites yl, yl + 1 of the stored row
 	char* __restrict__ df = (char*) A.df0;
 	const uint64_t pb = A.plane_bytes;
-	const uint64_t row = (uint64_t) (((x + A.ox) * A.Zs + (z + A.oz)) * A.Ys) * 2;
+	const uint64_t row = first * 2;
 	const uint32_t yb = yl * 2;
 	uint32_t w[27];
 #pragma unroll
@@ -1645,51 +1728,120 @@ int for_row_lists(const StepArgs& A, Go&& go)
 	return 0;
 }
 
-// Launch shape of k_aa_even_pair (one lane per two sites of a row); false
-// where the pairs would not be 4-byte aligned.
-inline bool pair_shape(const StepArgs& A, StepArgs& B, unsigned& threads, unsigned& grid)
+// Whether the populations fit the 256 MiB last-level cache, where one step
+// finds what the step before it wrote; nontemporal accesses give that up
+// (300x50x300 F16, 243 MB: 204 us for the two steps with them, 153 without).
+inline bool cache_resident(const StepArgs& A)
 {
-	if (((A.ny | A.offy | A.oy | A.Y | A.XYZ) & 1) || ((uintptr_t) A.df0 & 3))
-		return false;
-	B = A;
-	const uint32_t np = (uint32_t) A.ny / 2;
-	threads = np > 128 ? 256 : (np > 64 ? 128 : 64);
-	B.nyb = (np + threads - 1) / threads;
-	B.nblocks = B.nyb * (uint32_t) A.nz * (uint32_t) A.nx;  // no more blocks than one lane per site needs
-	const uint32_t padded = (B.nblocks + NXCD - 1) / NXCD * NXCD;
-	B.per_xcd = padded / NXCD;
-	grid = padded;
-	return true;
+	return 27 * A.plane_bytes <= (256ull << 20);
 }
 
-// The map-free periodic A-A kernels: the paired even step for the 2-byte
-// forms where the row allows it, else one site per lane.
-template <int ST, int COLL>
-int launch_periodic(const StepArgs& A, unsigned threads, unsigned grid, hipStream_t st)
+// Launch shape of an even A-A step with `per` sites per lane: the contiguous
+// range where the box covers whole rows and columns of a lattice without y and
+// z overlaps, else rows.  Returns whether to use nontemporal hints: where every
+// wave's accesses cover whole lines (the planes and each wave's first site
+// start on a 128-byte line) and the populations exceed the last-level cache.
+inline bool even_shape(StepArgs& A, uint32_t per, unsigned most, unsigned& threads, unsigned& grid, size_t elem)
 {
-	if constexpr (sizeof(typename Storage<ST>::elem) == 2 && ((LBM_PAIR_EVEN >> ST) & 1)) {
-		StepArgs B;
-		unsigned t2 = 0, g2 = 0;
-		if (A.even && pair_shape(A, B, t2, g2)) {
-			hipLaunchKernelGGL((k_aa_even_pair<ST, COLL>), dim3(g2), dim3(t2), 0, st, B);
+	const bool planes = A.plane_bytes % 128 == 0 && (uintptr_t) A.df0 % 128 == 0 && ! cache_resident(A);
+	bool whole;
+	if (A.oy == 0 && A.oz == 0 && A.ny == A.Y && A.nz == A.Z) {
+		A.flat = 1;
+		A.flat0 = (A.offx + A.ox) * A.Y * A.Z;
+		A.nflat = (int64_t) A.nx * A.Y * A.Z;
+		// smaller blocks where there would be fewer than eight for each CU
+		threads = most;
+		while (threads > 64 && (uint64_t) A.nflat < (uint64_t) threads * per * 2048)
+			threads /= 2;
+		A.nblocks = (uint32_t) ((A.nflat + (int64_t) threads * per - 1) / (threads * per));
+		whole = planes && (uint64_t) A.flat0 * elem % 128 == 0;
+	}
+	else {
+		const uint32_t n = (uint32_t) A.ny / per;
+		threads = n > 128 ? 256 : (n > 64 ? 128 : 64);
+		A.nyb = (n + threads - 1) / threads;
+		A.nblocks = A.nyb * (uint32_t) A.nz * (uint32_t) A.nx;  // no more blocks than one lane per site needs
+		whole = planes && (uint64_t) A.Ys * elem % 128 == 0 && (uint64_t) (A.oy + A.offy) * elem % 128 == 0;
+	}
+	const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
+	A.per_xcd = padded / NXCD;
+	grid = padded;
+	return whole;
+}
+
+template <int ST, int COLL>
+int even_launch(const StepArgs& A0, hipStream_t st)
+{
+	constexpr size_t E = sizeof(typename Storage<ST>::elem);
+	StepArgs A = A0;
+	unsigned threads = 0, grid = 0;
+	if constexpr (E == 2 && ((LBM_PAIR_EVEN >> ST) & 1)) {
+		// pairs must start at even stored offsets of every plane
+		// (the fixed-point form takes them in even rows only: in odd rows its
+		// stored integers stay those of the one-site kernel, whose fused
+		// operations round 1 in 10^4 of them to the neighbouring unit)
+		const bool flat = ! Storage<ST>::fixed && A.oy == 0 && A.oz == 0 && A.ny == A.Y && A.nz == A.Z;
+		const int64_t odd = flat ? ((A.offx + A.ox) * A.Y * A.Z) | (A.nx * A.Y * A.Z) : A.ny | A.offy | A.oy | A.Y;
+		if (! ((odd | A.XYZ) & 1) && ! ((uintptr_t) A.df0 & 3)) {
+			if (even_shape(A, 2, 256, threads, grid, E))
+				hipLaunchKernelGGL((k_aa_even_pair<ST, COLL, true>), dim3(grid), dim3(threads), 0, st, A);
+			else
+				hipLaunchKernelGGL((k_aa_even_pair<ST, COLL, false>), dim3(grid), dim3(threads), 0, st, A);
 			return hip_check(hipGetLastError(), "step launch");
 		}
 	}
-	if (ST != TNL_LBM_STORE_F64 && LBM_TPB_FP32 > 256 && A.ny % LBM_TPB_FP32 == 0) {
-		StepArgs B = A;
-		B.nyb = (uint32_t) A.ny / LBM_TPB_FP32;
-		B.nblocks = B.nyb * (uint32_t) A.nz * (uint32_t) A.nx;  // fewer blocks than at 256
-		const uint32_t padded = (B.nblocks + NXCD - 1) / NXCD * NXCD;
-		B.per_xcd = padded / NXCD;
-		if (A.even)
-			hipLaunchKernelGGL((k_aa_periodic<ST, COLL, true>), dim3(padded), dim3(LBM_TPB_FP32), 0, st, B);
-		else
-			hipLaunchKernelGGL((k_aa_periodic<ST, COLL, false>), dim3(padded), dim3(LBM_TPB_FP32), 0, st, B);
-	}
-	else if (A.even)
-		hipLaunchKernelGGL((k_aa_periodic<ST, COLL, true>), dim3(grid), dim3(threads), 0, st, A);
+	if (even_shape(A, 1, ST == TNL_LBM_STORE_F64 ? 256 : LBM_TPB_FP32, threads, grid, E))
+		hipLaunchKernelGGL((k_aa_even<ST, COLL, true>), dim3(grid), dim3(threads), 0, st, A);
 	else
-		hipLaunchKernelGGL((k_aa_periodic<ST, COLL, false>), dim3(grid), dim3(threads), 0, st, A);
+		hipLaunchKernelGGL((k_aa_even<ST, COLL, false>), dim3(grid), dim3(threads), 0, st, A);
+	return hip_check(hipGetLastError(), "step launch");
+}
+
+// The odd step: rows of whole blocks, else the linear mapping, whose waves are
+// all full (even and odd step together: 320^3 FP64 5.26 -> 4.63 ms, 512x30x512
+// F32 1042 -> 557 us, with the even step's flat range; where rows are whole
+// blocks the scalar row offsets win, 512^3 F16 2.46 against 2.52 ms).
+template <int ST, int COLL, bool NTO>
+void odd_launch(const StepArgs& A0, unsigned threads, unsigned grid, hipStream_t st)
+{
+	StepArgs A = A0;
+	if (A.ny % (int32_t) threads && (uint64_t) A.Ys * (uint64_t) A.Zs * sizeof(typename Storage<ST>::elem) <= (1ull << 32)) {
+		threads = 256;
+		const uint64_t plane = (uint64_t) A.ny * (uint64_t) A.nz;
+		while (threads > 64 && plane * (uint64_t) A.nx < (uint64_t) threads * 2048)
+			threads /= 2;
+		A.nyb = (uint32_t) ((plane + threads - 1) / threads);
+		A.nblocks = A.nyb * (uint32_t) A.nx;
+		const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
+		A.per_xcd = padded / NXCD;
+		hipLaunchKernelGGL((k_aa_odd<ST, COLL, NTO, true>), dim3(padded), dim3(threads), 0, st, A);
+		return;
+	}
+	if (ST != TNL_LBM_STORE_F64 && LBM_TPB_FP32 > 256 && A.ny % LBM_TPB_FP32 == 0) {
+		threads = LBM_TPB_FP32;
+		A.nyb = (uint32_t) A.ny / LBM_TPB_FP32;
+		A.nblocks = A.nyb * (uint32_t) A.nz * (uint32_t) A.nx;  // fewer blocks than at 256
+		grid = (A.nblocks + NXCD - 1) / NXCD * NXCD;
+		A.per_xcd = grid / NXCD;
+	}
+	hipLaunchKernelGGL((k_aa_odd<ST, COLL, NTO, false>), dim3(grid), dim3(threads), 0, st, A);
+}
+
+// The map-free periodic A-A kernels
+template <int ST, int COLL>
+int launch_periodic(const StepArgs& A, unsigned threads, unsigned grid, hipStream_t st)
+{
+	if (A.even)
+		return even_launch<ST, COLL>(A, st);
+	// nontemporal hints on the c_y = 0 accesses where rows start on lines, as
+	// in even_shape (301x187x129 FP64, both steps: 1428 us with them, 1377
+	// without; 512^3: 18.79 and 18.96 ms)
+	const bool nt = ! cache_resident(A) && A.plane_bytes % 128 == 0 && (uintptr_t) A.df0 % 128 == 0
+				 && (uint64_t) A.Ys * sizeof(typename Storage<ST>::elem) % 128 == 0;
+	if (nt)
+		odd_launch<ST, COLL, true>(A, threads, grid, st);
+	else
+		odd_launch<ST, COLL, false>(A, threads, grid, st);
 	return hip_check(hipGetLastError(), "step launch");
 }
 
