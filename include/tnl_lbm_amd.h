@@ -207,12 +207,12 @@ typedef struct tnl_lbm_d3q27_data {
 	const void* force_field;
 	/* Row lists of this map (no counterpart in the reference; NULL = none):
 	 * the output of tnl_lbm_classify_rows(SD, NULL, ...).  A step over the
-	 * whole box (offset 0, end = X, Y, Z) of the default cumulant in a
-	 * deviation storage form then runs each list through its own kernel:
-	 * rows of FLUID and PERIODIC sites only, rows that also hold WALL sites,
-	 * and the remaining rows through the kernel with every boundary code
-	 * (the F64 and F32 forms gain nothing from it and ignore the lists).  The
-	 * lists must describe the current map: classify again after changing it. */
+	 * whole box (offset 0, end = X, Y, Z) of the default cumulant then takes
+	 * its FLUID, PERIODIC and WALL sites through kernels without the other
+	 * boundary codes, and the other sites of the class 0 rows through the
+	 * kernel with every code (where those rows are at most an eighth of all;
+	 * the A-B steps of F64 and F32: where there are none).  The lists must
+	 * describe the current map: classify again after changing it.            */
 	const uint32_t* rows;
 	int64_t row_count[3];
 } tnl_lbm_d3q27_data;

@@ -289,8 +289,7 @@ inline uint32_t flags_for(const DIST& distributed, bool output_macro)
 // of local X*Z entries (a TNL array, say) and the three counts that
 // tnl_lbm_classify_rows writes.  Classify once after the map is set up and
 // again after every change of it, then pass the lists to step /
-// step_coupled: whole-box steps of the deviation forms, and every whole-box
-// coupled step, then run the rows of FLUID/PERIODIC (and WALL) sites
+// step_coupled: whole-box steps then run the FLUID, PERIODIC and WALL sites
 // through kernels without the other boundary codes.
 struct row_lists
 {

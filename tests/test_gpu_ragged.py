@@ -70,6 +70,13 @@ def test_whole_box_equals_its_sub_boxes(shape, storage):
         b.df[0].copy_(a.df[0])
 
 
+@pytest.mark.parametrize("storage,shape", [("f64", (80, 256, 64)), ("f64", (60, 208, 110)), ("f16dev", (200, 256, 100)),
+                                           ("f32", (100, 512, 50))])
+def test_boxes_beyond_the_cache(storage, shape):
+    """Populations above the last-level cache, planes on lines: the forms with hints."""
+    test_whole_box_equals_its_sub_boxes(shape, storage)
+
+
 @pytest.mark.parametrize("shape", [(3, 63, 5), (7, 97, 3), (2, 320, 2), (3, 513, 2)])
 def test_f64_against_the_oracle(shape):
     a = lattice(shape, "f64", 5)

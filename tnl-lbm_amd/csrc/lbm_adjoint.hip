@@ -33,10 +33,14 @@ int record_for(const StepArgs& A0, unsigned threads, unsigned grid, hipStream_t 
 	linearize(A, threads, grid);
 	// 32-bit slot offsets where each population array holds at most 4 GiB:
 	// -124 (FP64) / -151 (FP32) VALU, ~4% on the C4 duct (kernel trace)
-	if (narrow_slots(A.XYZ, sizeof(typename Storage<ST>::elem)))
-		hipLaunchKernelGGL((k_general<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, TAPE, true>), dim3(grid), dim3(threads), 0, st, A);
-	else
+	constexpr size_t E = sizeof(typename Storage<ST>::elem);
+	const bool nt = hint_streams(A, 54, E);
+	if (! narrow_slots(A.XYZ, E))
 		hipLaunchKernelGGL((k_general<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, TAPE>), dim3(grid), dim3(threads), 0, st, A);
+	else if (nt)
+		hipLaunchKernelGGL((k_general<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, TAPE, true, false, true>), dim3(grid), dim3(threads), 0, st, A);
+	else
+		hipLaunchKernelGGL((k_general<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, TAPE, true>), dim3(grid), dim3(threads), 0, st, A);
 	return hip_check(hipGetLastError(), "recording step launch");
 }
 

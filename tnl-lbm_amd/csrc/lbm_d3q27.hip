@@ -459,38 +459,61 @@ int tnl_lbm_nse_ade_step(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* ns
 			return rc;
 	auto go = [&](auto stc) {
 		constexpr int ST = decltype(stc)::value;
-		// 2-byte forms: 32-bit slot offsets where each population array (D3Q27
-		// and D3Q7 share XYZ) holds at most 4 GiB, as in the map kernel
-		constexpr bool two = sizeof(typename Storage<ST>::elem) == 2;
-		const bool o32 = two && narrow_slots(A.XYZ, 2);
-		auto one = [&](auto lc, const StepArgs& C, unsigned t, unsigned g) {
-			constexpr int LEAN = decltype(lc)::value;
-			if (o32) {
-				if constexpr (two) {
-					if (cfg->pattern == TNL_LBM_PATTERN_AA)
-						hipLaunchKernelGGL((k_nse_ade<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AA, true, LEAN>), dim3(g), dim3(t), 0, st, C, B);
-					else
-						hipLaunchKernelGGL((k_nse_ade<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, true, LEAN>), dim3(g), dim3(t), 0, st, C, B);
+		constexpr size_t E = sizeof(typename Storage<ST>::elem);
+		const bool ab = cfg->pattern == TNL_LBM_PATTERN_AB;
+		// every row in one launch of the general kernel, or the listed ones
+		auto general = [&](auto lc, const StepArgs& C, unsigned t, unsigned g) {
+			constexpr bool LISTED = decltype(lc)::value;
+			auto form = [&](auto oc) {
+				constexpr bool O32 = decltype(oc)::value;
+				if (! ab)
+					hipLaunchKernelGGL((k_nse_ade<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AA, O32, LISTED>), dim3(g), dim3(t), 0, st, C, B);
+				else if (LISTED || ! hint_streams(C, 68, E))
+					hipLaunchKernelGGL((k_nse_ade<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, O32, LISTED>), dim3(g), dim3(t), 0, st, C, B);
+				else if constexpr (! LISTED)
+					hipLaunchKernelGGL((k_nse_ade<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, O32, false, true>), dim3(g), dim3(t), 0, st, C, B);
+			};
+			// 2-byte forms: 32-bit slot offsets where each population array
+			// (D3Q27 and D3Q7 share XYZ) holds at most 4 GiB, as in the map kernel
+			if constexpr (E == 2) {
+				if (narrow_slots(C.XYZ, 2)) {
+					form(std::true_type{});
+					return hip_check(hipGetLastError(), "nse_ade launch");
 				}
 			}
-			else if (cfg->pattern == TNL_LBM_PATTERN_AA)
-				hipLaunchKernelGGL((k_nse_ade<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AA, false, LEAN>), dim3(g), dim3(t), 0, st, C, B);
-			else
-				hipLaunchKernelGGL((k_nse_ade<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, false, LEAN>), dim3(g), dim3(t), 0, st, C, B);
+			form(std::false_type{});
 			return hip_check(hipGetLastError(), "nse_ade launch");
 		};
-		if (A.lists)
-			return for_row_lists(A, [&](const StepArgs& C, unsigned t, unsigned g, int lean) {
-				if (lean == 1)
-					return one(std::integral_constant<int, 1>{}, C, t, g);
-				if (lean == 2)
-					return one(std::integral_constant<int, 2>{}, C, t, g);
-				return one(std::integral_constant<int, 3>{}, C, t, g);
+		// the lean kernels step both lattices in one parity
+		if (lean_split(A, E) && (ab || B.even == A.even)) {
+			lean_shape(A, ab ? 68 : 34, E, [&](const StepArgs& C, unsigned t, unsigned g, bool lin) {
+				auto mode = [&](auto mc) {
+					constexpr int MODE = decltype(mc)::value;
+					if (lin)
+						hipLaunchKernelGGL((k_lean_ade<ST, MODE, true, false>), dim3(g), dim3(t), 0, st, C, B);
+					else
+						hipLaunchKernelGGL((k_lean_ade<ST, MODE, false, true>), dim3(g), dim3(t), 0, st, C, B);
+				};
+				if (ab)
+					mode(std::integral_constant<int, LEAN_AB>{});
+				else if (A.even)
+					mode(std::integral_constant<int, LEAN_EVEN>{});
+				else
+					mode(std::integral_constant<int, LEAN_ODD>{});
 			});
+			if (int rc = hip_check(hipGetLastError(), "nse_ade launch"))
+				return rc;
+			if (A.list_count[0] == 0)
+				return (int) TNL_LBM_OK;
+			StepArgs C = A;
+			unsigned t = threads, g = grid;
+			list_shape(C, A.lists, (uint32_t) A.list_count[0], t, g);
+			return general(std::true_type{}, C, t, g);
+		}
 		StepArgs C = A;
 		unsigned t = threads, g = grid;
 		linearize(C, t, g);
-		return one(std::integral_constant<int, 0>{}, C, t, g);
+		return general(std::false_type{}, C, t, g);
 	};
 	STORAGE_SWITCH(cfg->storage, go(std::integral_constant<int, ST>{}));
 }

@@ -77,6 +77,24 @@ struct StepArgs
 	int64_t list_count[3];
 };
 
+enum : int16_t
+{
+	GEO_FLUID = 0, GEO_WALL, GEO_INFLOW, GEO_INFLOW_LEFT, GEO_INFLOW_BB_LEFT, GEO_INFLOW_EQ_LEFT, GEO_OUTFLOW_EQ,
+	GEO_OUTFLOW_RIGHT, GEO_OUTFLOW_RIGHT_INTERP, GEO_PERIODIC, GEO_NOTHING, GEO_SYM_TOP, GEO_SYM_BOTTOM, GEO_SYM_LEFT,
+	GEO_SYM_RIGHT, GEO_SYM_BACK, GEO_SYM_FRONT
+};
+
+
+// the codes of most sites: collide and stream, or bounce back
+LBM_DEV bool plain(int16_t gi)
+{
+	return gi == GEO_FLUID || gi == GEO_PERIODIC || gi == GEO_WALL;
+}
+LBM_DEV bool plain_scalar(int16_t ga)
+{
+	return ga == A_FLUID || ga == A_PERIODIC || ga == A_WALL;
+}
+
 constexpr int NXCD = 8;
 
 // one x plane of a population array of `elem`-byte elements takes 32-bit offsets
@@ -279,7 +297,8 @@ constexpr float out_factor(int q)
 }
 
 template <int ST, int COLL>
-LBM_DEV void collide_site(typename Storage<ST>::real* f, const StepArgs& A, typename Storage<ST>::real& rho,
+LBM_DEV void collide_site(typename Storage<ST>::real* f, const StepArgs& A, typename Storage<ST>::real Fx,
+						  typename Storage<ST>::real Fy, typename Storage<ST>::real Fz, typename Storage<ST>::real& rho,
 						  typename Storage<ST>::real& vx, typename Storage<ST>::real& vy, typename Storage<ST>::real& vz)
 {
 	using real = typename Storage<ST>::real;
@@ -287,11 +306,59 @@ LBM_DEV void collide_site(typename Storage<ST>::real* f, const StepArgs& A, type
 		rho = vx = vy = vz = 0;
 	}
 	else if constexpr (fast_collision<ST, COLL>) {
-		FastCum<Storage<ST>::dev>::collide(f, (real) A.fx, (real) A.fy, (real) A.fz, (real) A.omega1, true, rho, vx, vy, vz);
+		FastCum<Storage<ST>::dev>::collide(f, Fx, Fy, Fz, (real) A.omega1, true, rho, vx, vy, vz);
 	}
 	else {
-		Phys<ST>::density_velocity(f, (real) A.fx, (real) A.fy, (real) A.fz, rho, vx, vy, vz);
-		collide<ST, COLL>(f, rho, vx, vy, vz, A, (real) A.fx, (real) A.fy, (real) A.fz);
+		Phys<ST>::density_velocity(f, Fx, Fy, Fz, rho, vx, vy, vz);
+		collide<ST, COLL>(f, rho, vx, vy, vz, A, Fx, Fy, Fz);
+	}
+}
+template <int ST, int COLL>
+LBM_DEV void collide_site(typename Storage<ST>::real* f, const StepArgs& A, typename Storage<ST>::real& rho,
+						  typename Storage<ST>::real& vx, typename Storage<ST>::real& vy, typename Storage<ST>::real& vz)
+{
+	using real = typename Storage<ST>::real;
+	collide_site<ST, COLL>(f, A, (real) A.fx, (real) A.fy, (real) A.fz, rho, vx, vy, vz);
+}
+
+// Full-way bounce-back (bc.h:201-221) of loaded populations, times the power of
+// two that encode_all takes off again.
+template <int ST, int COLL>
+LBM_DEV void bounce_back(typename Storage<ST>::real* f)
+{
+	using real = typename Storage<ST>::real;
+#pragma unroll
+	for (int q = 1; q < 27; q += 2) {
+		const real t = f[q] * (real) (1.0f / out_factor<ST, COLL>(q));
+		f[q] = f[q + 1] * (real) (1.0f / out_factor<ST, COLL>(q));
+		f[q + 1] = t;
+	}
+}
+
+// Post-collision populations to their stored form: put(q, element) in turn
+// (the fixed-point form converts two per instruction).
+template <int ST, int COLL, typename Put>
+LBM_DEV void encode_all(const typename Storage<ST>::real* f, const StepArgs& A, Put&& put)
+{
+	using S = Storage<ST>;
+	using elem = typename S::elem;
+	if constexpr (S::fixed) {
+#pragma unroll
+		for (int q = 0; q < 27; q += 2) {
+			const int q1 = q + 1 < 27 ? q + 1 : q;
+			const auto r = __builtin_amdgcn_cvt_pknorm_i16(f[q] * A.cls_inv[ncls(q)], f[q1] * A.cls_inv[ncls(q1)]);
+			put(q, (elem) r[0]);
+			if (q + 1 < 27)
+				put(q1, (elem) r[1]);
+		}
+	}
+	else {
+#pragma unroll
+		for (int q = 0; q < 27; q++) {
+			elem v;
+			S::st(&v, f[q] * out_factor<ST, COLL>(q));
+			put(q, v);
+		}
 	}
 }
 
@@ -409,7 +476,29 @@ LBM_DEV bool even_site(const StepArgs& A, uint32_t per, uint64_t& row, uint32_t&
 // itself instead of meeting its other half in L2: (301, 187, 129) F64 985 us
 // with the hints and 707 without, F32 (200, 100, 400) 578 and 303; with whole
 // lines they gain 2% (F64) to 10% (F16) at 512^3.
-template <int ST, int COLL, bool NTE>
+// MAP: the step of a lattice with a geometry map, at its plain sites (FLUID,
+// PERIODIC and WALL; sites of any other code are left to the general kernel).
+// A wall site's even step is the identity: the bounce-back swaps q and opp(q)
+// and the store swaps them back.  Waves of walls alone leave theirs; in other
+// waves the walls store what they loaded, since a gap would leave partial lines.
+
+// whether the site collides (a wall keeps its populations)
+LBM_DEV bool even_active(const StepArgs& A, int64_t s)
+{
+	const int16_t gi = A.map[s];
+	return gi == GEO_FLUID || gi == GEO_PERIODIC;
+}
+LBM_DEV void wall_macro(const StepArgs& A, int64_t s, bool f64)
+{
+	if (A.out_macro && A.map[s] == GEO_WALL) {
+		if (f64)
+			write_macro(A, s, 1.0, 0.0, 0.0, 0.0);
+		else
+			write_macro(A, s, 1.0f, 0.0f, 0.0f, 0.0f);
+	}
+}
+
+template <int ST, int COLL, bool NTE, bool MAP = false>
 __global__ void __launch_bounds__(ST == TNL_LBM_STORE_F64 ? 256 : LBM_TPB_FP32)
 __attribute__((amdgpu_waves_per_eu(ST == TNL_LBM_STORE_F64 ? LBM_WAVES_F64 : 1, ST == TNL_LBM_STORE_F64 ? LBM_MAXWAVES_F64 : 8)))
 k_aa_even(const StepArgs A)
@@ -424,48 +513,53 @@ k_aa_even(const StepArgs A)
 	uint32_t yl;
 	if (! even_site(A, 1, first, yl))
 		return;
+	bool wall = false;
+	if constexpr (MAP) {
+		const int16_t gi = A.map[(int64_t) first + yl];
+		wall = gi == GEO_WALL;
+		const bool moves = gi == GEO_FLUID || gi == GEO_PERIODIC;
+		const uint64_t any = __ballot(moves);
+		if (! (moves || (wall && any))) {
+			wall_macro(A, (int64_t) first + yl, ST == TNL_LBM_STORE_F64);
+			return;
+		}
+	}
 	char* __restrict__ df = (char*) A.df0;
 	const uint64_t pb = A.plane_bytes;
-	real f[27];
 	const uint64_t row = first * E;
 	const uint32_t yb = yl * E;
+	real f[27];
 #pragma unroll
 	for (int q = 0; q < 27; q++) {
 		const elem* p = (const elem*) (sptr<PIN>(df + ((uint64_t) q * pb + row)) + yb);
 		const elem v = NT ? ld_nt(p) : *p;
 		f[q] = S::ld(&v, A.cls_sc[ncls(q)]);
 	}
-	real rho, vx, vy, vz;
-	collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
+	real rho = 1, vx = 0, vy = 0, vz = 0;
+	if constexpr (MAP) {
+		real Fx = (real) A.fx, Fy = (real) A.fy, Fz = (real) A.fz;
+		if (A.force)
+			add_site_force(A, (int64_t) first + yl, Fx, Fy, Fz);
+		if (wall)
+			bounce_back<ST, COLL>(f);
+		if (! wall)
+			collide_site<ST, COLL>(f, A, Fx, Fy, Fz, rho, vx, vy, vz);
+	}
+	else
+		collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
 	char* out = after<PIN>(df, f[26]);
-	if constexpr (S::fixed) {
-		// two populations per conversion
-#pragma unroll
-		for (int q = 0; q < 27; q += 2) {
-			const int q1 = q + 1 < 27 ? q + 1 : q;
-			const auto r = __builtin_amdgcn_cvt_pknorm_i16(f[q] * A.cls_inv[ncls(q)], f[q1] * A.cls_inv[ncls(q1)]);
-			elem* p0 = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q) * pb + row)) + yb);
-			NT ? st_nt(p0, (elem) r[0]) : (void) (*p0 = r[0]);
-			if (q + 1 < 27) {
-				elem* p1 = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q1) * pb + row)) + yb);
-				NT ? st_nt(p1, (elem) r[1]) : (void) (*p1 = r[1]);
-			}
-		}
-	}
-	else {
-#pragma unroll
-		for (int q = 0; q < 27; q++) {
-			elem v;
-			S::st(&v, f[q] * out_factor<ST, COLL>(q));
-			elem* p = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q) * pb + row)) + yb);
-			if (NT)
-				st_nt(p, v);
-			else
-				*p = v;
-		}
-	}
+	uint32_t ob = yb;
+	if constexpr (MAP)
+		asm volatile("" : "+v"(ob));  // in this block, for the scalar-base form
+	encode_all<ST, COLL>(f, A, [&](int q, elem e) {
+		elem* p = (elem*) (sptr<PIN>(out + ((uint64_t) opp(q) * pb + row)) + ob);
+		if (NT)
+			st_nt(p, e);
+		else
+			*p = e;
+	});
 	if (A.out_macro)
-		write_macro(A, (int64_t) (row / E) + yl, rho, vx, vy, vz);
+		write_macro(A, (int64_t) first + yl, rho, vx, vy, vz);
 }
 
 // LIN: consecutive lanes walk the y-z plane of one x, row after row, so that a
@@ -532,31 +626,12 @@ k_aa_odd(const StepArgs A)
 	collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
 	char* out = after<PIN_ODD>(df, f[26]);
 	auto dst = [&](int q) { return slot_of(out, q, CX[q], CY[q], CZ[q]); };
-	auto put = [&](int q, elem v) {
+	encode_all<ST, COLL>(f, A, [&](int q, elem v) {
 		if (NT_ODD && CY[q] == 0)
 			st_nt(dst(q), v);
 		else
 			*dst(q) = v;
-	};
-	if constexpr (S::fixed) {
-		// two populations per conversion
-#pragma unroll
-		for (int q = 0; q < 27; q += 2) {
-			const int q1 = q + 1 < 27 ? q + 1 : q;
-			const auto r = __builtin_amdgcn_cvt_pknorm_i16(f[q] * A.cls_inv[ncls(q)], f[q1] * A.cls_inv[ncls(q1)]);
-			put(q, (elem) r[0]);
-			if (q + 1 < 27)
-				put(q1, (elem) r[1]);
-		}
-	}
-	else {
-#pragma unroll
-		for (int q = 0; q < 27; q++) {
-			elem v;
-			S::st(&v, f[q] * out_factor<ST, COLL>(q));
-			put(q, v);
-		}
-	}
+	});
 	if (A.out_macro)
 		write_macro(A, (xs[1] * A.Zs + zs[1]) * A.Ys + yl, rho, vx, vy, vz);
 }
@@ -617,12 +692,20 @@ struct PairCodec
 // high halves still hold site s + 1's inputs, so one packed array serves
 // both sites (binary16 writes a half and keeps the other in one
 // instruction).
-template <int ST, int COLL>
+template <int ST, int COLL, bool MAP = false>
 LBM_DEV void collide_pair(uint32_t* w, const StepArgs& A, int64_t s)
 {
 	using C = PairCodec<ST, COLL>;
 	float f[27];
 	float rho, vx, vy, vz;
+	auto site = [&](int64_t i) {
+		float Fx = (float) A.fx, Fy = (float) A.fy, Fz = (float) A.fz;
+		if (MAP && A.force)
+			add_site_force(A, i, Fx, Fy, Fz);
+		collide_site<ST, COLL>(f, A, Fx, Fy, Fz, rho, vx, vy, vz);
+		if (A.out_macro)
+			write_macro(A, i, rho, vx, vy, vz);
+	};
 	if constexpr (C::PACK2) {
 		// I16 and BF16 convert two values per instruction: site s's scaled
 		// outputs wait as floats, in the registers its decoded inputs held,
@@ -632,18 +715,14 @@ LBM_DEV void collide_pair(uint32_t* w, const StepArgs& A, int64_t s)
 #pragma unroll
 		for (int q = 0; q < 27; q++)
 			f[q] = C::get(w[q] & 0xffffu, q, A);
-		collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
-		if (A.out_macro)
-			write_macro(A, s, rho, vx, vy, vz);
+		site(s);
 #pragma unroll
 		for (int q = 0; q < 27; q++)
 			a[q] = C::scaled(f[q], q, A);
 #pragma unroll
 		for (int q = 0; q < 27; q++)
 			f[q] = C::get(w[q] >> 16, q, A);
-		collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
-		if (A.out_macro)
-			write_macro(A, s + 1, rho, vx, vy, vz);
+		site(s + 1);
 #pragma unroll
 		for (int q = 0; q < 27; q++)
 			w[q] = C::pack2(a[q], C::scaled(f[q], q, A));
@@ -652,24 +731,21 @@ LBM_DEV void collide_pair(uint32_t* w, const StepArgs& A, int64_t s)
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		f[q] = C::get(w[q] & 0xffffu, q, A);
-	collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
-	if (A.out_macro)
-		write_macro(A, s, rho, vx, vy, vz);
+	site(s);
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		w[q] = (w[q] & 0xffff0000u) | C::put(f[q], q, A);
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		f[q] = C::get(w[q] >> 16, q, A);
-	collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
-	if (A.out_macro)
-		write_macro(A, s + 1, rho, vx, vy, vz);
+	site(s + 1);
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		w[q] = (w[q] & 0xffffu) | (C::put(f[q], q, A) << 16);
 }
 
-template <int ST, int COLL, bool NTE>
+// MAP as in k_aa_even: a lane with one site that collides stores that half.
+template <int ST, int COLL, bool NTE, bool MAP = false>
 __global__ void __launch_bounds__(256) k_aa_even_pair(const StepArgs A)
 {
 	constexpr bool NT = NTE && ((LBM_NT_EVEN >> ST) & 1);
@@ -682,13 +758,36 @@ __global__ void __launch_bounds__(256) k_aa_even_pair(const StepArgs A)
 	const uint64_t pb = A.plane_bytes;
 	const uint64_t row = first * 2;
 	const uint32_t yb = yl * 2;
+	bool lo = true, hi = true;
+	if constexpr (MAP) {
+		lo = even_active(A, (int64_t) first + yl);
+		hi = even_active(A, (int64_t) first + yl + 1);
+		if (! lo && ! hi) {
+			wall_macro(A, (int64_t) first + yl, false);
+			wall_macro(A, (int64_t) first + yl + 1, false);
+			return;
+		}
+	}
 	uint32_t w[27];
 #pragma unroll
 	for (int q = 0; q < 27; q++) {
 		const uint32_t* p = (const uint32_t*) (sptr<PIN>(df + ((uint64_t) q * pb + row)) + yb);
 		w[q] = NT ? __builtin_nontemporal_load(p) : *p;
 	}
-	collide_pair<ST, COLL>(w, A, (int64_t) (row / 2) + yl);
+	collide_pair<ST, COLL, MAP>(w, A, (int64_t) (row / 2) + yl);
+	if constexpr (MAP) {
+		if (! (lo && hi)) {
+			// one plain site of the pair: its half only
+			wall_macro(A, (int64_t) first + yl + (lo ? 1 : 0), false);
+			uint32_t ob = lo ? yb : yb + 2;
+			asm volatile("" : "+v"(ob));
+#pragma unroll
+			for (int q = 0; q < 27; q++)
+				*(uint16_t*) (sptr<PIN>(after<PIN>(df, w[q]) + ((uint64_t) opp(q) * pb + row)) + ob)
+					= (uint16_t) (lo ? w[q] : w[q] >> 16);
+			return;
+		}
+	}
 	// The stores use the loads' lane offset, kept opaque: when the compiler
 	// sees the two equal it shares 64-bit lane pointers between loads and
 	// stores and drops both out of the scalar-base (saddr) form.  Each store's
@@ -709,13 +808,6 @@ __global__ void __launch_bounds__(256) k_aa_even_pair(const StepArgs A)
 // ===========================================================================
 // General path: geometry map + D3Q27_BC_All, A-A or A-B.
 // ===========================================================================
-enum : int16_t
-{
-	GEO_FLUID = 0, GEO_WALL, GEO_INFLOW, GEO_INFLOW_LEFT, GEO_INFLOW_BB_LEFT, GEO_INFLOW_EQ_LEFT, GEO_OUTFLOW_EQ,
-	GEO_OUTFLOW_RIGHT, GEO_OUTFLOW_RIGHT_INTERP, GEO_PERIODIC, GEO_NOTHING, GEO_SYM_TOP, GEO_SYM_BOTTOM, GEO_SYM_LEFT,
-	GEO_SYM_RIGHT, GEO_SYM_BACK, GEO_SYM_FRONT
-};
-
 struct Nb
 {
 	int64_t m, o, p;  // storage coordinates (overlap-shifted) of c = -1, 0, +1
@@ -804,14 +896,16 @@ LBM_DEV E* slot0(E* base, int q, const StepArgs& A, int64_t s)
 // access is one scalar-base load or store, in place of a 64-bit address per
 // lane and access.
 //
-// LEAN: the sites of the launch carry only FLUID or PERIODIC codes (1), or
-// those and WALL (2), as the row lists of tnl_lbm_classify_rows guarantee;
-// every other boundary path is left out of the kernel.  (The kernels take
-// LEAN 3 for the general paths over a row list: General sees 0.)  A kernel's register
-// allocation is the maximum over all of its paths, so the rarely taken ones
-// set it for every site: the F16 A-B map kernel needs 97 VGPRs with all of
-// them, 49 with FLUID and PERIODIC alone.
-template <int ST, int COLL, int PATTERN, int TAPE = 0, bool O32 = false, int LEAN = 0>
+// LISTED: the launch covers rows that hold other codes than the plain ones, and
+// steps their other sites only: the plain ones belong to the lean kernels.
+//
+// NTG: nontemporal hints on the A-B streams no other wave touches in this step
+// (the site's own slots, and the pulls with c_y = 0; the +-1 shifted rows share
+// cache lines with the neighbouring wave), where rows start on lines and the
+// arrays exceed the last-level cache (hint_streams): 256^3 F16 +2%, F32 +3%;
+// rows off the lines 301x187x129 F16 282 us with them and 187 without, arrays
+// within the cache 128x64x64 FP64 48.6 and 41.
+template <int ST, int COLL, int PATTERN, int TAPE = 0, bool O32 = false, bool LISTED = false, bool NTG = false>
 struct General
 {
 	using S = Storage<ST>;
@@ -822,10 +916,7 @@ struct General
 	static constexpr int EQK = eq_kind_of(COLL);
 	static constexpr bool FAST = fast_collision<ST, COLL>;
 
-	// Nontemporal hints on the streams no other wave touches in this step:
-	// the site's own slots, and the pulls and pushes with c_y = 0 (the +-1
-	// shifted rows share cache lines with the neighbouring wave)
-	static constexpr bool NT = (LBM_NT_GENERAL >> ST) & 1;
+	static constexpr bool NT = NTG && ((LBM_NT_GENERAL >> ST) & 1);
 	static LBM_DEV real ldq(const elem* p, float sc, bool nt)
 	{
 		if (nt) {
@@ -914,6 +1005,8 @@ struct General
 	{
 		const int64_t s0 = sidx(A, x + A.ox, y + A.oy, z + A.oz);
 		const int16_t gi = A.map ? __builtin_nontemporal_load(A.map + s0) : (int16_t) GEO_PERIODIC;
+		if (LISTED && plain(gi))
+			return;
 		const bool per = gi == GEO_PERIODIC;
 		NX = neighbours<AA>(x, A.X, A.ox, A.dist_x, per);
 		NY = neighbours<AA>(y, A.Y, A.oy, A.dist_y, per);
@@ -925,12 +1018,12 @@ struct General
 		real rho = 1, vx = 0, vy = 0, vz = 0;
 		const elem* __restrict__ cur = (const elem*) A.df0;
 
-		if (LEAN || gi != GEO_NOTHING) {
+		if (gi != GEO_NOTHING) {
 			// pull location (bc.h:72-74); OUTFLOW_RIGHT pulls as if located at x-1
 			Nb PX = NX;
-			if (! LEAN && gi == GEO_OUTFLOW_RIGHT)
+			if (gi == GEO_OUTFLOW_RIGHT)
 				PX.p = PX.o = NX.m;
-			if (! LEAN && gi == GEO_OUTFLOW_RIGHT_INTERP) {
+			if (gi == GEO_OUTFLOW_RIGHT_INTERP) {
 				// streamingInterpRight (streaming_AB.h:446-478)
 				const real cs = (real) 0.5773502691896257;
 #pragma unroll
@@ -971,13 +1064,7 @@ struct General
 					tm[k] = (TT) m[k];
 			}
 			const real rest = S::dev ? (real) 1 : (real) 0;
-			if constexpr (LEAN != 0) {
-				if (LEAN == 2 && gi == GEO_WALL)
-					bounce_back(f, rho, vx, vy, vz);
-				else if (! FAST)
-					P::density_velocity(f, Fx, Fy, Fz, rho, vx, vy, vz);
-			}
-			else switch (gi) {
+			switch (gi) {
 				case GEO_INFLOW:
 					inflow(A, y, z, vx, vy, vz);
 					rho = 1;
@@ -1092,21 +1179,20 @@ struct General
 					break;
 			}
 			// doCollision (bc.h:406-412)
-			const bool do_coll = LEAN ? (LEAN == 1 || gi != GEO_WALL)
-									  : (gi == GEO_FLUID || gi == GEO_PERIODIC || gi == GEO_OUTFLOW_RIGHT || gi == GEO_OUTFLOW_RIGHT_INTERP
-										 || gi == GEO_INFLOW_LEFT || gi == GEO_INFLOW_BB_LEFT);
+			const bool do_coll = gi == GEO_FLUID || gi == GEO_PERIODIC || gi == GEO_OUTFLOW_RIGHT || gi == GEO_OUTFLOW_RIGHT_INTERP
+							  || gi == GEO_INFLOW_LEFT || gi == GEO_INFLOW_BB_LEFT;
 			if constexpr (FAST) {
 				// FP32 forms, default cumulant: the raw-moment formulation (as the periodic kernel)
 				// wherever rho and u are the site's own; the boundary codes that replace them keep
 				// the reference chain
-				if (LEAN ? do_coll : (gi == GEO_FLUID || gi == GEO_PERIODIC)) {
+				if (gi == GEO_FLUID || gi == GEO_PERIODIC) {
 					using FC = FastCum<S::dev>;
 					FC::collide(f, Fx, Fy, Fz, (real) A.omega1, true, rho, vx, vy, vz);
 #pragma unroll
 					for (int q = 0; q < 27; q++)
 						f[q] *= FC::unscale(q);
 				}
-				else if (! LEAN && do_coll)
+				else if (do_coll)
 					collide<ST, COLL>(f, rho, vx, vy, vz, A, Fx, Fy, Fz);
 			}
 			else if (do_coll)
@@ -1150,16 +1236,14 @@ struct General
 // The FP64 default cumulant needs ~170 VGPRs here: asking for 3 waves per SIMD
 // (<= 168) costs at most 2 spilled registers; the alternative operators keep
 // their registers.
-// LEAN 0: the box (or sub-box) of the launch, every code; 1, 2: a row list
-// of that lean level; 3: a row list through the general paths
-template <int ST, int COLL, int PATTERN, int TAPE = 0, bool O32 = false, int LEAN = 0>
+template <int ST, int COLL, int PATTERN, int TAPE = 0, bool O32 = false, bool LISTED = false, bool NTG = false>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(COLL == TNL_LBM_COLL_CUM ? 3 : 1, 8))) k_general(const StepArgs A)
 {
 	int64_t x, z, y;
-	if (! block_coords<true, LEAN != 0>(A, x, z, y))
+	if (! block_coords<true, LISTED>(A, x, z, y))
 		return;
-	General<ST, COLL, PATTERN, TAPE, O32, LEAN == 3 ? 0 : LEAN>::site(A, x, y, z);
+	General<ST, COLL, PATTERN, TAPE, O32, LISTED, NTG>::site(A, x, y, z);
 }
 
 // ===========================================================================
@@ -1177,119 +1261,102 @@ struct AdeIn
 	typename Storage<ST>::real D, S;
 };
 
-template <int ST, int PATTERN, bool O32 = false, int LEAN = 0>
-LBM_DEV void ade_load(const StepArgs& A, const AdeArgs& B, int64_t s0, const Nb& NX, const Nb& NY, const Nb& NZ,
-					  AdeIn<ST>& in)
+// src(q): pointer to the stored population q pulled here, qs(q) its storage
+// direction, nt(q) whether to hint
+template <int ST, bool LEAN, typename Src>
+LBM_DEV void ade_load(const StepArgs& A, const AdeArgs& B, int64_t s0, int16_t gi, Src&& src, AdeIn<ST>& in)
 {
 	using K = Ade7<ST>;
 	using real = typename K::real;
-	using elem = typename K::elem;
-	constexpr bool AA = PATTERN == TNL_LBM_PATTERN_AA;
-	const int16_t gi = B.map ? B.map[s0] : (int16_t) A_PERIODIC;
 	in.gi = gi;
-	const real pr = (real) B.phi_ref, isc = (real) 1 / (real) B.scale;
 	auto macro_at = [&](const void* p) -> real {
 		return A.macro_f64 ? (real) ((const double*) p)[s0] : (real) ((const float*) p)[s0];
 	};
 	// D3Q7_MACRO_Default::copyQuantities (d3q7/macro.h:38-42)
 	in.D = B.diff ? macro_at(B.diff) : (real) B.D;
 	in.S = B.source ? macro_at(B.source) : (real) 0;
+	const real pr = (real) B.phi_ref, isc = (real) 1 / (real) B.scale;
 	if (LEAN || gi != A_NOTHING) {
-		const elem* cur = (const elem*) B.df0;
-		Nb PX = NX;
-		if (! LEAN && gi == A_OUTFLOW_RIGHT)
-			PX.p = PX.o = NX.m;
-		// nontemporal hints as in the D3Q27 update: own slots and c_y = 0 pulls
-		constexpr bool NT = (LBM_NT_GENERAL >> ST) & 1;
-		auto ld = [&](const elem* p, int qs, bool nt) -> real {
-			if (nt) {
-				const elem v = ld_nt(p);
-				return K::ld(&v, qs, pr, isc);
-			}
-			return K::ld(p, qs, pr, isc);
-		};
 #pragma unroll
-		for (int q = 0; q < 7; q++) {
-			if (AA && B.even)
-				in.f[q] = ld(slot0<O32>(cur, q, A, s0), q, NT);
-			else if (AA)
-				in.f[q] = ld(slot<O32>(cur, opp(q), A, PX[-CX[q]], NY[-CY[q]], NZ[-CZ[q]]), opp(q), NT && CY[q] == 0);
-			else
-				in.f[q] = ld(slot<O32>(cur, q, A, PX[-CX[q]], NY[-CY[q]], NZ[-CZ[q]]), q, NT && CY[q] == 0);
-		}
+		for (int q = 0; q < 7; q++)
+			in.f[q] = src(q, pr, isc);
 	}
 }
 
-// LEAN as in General: 1 = A_FLUID and A_PERIODIC sites only, 2 = those and A_WALL
-template <int ST, int PATTERN, bool O32 = false, int LEAN = 0>
-LBM_DEV void ade_site(const StepArgs& A, const AdeArgs& B, int64_t s0, typename Storage<ST>::real vx,
-					  typename Storage<ST>::real vy, typename Storage<ST>::real vz, const Nb& NX, const Nb& NY, const Nb& NZ,
-					  const AdeIn<ST>& in)
+// one pulled population: nontemporal where `nt`
+template <int ST>
+LBM_DEV typename Storage<ST>::real ade_get(const typename Storage<ST>::elem* p, int qs, typename Storage<ST>::real pr,
+										   typename Storage<ST>::real isc, bool nt)
+{
+	if (nt) {
+		const auto v = ld_nt(p);
+		return Ade7<ST>::ld(&v, qs, pr, isc);
+	}
+	return Ade7<ST>::ld(p, qs, pr, isc);
+}
+template <int ST>
+LBM_DEV void ade_put(typename Storage<ST>::elem* p, int qs, typename Storage<ST>::real v, typename Storage<ST>::real pr,
+					 typename Storage<ST>::real sc, bool nt)
+{
+	if (nt) {
+		typename Storage<ST>::elem e;
+		Ade7<ST>::st(&e, qs, v, pr, sc);
+		st_nt(p, e);
+	}
+	else
+		Ade7<ST>::st(p, qs, v, pr, sc);
+}
+
+// boundary codes and collision of the loaded populations: f post-collision,
+// returns phi.  LEAN: the plain codes only.
+template <int ST, bool LEAN>
+LBM_DEV typename Storage<ST>::real ade_update(const AdeArgs& B, const AdeIn<ST>& in, typename Storage<ST>::real vx,
+											  typename Storage<ST>::real vy, typename Storage<ST>::real vz,
+											  typename Storage<ST>::real* f)
 {
 	using K = Ade7<ST>;
 	using real = typename K::real;
-	using elem = typename K::elem;
-	constexpr bool AA = PATTERN == TNL_LBM_PATTERN_AA;
 	const int16_t gi = in.gi;
-	const real pr = (real) B.phi_ref, sc = (real) B.scale;
-	const real D = in.D;
 	real phi = 0;
-	if (LEAN || gi != A_NOTHING) {
-		real f[7];
 #pragma unroll
-		for (int q = 0; q < 7; q++)
-			f[q] = in.f[q];
-		if constexpr (LEAN != 0) {
+	for (int q = 0; q < 7; q++)
+		f[q] = in.f[q];
+	if constexpr (LEAN) {
+		phi = K::density(f);
+		if (gi == A_WALL)
+			K::bounce_back(f);
+	}
+	else switch (gi) {
+		case A_INFLOW:
+			phi = (real) B.inflow_phi;
+			K::set_eq(f, phi, vx, vy, vz);
+			break;
+		case A_WALL:
 			phi = K::density(f);
-			if (LEAN == 2 && gi == A_WALL)
-				K::bounce_back(f);
-		}
-		else switch (gi) {
-			case A_INFLOW:
-				phi = (real) B.inflow_phi;
-				K::set_eq(f, phi, vx, vy, vz);
-				break;
-			case A_WALL:
-				phi = K::density(f);
-				K::bounce_back(f);
-				break;
-			case A_SYM_TOP: f[zzm] = f[zzp]; phi = K::density(f); break;
-			case A_SYM_BOTTOM: f[zzp] = f[zzm]; phi = K::density(f); break;
-			case A_SYM_LEFT: f[pzz] = f[mzz]; phi = K::density(f); break;
-			case A_SYM_RIGHT: f[mzz] = f[pzz]; phi = K::density(f); break;
-			case A_SYM_BACK: f[zpz] = f[zmz]; phi = K::density(f); break;
-			case A_SYM_FRONT: f[zmz] = f[zpz]; phi = K::density(f); break;
-			default: phi = K::density(f); break;
-		}
-		if (LEAN ? (LEAN == 1 || gi != A_WALL) : (gi == A_FLUID || gi == A_PERIODIC || gi == A_SOLID || gi == A_OUTFLOW_RIGHT)) {
-			K::collide(B.collision, f, phi, vx, vy, vz, D);
-			if (B.source) {
+			K::bounce_back(f);
+			break;
+		case A_SYM_TOP: f[zzm] = f[zzp]; phi = K::density(f); break;
+		case A_SYM_BOTTOM: f[zzp] = f[zzm]; phi = K::density(f); break;
+		case A_SYM_LEFT: f[pzz] = f[mzz]; phi = K::density(f); break;
+		case A_SYM_RIGHT: f[mzz] = f[pzz]; phi = K::density(f); break;
+		case A_SYM_BACK: f[zpz] = f[zmz]; phi = K::density(f); break;
+		case A_SYM_FRONT: f[zmz] = f[zpz]; phi = K::density(f); break;
+		default: phi = K::density(f); break;
+	}
+	if (LEAN ? gi != A_WALL : (gi == A_FLUID || gi == A_PERIODIC || gi == A_SOLID || gi == A_OUTFLOW_RIGHT)) {
+		K::collide(B.collision, f, phi, vx, vy, vz, in.D);
+		if (B.source) {
 #pragma unroll
-				for (int q = 0; q < 7; q++)
-					f[q] += (real) w7(q) * in.S;
-			}
-		}
-		elem* out = (elem*) (AA ? B.df0 : B.df1);
-		constexpr bool NT = (LBM_NT_GENERAL >> ST) & 1;
-		auto st = [&](elem* p, int qs, real v, bool nt) {
-			if (nt) {
-				elem e;
-				K::st(&e, qs, v, pr, sc);
-				st_nt(p, e);
-			}
-			else
-				K::st(p, qs, v, pr, sc);
-		};
-#pragma unroll
-		for (int q = 0; q < 7; q++) {
-			if (AA && B.even)
-				st(slot0<O32>(out, opp(q), A, s0), opp(q), f[q], NT);
-			else if (AA)
-				st(slot<O32>(out, q, A, NX[CX[q]], NY[CY[q]], NZ[CZ[q]]), q, f[q], NT && CY[q] == 0);
-			else
-				st(slot0<O32>(out, q, A, s0), q, f[q], NT);
+			for (int q = 0; q < 7; q++)
+				f[q] += (real) w7(q) * in.S;
 		}
 	}
+	return phi;
+}
+
+template <int ST>
+LBM_DEV void write_phi(const StepArgs& A, const AdeArgs& B, int64_t s0, typename Storage<ST>::real phi)
+{
 	if (A.out_macro && B.macro) {
 		if (A.macro_f64)
 			((double*) B.macro)[s0] = phi;
@@ -1298,27 +1365,271 @@ LBM_DEV void ade_site(const StepArgs& A, const AdeArgs& B, int64_t s0, typename 
 	}
 }
 
-// LEAN as for k_general
-template <int ST, int COLL, int PATTERN, bool O32 = false, int LEAN = 0>
+// LISTED, NTG as in General; a site is plain where both of its codes are
+template <int ST, int COLL, int PATTERN, bool O32 = false, bool LISTED = false, bool NTG = false>
 __global__ void __launch_bounds__(256) k_nse_ade(const StepArgs A, const AdeArgs B)
 {
-	constexpr int LV = LEAN == 3 ? 0 : LEAN;
+	using K = Ade7<ST>;
+	using real = typename K::real;
+	using elem = typename K::elem;
 	int64_t x, z, y;
-	if (! block_coords<true, LEAN != 0>(A, x, z, y))
+	if (! block_coords<true, LISTED>(A, x, z, y))
 		return;
 	constexpr bool AA = PATTERN == TNL_LBM_PATTERN_AA;
+	constexpr bool NT = NTG && ((LBM_NT_GENERAL >> ST) & 1);
 	const int64_t s0 = ((x + A.ox) * A.Zs + (z + A.oz)) * A.Ys + (y + A.oy);
+	const int16_t gn = A.map ? A.map[s0] : (int16_t) GEO_PERIODIC;
+	const int16_t ga = B.map ? B.map[s0] : (int16_t) A_PERIODIC;
+	if (LISTED && plain(gn) && plain_scalar(ga))
+		return;
 	// neighbours as General::site forms them (periodic wrap for PERIODIC-coded sites)
-	const bool per = (A.map ? A.map[s0] : (int16_t) GEO_PERIODIC) == GEO_PERIODIC;
+	const bool per = gn == GEO_PERIODIC;
 	const Nb NX = neighbours<AA>(x, A.X, A.ox, A.dist_x, per);
 	const Nb NY = neighbours<AA>(y, A.Y, A.oy, A.dist_y, per);
 	const Nb NZ = neighbours<AA>(z, A.Z, A.oz, A.dist_z, per);
+	Nb PX = NX;
+	if (ga == A_OUTFLOW_RIGHT)
+		PX.p = PX.o = NX.m;
 	AdeIn<ST> in;
-	ade_load<ST, PATTERN, O32, LV>(A, B, s0, NX, NY, NZ, in);
-	typename Storage<ST>::real vx, vy, vz;
+	const elem* cur = (const elem*) B.df0;
+	ade_load<ST, false>(A, B, s0, ga,
+				 [&](int q, real pr, real isc) {
+					 if (AA && B.even)
+						 return ade_get<ST>(slot0<O32>(cur, q, A, s0), q, pr, isc, NT);
+					 const int qs = AA ? opp(q) : q;
+					 return ade_get<ST>(slot<O32>(cur, qs, A, PX[-CX[q]], NY[-CY[q]], NZ[-CZ[q]]), qs, pr, isc, NT && CY[q] == 0);
+				 },
+				 in);
+	real vx, vy, vz;
 	Nb GX, GY, GZ;
-	General<ST, COLL, PATTERN, 0, O32, LV>::site(A, x, y, z, vx, vy, vz, GX, GY, GZ);
-	ade_site<ST, PATTERN, O32, LV>(A, B, s0, vx, vy, vz, NX, NY, NZ, in);
+	General<ST, COLL, PATTERN, 0, O32, false, NTG>::site(A, x, y, z, vx, vy, vz, GX, GY, GZ);
+	real phi = 0;
+	if (ga != A_NOTHING) {
+		real f[7];
+		phi = ade_update<ST, false>(B, in, vx, vy, vz, f);
+		elem* out = (elem*) (AA ? B.df0 : B.df1);
+		const real pr = (real) B.phi_ref, sc = (real) B.scale;
+#pragma unroll
+		for (int q = 0; q < 7; q++) {
+			if (AA && B.even)
+				ade_put<ST>(slot0<O32>(out, opp(q), A, s0), opp(q), f[q], pr, sc, NT);
+			else if (AA)
+				ade_put<ST>(slot<O32>(out, q, A, NX[CX[q]], NY[CY[q]], NZ[CZ[q]]), q, f[q], pr, sc, NT && CY[q] == 0);
+			else
+				ade_put<ST>(slot0<O32>(out, q, A, s0), q, f[q], pr, sc, NT);
+		}
+	}
+	write_phi<ST>(A, B, s0, phi);
+}
+
+// ===========================================================================
+// Lean kernels: the plain sites (FLUID, PERIODIC, WALL) of a box with a
+// geometry map, flow alone (A-A odd step, A-B step) or coupled (all three).
+// The sites of any other code are skipped; a launch of the general kernels
+// over the rows that hold them (LISTED) steps those.
+//
+// A kernel's registers are the maximum over all of its paths, so the rarely
+// taken boundary codes cost every site of the general kernels their occupancy
+// (F16 A-B: 97 VGPRs with all 17 codes, 48 with these).  Beyond that, a block
+// lies in one x plane (LIN) or in one row, so x (and z) are wave-uniform and a
+// slot is a scalar base plus a 32-bit per-lane offset; per-lane coordinates
+// cost about 150 VALU instructions a site.  Only the choice between the
+// periodic wrap and the clamp at a face depends on the site's code: where the
+// two differ, the lanes of either kind run in turn.
+// Bound: HBM.  Both steps, against the list kernels with per-lane coordinates:
+// 256^3 with z walls A-A F16 816 -> 710 us, F32 1484 -> 1368, FP64 2934 ->
+// 2761; A-B 301x187x129 F16 571 -> 363 (rows off the lines); coupled A-A 256^3
+// F16 1074 -> 985; coupled A-B aligned: equal (4.9 TB/s).
+// ===========================================================================
+constexpr int LEAN_EVEN = 0, LEAN_ODD = 1, LEAN_AB = 2;
+
+template <bool LIN>
+struct Stencil
+{
+	uint64_t xoff[3];       // sites before the x plane of -1, 0, +1 (wave-uniform)
+	uint32_t zs[3], zr[3];  // stored z: wave-uniform, or (LIN) the z row's per-lane offset in its plane
+	uint32_t ys[3];         // stored y, per lane
+	// Called in the basic block of each group of accesses: a lane offset that is
+	// extended to 64 bits in another block leaves the scalar-base form.
+	LBM_DEV void local()
+	{
+#pragma unroll
+		for (int c = 0; c < 3; c++) {
+			asm volatile("" : "+v"(ys[c]));
+			if constexpr (LIN)
+				asm volatile("" : "+v"(zr[c]));
+		}
+	}
+	// the site's own stored index
+	LBM_DEV int64_t own(const StepArgs& A) const
+	{
+		int64_t s = (int64_t) xoff[1] + (LIN ? zr[1] : zs[1] * (uint32_t) A.Ys) + ys[1];
+		asm volatile("" : "+v"(s));
+		return s;
+	}
+	// slot of direction q: pb is the byte stride between directions
+	template <typename E>
+	LBM_DEV E* slot(E* base, uint64_t pb, const StepArgs& A, int q, int cx, int cy, int cz) const
+	{
+		if constexpr (LIN)
+			return at((E*) sptr<true>((char*) base + ((uint64_t) q * pb + xoff[1 + cx] * sizeof(E))), zr[1 + cz] + ys[1 + cy]);
+		else
+			return at((E*) sptr<true>((char*) base + ((uint64_t) q * pb + (xoff[1 + cx] + (uint64_t) (zs[1 + cz] * (uint32_t) A.Ys)) * sizeof(E))),
+					  ys[1 + cy]);
+	}
+};
+
+// neighbours<AA> of a per-lane coordinate in 32 bits (extents below 2^30)
+template <bool AA>
+LBM_DEV void neighbours32(uint32_t* r, int32_t c, int32_t n, int32_t o, bool dist, bool periodic)
+{
+	const int32_t pw = (! dist && c == n - 1) ? 0 : c + 1, mw = (! dist && c == 0) ? n - 1 : c - 1;
+	const int32_t pc = AA ? (c + 1 < n + o ? c + 1 : 0) : (c + 1 < n - 1 + o ? c + 1 : n - 1 + o);
+	const int32_t mc = AA ? (c - 1 >= -o ? c - 1 : n - 1) : (c - 1 > -o ? c - 1 : -o);
+	r[0] = (uint32_t) ((periodic ? mw : mc) + o);
+	r[1] = (uint32_t) (c + o);
+	r[2] = (uint32_t) ((periodic ? pw : pc) + o);
+}
+
+// A wave-uniform value the compiler may not form ahead of this point: the scalar
+// bases of 27 directions, hoisted out of a loop or above the collision, would
+// spill.
+template <typename T>
+LBM_DEV T here(T v)
+{
+	asm volatile("" : "+s"(v));
+	return v;
+}
+template <int ST, int MODE, bool LIN, bool NTG, bool ADE>
+LBM_DEV void lean_site(const StepArgs& A, const AdeArgs& B)
+{
+	using S = Storage<ST>;
+	using real = typename S::real;
+	using elem = typename S::elem;
+	constexpr int COLL = TNL_LBM_COLL_CUM;
+	constexpr bool AA = MODE != LEAN_AB;
+	constexpr bool NT = NTG && ((LBM_NT_GENERAL >> ST) & 1);
+	int64_t x, z, y;
+	if (! box_coords<LIN>(A, x, z, y))
+		return;
+	const int64_t s0 = ((x + A.ox) * A.Zs + (z + A.oz)) * A.Ys + (y + A.oy);
+	const int16_t gi = A.map ? A.map[s0] : (int16_t) GEO_PERIODIC;
+	const int16_t ga = ADE && B.map ? B.map[s0] : (int16_t) A_PERIODIC;
+	const bool per = gi == GEO_PERIODIC, wall = gi == GEO_WALL;
+	const bool mine = plain(gi) && plain_scalar(ga);
+	const Nb XW = neighbours<AA>(x, A.X, A.ox, A.dist_x, true), XC = neighbours<AA>(x, A.X, A.ox, A.dist_x, false);
+	const Nb ZW = neighbours<AA>(z, A.Z, A.oz, A.dist_z, true), ZC = neighbours<AA>(z, A.Z, A.oz, A.dist_z, false);
+	bool same = MODE == LEAN_EVEN || (XW.m == XC.m && XW.p == XC.p);
+	if (! LIN && MODE != LEAN_EVEN)
+		same = same && ZW.m == ZC.m && ZW.p == ZC.p;
+	auto kind = [&](const Nb& NX, const Nb& NZ) __attribute__((always_inline)) {
+		Stencil<LIN> N;
+		const uint64_t pb = here(A.plane_bytes);
+		const uint64_t plane = (uint64_t) (A.Zs * A.Ys);
+		N.xoff[0] = NX.m * plane;
+		N.xoff[1] = NX.o * plane;
+		N.xoff[2] = NX.p * plane;
+		// (formed here: the offsets of both kinds would stay live)
+		int32_t yl = (int32_t) y;
+		asm volatile("" : "+v"(yl));
+		neighbours32<AA>(N.ys, yl, (int32_t) A.Y, (int32_t) A.oy, A.dist_y, per);
+		if constexpr (LIN) {
+			int32_t zl = (int32_t) z;
+			asm volatile("" : "+v"(zl));
+			neighbours32<AA>(N.zr, zl, (int32_t) A.Z, (int32_t) A.oz, A.dist_z, per);
+#pragma unroll
+			for (int c = 0; c < 3; c++)
+				N.zr[c] *= (uint32_t) A.Ys;
+		}
+		else {
+			N.zs[0] = (uint32_t) NZ.m;
+			N.zs[1] = (uint32_t) NZ.o;
+			N.zs[2] = (uint32_t) NZ.p;
+		}
+		// the slot of population q pulled here, and pushed
+		auto src = [&](const elem* base, int q) {
+			if constexpr (MODE == LEAN_EVEN)
+				return N.slot(base, pb, A, q, 0, 0, 0);
+			else
+				return N.slot(base, pb, A, MODE == LEAN_ODD ? opp(q) : q, -CX[q], -CY[q], -CZ[q]);
+		};
+		auto dst = [&](elem* base, uint64_t pbo, int q) {
+			if constexpr (MODE == LEAN_ODD)
+				return N.slot(base, pbo, A, q, CX[q], CY[q], CZ[q]);
+			else
+				return N.slot(base, pbo, A, MODE == LEAN_EVEN ? opp(q) : q, 0, 0, 0);
+		};
+		AdeIn<ST> in;
+		N.local();
+		if constexpr (ADE) {
+			const elem* acur = (const elem*) here((char*) B.df0);
+			ade_load<ST, true>(A, B, N.own(A), ga,
+							   [&](int q, real pr, real isc) {
+								   return ade_get<ST>(src(acur, q), MODE == LEAN_ODD ? opp(q) : q, pr, isc,
+													  NT && (MODE == LEAN_EVEN || CY[q] == 0));
+							   },
+							   in);
+			N.local();
+		}
+		real f[27];
+		const elem* cur = (const elem*) here((char*) A.df0);
+#pragma unroll
+		for (int q = 0; q < 27; q++) {
+			const elem* p = src(cur, q);
+			const elem v = NT && (MODE == LEAN_EVEN || CY[q] == 0) ? ld_nt(p) : *p;
+			f[q] = S::ld(&v, A.cls_sc[ncls(q)]);
+		}
+		auto put = [&](elem* out, uint64_t pbo, int q, elem e) {
+			elem* p = dst(out, pbo, q);
+			if (NT && (MODE != LEAN_ODD || CY[q] == 0))
+				st_nt(p, e);
+			else
+				*p = e;
+		};
+		real rho = 1, vx = 0, vy = 0, vz = 0;
+		real Fx = (real) here(A.fx), Fy = (real) here(A.fy), Fz = (real) here(A.fz);
+		if (A.force)
+			add_site_force(A, N.own(A), Fx, Fy, Fz);
+		if (wall)
+			bounce_back<ST, COLL>(f);
+		if (! wall)
+			collide_site<ST, COLL>(f, A, Fx, Fy, Fz, rho, vx, vy, vz);
+		elem* out = (elem*) after<true>((char*) (AA ? A.df0 : A.df1), f[26]);
+		const uint64_t pbo = here(A.plane_bytes);
+		N.local();
+		encode_all<ST, COLL>(f, A, [&](int q, elem e) { put(out, pbo, q, e); });
+		if (A.out_macro)
+			write_macro(A, N.own(A), rho, vx, vy, vz);
+		if constexpr (ADE) {
+			real g[7];
+			const real phi = ade_update<ST, true>(B, in, vx, vy, vz, g);
+			elem* aout = (elem*) after<true>((char*) (AA ? B.df0 : B.df1), g[6]);
+			const real pr = (real) B.phi_ref, sc = (real) B.scale;
+			const uint64_t pbo = here(A.plane_bytes);
+			N.local();
+#pragma unroll
+			for (int q = 0; q < 7; q++)
+				ade_put<ST>(dst(aout, pbo, q), MODE == LEAN_EVEN ? opp(q) : q, g[q], pr, sc, NT && (MODE != LEAN_ODD || CY[q] == 0));
+			write_phi<ST>(A, B, N.own(A), phi);
+		}
+	};
+	if (mine && (same || per))
+		kind(XW, ZW);
+	if (! same && mine && ! per)
+		kind(XC, ZC);
+}
+
+template <int ST, int MODE, bool LIN, bool NTG>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ST == TNL_LBM_STORE_F64 ? 3 : 4, 8)))
+k_lean(const StepArgs A)
+{
+	lean_site<ST, MODE, LIN, NTG, false>(A, AdeArgs{});
+}
+template <int ST, int MODE, bool LIN, bool NTG>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ST == TNL_LBM_STORE_F64 ? 3 : 4, 8)))
+k_lean_ade(const StepArgs A, const AdeArgs B)
+{
+	lean_site<ST, MODE, LIN, NTG, true>(A, B);
 }
 
 template <int ST>
@@ -1707,33 +2018,20 @@ inline void list_shape(StepArgs& A, const uint32_t* rows, uint32_t nrows, unsign
 	grid = padded;
 }
 
-// The row lists of a full-box step: one launch per non-empty list, the lean
-// kernels (LEAN 1, 2) for classes 1 and 2 and the general paths over a list
-// (LEAN 3) for class 0.  go(B, threads, grid, lean) makes one launch.
-template <typename Go>
-int for_row_lists(const StepArgs& A, Go&& go)
-{
-	int64_t off = 0;
-	for (int c = 0; c < 3; c++) {
-		const int64_t n = A.list_count[c];
-		if (n > 0) {
-			StepArgs B = A;
-			unsigned threads = 0, grid = 0;
-			list_shape(B, A.lists + off, (uint32_t) n, threads, grid);
-			if (int rc = go(B, threads, grid, c == 0 ? 3 : c))
-				return rc;
-		}
-		off += n;
-	}
-	return 0;
-}
-
 // Whether the populations fit the 256 MiB last-level cache, where one step
 // finds what the step before it wrote; nontemporal accesses give that up
 // (300x50x300 F16, 243 MB: 204 us for the two steps with them, 153 without).
-inline bool cache_resident(const StepArgs& A)
+inline bool cache_resident(const StepArgs& A, uint64_t planes = 27)
 {
-	return 27 * A.plane_bytes <= (256ull << 20);
+	return planes * A.plane_bytes <= (256ull << 20);
+}
+// Whether a step over `planes` population planes in all hints the streams that
+// no other wave touches: rows and planes start on lines, and the arrays exceed
+// the last-level cache.
+inline bool hint_streams(const StepArgs& A, uint64_t planes, size_t elem)
+{
+	return ! cache_resident(A, planes) && A.plane_bytes % 128 == 0 && (uintptr_t) A.df0 % 128 == 0
+		&& (uintptr_t) A.df1 % 128 == 0 && (uint64_t) A.Ys * elem % 128 == 0;
 }
 
 // Launch shape of an even A-A step with `per` sites per lane: the contiguous
@@ -1769,7 +2067,14 @@ inline bool even_shape(StepArgs& A, uint32_t per, unsigned most, unsigned& threa
 	return whole;
 }
 
-template <int ST, int COLL>
+// Whether rows in which walls and other sites may meet are common (class 2, an
+// eighth of the rows or more): the pairs of such rows would be split
+inline bool mixed_rows(const StepArgs& A)
+{
+	return A.list_count[2] * 8 > A.X * A.Z;
+}
+
+template <int ST, int COLL, bool MAP = false>
 int even_launch(const StepArgs& A0, hipStream_t st)
 {
 	constexpr size_t E = sizeof(typename Storage<ST>::elem);
@@ -1782,18 +2087,18 @@ int even_launch(const StepArgs& A0, hipStream_t st)
 		// operations round 1 in 10^4 of them to the neighbouring unit)
 		const bool flat = ! Storage<ST>::fixed && A.oy == 0 && A.oz == 0 && A.ny == A.Y && A.nz == A.Z;
 		const int64_t odd = flat ? ((A.offx + A.ox) * A.Y * A.Z) | (A.nx * A.Y * A.Z) : A.ny | A.offy | A.oy | A.Y;
-		if (! ((odd | A.XYZ) & 1) && ! ((uintptr_t) A.df0 & 3)) {
+		if (! ((odd | A.XYZ) & 1) && ! ((uintptr_t) A.df0 & 3) && ! (MAP && mixed_rows(A))) {
 			if (even_shape(A, 2, 256, threads, grid, E))
-				hipLaunchKernelGGL((k_aa_even_pair<ST, COLL, true>), dim3(grid), dim3(threads), 0, st, A);
+				hipLaunchKernelGGL((k_aa_even_pair<ST, COLL, true, MAP>), dim3(grid), dim3(threads), 0, st, A);
 			else
-				hipLaunchKernelGGL((k_aa_even_pair<ST, COLL, false>), dim3(grid), dim3(threads), 0, st, A);
+				hipLaunchKernelGGL((k_aa_even_pair<ST, COLL, false, MAP>), dim3(grid), dim3(threads), 0, st, A);
 			return hip_check(hipGetLastError(), "step launch");
 		}
 	}
 	if (even_shape(A, 1, ST == TNL_LBM_STORE_F64 ? 256 : LBM_TPB_FP32, threads, grid, E))
-		hipLaunchKernelGGL((k_aa_even<ST, COLL, true>), dim3(grid), dim3(threads), 0, st, A);
+		hipLaunchKernelGGL((k_aa_even<ST, COLL, true, MAP>), dim3(grid), dim3(threads), 0, st, A);
 	else
-		hipLaunchKernelGGL((k_aa_even<ST, COLL, false>), dim3(grid), dim3(threads), 0, st, A);
+		hipLaunchKernelGGL((k_aa_even<ST, COLL, false, MAP>), dim3(grid), dim3(threads), 0, st, A);
 	return hip_check(hipGetLastError(), "step launch");
 }
 
@@ -1836,31 +2141,87 @@ int launch_periodic(const StepArgs& A, unsigned threads, unsigned grid, hipStrea
 	// nontemporal hints on the c_y = 0 accesses where rows start on lines, as
 	// in even_shape (301x187x129 FP64, both steps: 1428 us with them, 1377
 	// without; 512^3: 18.79 and 18.96 ms)
-	const bool nt = ! cache_resident(A) && A.plane_bytes % 128 == 0 && (uintptr_t) A.df0 % 128 == 0
-				 && (uint64_t) A.Ys * sizeof(typename Storage<ST>::elem) % 128 == 0;
-	if (nt)
+	if (hint_streams(A, 27, sizeof(typename Storage<ST>::elem)))
 		odd_launch<ST, COLL, true>(A, threads, grid, st);
 	else
 		odd_launch<ST, COLL, false>(A, threads, grid, st);
 	return hip_check(hipGetLastError(), "step launch");
 }
 
-// One launch of the map kernel at lean level LEAN (k_general)
-template <int ST, int COLL, int LEAN>
-void launch_general(int pattern, const StepArgs& B, unsigned threads, unsigned grid, hipStream_t st, bool o32)
+// Whether a full-box launch with row lists takes the lean kernels: x planes
+// within 32-bit offsets, and few rows with other codes (each of those is read
+// again by the general kernel; from an eighth of the rows on, that launch costs
+// what the lean one saves)
+inline bool lean_split(const StepArgs& A, size_t elem)
 {
-	if (o32) {
-		if constexpr (sizeof(typename Storage<ST>::elem) == 2) {
-			if (pattern == TNL_LBM_PATTERN_AA)
-				hipLaunchKernelGGL((k_general<ST, COLL, TNL_LBM_PATTERN_AA, 0, true, LEAN>), dim3(grid), dim3(threads), 0, st, B);
-			else
-				hipLaunchKernelGGL((k_general<ST, COLL, TNL_LBM_PATTERN_AB, 0, true, LEAN>), dim3(grid), dim3(threads), 0, st, B);
+	const int64_t rows = A.list_count[0] + A.list_count[1] + A.list_count[2];
+	return A.lists && narrow_planes(A, elem) && rows == A.X * A.Z && A.list_count[0] * 8 <= rows;
+}
+
+// Launch shape of a lean kernel: rows of whole blocks with hints, else the
+// linear mapping without.  go(shape, threads, grid, lin).
+template <typename Go>
+void lean_shape(const StepArgs& A0, uint64_t planes, size_t elem, Go&& go)
+{
+	StepArgs A = A0;
+	A.rows = nullptr;
+	unsigned threads = A.ny > 128 ? 256 : (A.ny > 64 ? 128 : 64);
+	const bool lin = A.ny % (int32_t) threads || ! hint_streams(A, planes, elem);
+	if (lin) {
+		const uint64_t plane = (uint64_t) A.ny * (uint64_t) A.nz;
+		threads = 256;
+		while (threads > 64 && plane * (uint64_t) A.nx < (uint64_t) threads * 2048)
+			threads /= 2;
+		A.nyb = (uint32_t) ((plane + threads - 1) / threads);
+		A.nblocks = A.nyb * (uint32_t) A.nx;
+	}
+	else {
+		A.nyb = (uint32_t) A.ny / threads;
+		A.nblocks = A.nyb * (uint32_t) A.nz * (uint32_t) A.nx;
+	}
+	const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
+	A.per_xcd = padded / NXCD;
+	go(A, threads, padded, lin);
+}
+
+template <int ST, int MODE>
+void lean_launch(const StepArgs& A, hipStream_t st)
+{
+	lean_shape(A, MODE == LEAN_AB ? 54 : 27, sizeof(typename Storage<ST>::elem),
+			   [&](const StepArgs& C, unsigned t, unsigned g, bool lin) {
+				   if (lin)
+					   hipLaunchKernelGGL((k_lean<ST, MODE, true, false>), dim3(g), dim3(t), 0, st, C);
+				   else
+					   hipLaunchKernelGGL((k_lean<ST, MODE, false, true>), dim3(g), dim3(t), 0, st, C);
+			   });
+}
+
+// One launch of the map kernel
+template <int ST, int COLL, bool LISTED>
+void launch_general(int pattern, const StepArgs& B, unsigned threads, unsigned grid, hipStream_t st)
+{
+	constexpr bool two = sizeof(typename Storage<ST>::elem) == 2;
+	// 2-byte forms: 32-bit slot offsets where a population array is under
+	// 4 GiB (F16 384^3 channel: A-A 1821 -> 1430 us, 139 -> 106 VGPRs;
+	// A-B -2%; neutral for the 4- and 8-byte forms, which keep 64-bit)
+	const bool o32 = two && narrow_slots(B.XYZ, sizeof(typename Storage<ST>::elem));
+	const bool nt = ! LISTED && pattern == TNL_LBM_PATTERN_AB && hint_streams(B, 54, sizeof(typename Storage<ST>::elem));
+	auto go = [&](auto oc) {
+		constexpr bool O32 = decltype(oc)::value;
+		if (pattern == TNL_LBM_PATTERN_AA)
+			hipLaunchKernelGGL((k_general<ST, COLL, TNL_LBM_PATTERN_AA, 0, O32, LISTED>), dim3(grid), dim3(threads), 0, st, B);
+		else if (! nt)
+			hipLaunchKernelGGL((k_general<ST, COLL, TNL_LBM_PATTERN_AB, 0, O32, LISTED>), dim3(grid), dim3(threads), 0, st, B);
+		else if constexpr (! LISTED)
+			hipLaunchKernelGGL((k_general<ST, COLL, TNL_LBM_PATTERN_AB, 0, O32, false, true>), dim3(grid), dim3(threads), 0, st, B);
+	};
+	if constexpr (two) {
+		if (o32) {
+			go(std::true_type{});
+			return;
 		}
 	}
-	else if (pattern == TNL_LBM_PATTERN_AA)
-		hipLaunchKernelGGL((k_general<ST, COLL, TNL_LBM_PATTERN_AA, 0, false, LEAN>), dim3(grid), dim3(threads), 0, st, B);
-	else
-		hipLaunchKernelGGL((k_general<ST, COLL, TNL_LBM_PATTERN_AB, 0, false, LEAN>), dim3(grid), dim3(threads), 0, st, B);
+	go(std::false_type{});
 }
 
 template <int ST, int COLL>
@@ -1869,32 +2230,30 @@ int launch_step(const tnl_lbm_config* cfg, const StepArgs& A, unsigned threads, 
 	// the map-free periodic kernels take the homogeneous force only
 	if (! A.map && ! A.force && cfg->pattern == TNL_LBM_PATTERN_AA)
 		return launch_periodic<ST, COLL>(A, threads, grid, st);
-	// 2-byte forms: 32-bit slot offsets where a population array is under
-	// 4 GiB (F16 384^3 channel: A-A 1821 -> 1430 us, 139 -> 106 VGPRs;
-	// A-B -2%; neutral for the 4- and 8-byte forms, which keep 64-bit)
-	bool o32 = false;
-	if constexpr (sizeof(typename Storage<ST>::elem) == 2)
-		o32 = narrow_slots(A.XYZ, sizeof(typename Storage<ST>::elem));
-	// row lists for the deviation forms, whose map kernel is bound by its
-	// registers and instruction issue (384^3 with z walls, lean against
-	// general: I16 -22%, F16 A-B -8%, BF16 -6%, F32_DEV -2%); the F64 and F32
-	// map kernels gain nothing, and a class-0 list costs them an extra launch
-	// (C4 duct +4 to +6%)
-	if constexpr (COLL == TNL_LBM_COLL_CUM && Storage<ST>::dev) {
-		if (A.lists)
-			return for_row_lists(A, [&](const StepArgs& B, unsigned t, unsigned g, int lean) {
-				if (lean == 1)
-					launch_general<ST, COLL, 1>(cfg->pattern, B, t, g, st, o32);
-				else if (lean == 2)
-					launch_general<ST, COLL, 2>(cfg->pattern, B, t, g, st, o32);
-				else
-					launch_general<ST, COLL, 3>(cfg->pattern, B, t, g, st, o32);
-				return hip_check(hipGetLastError(), "step launch");
-			});
+	// The lean kernels for the plain sites, then the rows that hold others.
+	// The A-B steps of FP64 and F32 take them where there are none such: their
+	// map kernel is bound by HBM, and the second launch costs more than it gains.
+	if constexpr (COLL == TNL_LBM_COLL_CUM) {
+		if (lean_split(A, sizeof(typename Storage<ST>::elem)) && (Storage<ST>::dev || cfg->pattern == TNL_LBM_PATTERN_AA || A.list_count[0] == 0)) {
+			if (cfg->pattern == TNL_LBM_PATTERN_AB)
+				lean_launch<ST, LEAN_AB>(A, st);
+			else if (! A.even)
+				lean_launch<ST, LEAN_ODD>(A, st);
+			else if (int rc = even_launch<ST, COLL, true>(A, st))
+				return rc;
+			if (int rc = hip_check(hipGetLastError(), "step launch"))
+				return rc;
+			if (A.list_count[0] > 0) {
+				StepArgs B = A;
+				list_shape(B, A.lists, (uint32_t) A.list_count[0], threads, grid);
+				launch_general<ST, COLL, true>(cfg->pattern, B, threads, grid, st);
+			}
+			return hip_check(hipGetLastError(), "step launch");
+		}
 	}
 	StepArgs B = A;
 	linearize(B, threads, grid);
-	launch_general<ST, COLL, 0>(cfg->pattern, B, threads, grid, st, o32);
+	launch_general<ST, COLL, false>(cfg->pattern, B, threads, grid, st);
 	return hip_check(hipGetLastError(), "step launch");
 }
 
