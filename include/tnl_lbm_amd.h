@@ -387,7 +387,8 @@ int tnl_lbm_d3q27_reduce_gradients(const tnl_lbm_config* cfg, const tnl_lbm_d3q2
  * Replaces the per-slot DistributedNDArraySynchronizer passes of
  * lbm_block.hpp:434-470 (sync directions df_sync_directions, defs.h:352-385,
  * reversed on even A-A steps and shifted by one site on odd ones).  The
- * copies are asynchronous on `stream`; the two lattices may live on
+ * copies are asynchronous on `stream`, one launch where both lattices are on
+ * its GPU; they may also live on
  * different GPUs that have peer access.  Both must have the same Y, Z, oy,
  * oz and storage form.                                                      */
 enum tnl_lbm_halo_phase { TNL_LBM_HALO_PULL = 0, TNL_LBM_HALO_PUSH = 1 };
