@@ -21,6 +21,7 @@
 #include <mutex>
 #include <string>
 #include <type_traits>
+#include <vector>
 
 #include "lbm_adjoint.hpp"
 #include "lbm_step.hpp"
@@ -202,6 +203,94 @@ static int scratch_address(double** out)
 	}
 	*out = g_scratch_addr[dev];
 	return TNL_LBM_OK;
+}
+
+// ---- FP64 reductions ---------------------------------------------------------
+// Buffers of the FP64 reductions that return to the host: the partial sums
+// (device) and the results (pinned host memory that the last kernel writes
+// itself: no copy to wait for).  A reduction takes a pair for its duration and,
+// having synchronised its stream, gives it back, so there are as many as
+// reductions have ever run at once on a device (49 KB each), held until the
+// process ends.
+constexpr int RED_ROWS = RED_BLOCKS * RED_N > GRAD_BLOCKS * 2 ? RED_BLOCKS * RED_N : GRAD_BLOCKS * 2;
+struct RedBuffers
+{
+	double* partial = nullptr;
+	double* out = nullptr;
+};
+class RedLease
+{
+public:
+	RedBuffers b;
+	int take()
+	{
+		if (int rc = hip_check(hipGetDevice(&dev), "hipGetDevice"))
+			return rc;
+		if (dev < 0 || dev >= MAX_DEVICES)
+			return fail(TNL_LBM_ERR_ARG, "device ordinal beyond the reduction buffers' table");
+		{
+			std::lock_guard<std::mutex> lock(mutex());
+			auto& spare = list()[dev];
+			if (! spare.empty()) {
+				b = spare.back();
+				spare.pop_back();
+				return TNL_LBM_OK;
+			}
+		}
+		if (int rc = hip_check(hipMalloc(&b.partial, sizeof(double) * RED_ROWS), "hipMalloc reduce buffer"))
+			return rc;
+		if (int rc = hip_check(hipHostMalloc(&b.out, sizeof(double) * RED_N), "hipHostMalloc reduce result")) {
+			(void) hipFree(b.partial);
+			return rc;
+		}
+		return TNL_LBM_OK;
+	}
+	// after the stream has been synchronised
+	void give_back()
+	{
+		std::lock_guard<std::mutex> lock(mutex());
+		list()[dev].push_back(b);
+	}
+
+private:
+	static constexpr int MAX_DEVICES = 64;
+	int dev = -1;
+	// never destroyed: a reduction may run while static objects are
+	static std::mutex& mutex()
+	{
+		static std::mutex& m = *new std::mutex;
+		return m;
+	}
+	static std::vector<RedBuffers>* list()
+	{
+		static auto* l = new std::vector<RedBuffers>[MAX_DEVICES];
+		return l;
+	}
+};
+
+template <typename Launch>
+static int reduce_to_host(hipStream_t st, double* out, int n, Launch&& launch)
+{
+	RedLease lease;
+	if (int rc = lease.take())
+		return rc;
+	// (after an error the buffers may still be in use: they are not taken again)
+	if (int rc = launch(lease.b.partial, lease.b.out))
+		return rc;
+	if (int rc = hip_check(hipStreamSynchronize(st), "reduce sync"))
+		return rc;
+	for (int i = 0; i < n; i++)
+		out[i] = lease.b.out[i];
+	lease.give_back();
+	return TNL_LBM_OK;
+}
+
+// the six sums of the macro field -> out (device-visible) on `st`
+static int launch_reduce_macro(const MacroArgs& M, double* partial, double* out, hipStream_t st)
+{
+	hipLaunchKernelGGL(k_reduce_macro, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, st, M, partial);
+	hipLaunchKernelGGL((k_reduce_final<RED_N, RED_BLOCKS>), dim3(1), dim3(1024), 0, st, (const double*) partial, out);
+	return hip_check(hipGetLastError(), "reduce launch");
 }
 
 // ---- x-slab halo ------------------------------------------------------------
@@ -780,34 +869,6 @@ int tnl_lbm_d3q27_halo_x(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* lo
 	return TNL_LBM_OK;
 }
 
-// Partial sums of the FP64 reductions: one buffer per (host thread,
-// device), allocated on that thread's first reduction on the device and held
-// until the process ends (RED_BLOCKS + 1 rows of RED_N doubles, 49 KB).
-// Each reduction synchronises its stream before it returns, so the next one
-// of the same thread may reuse the buffer on any stream.
-static int partial_buffer(double** out)
-{
-	constexpr int MAX_DEVICES = 64;
-	static thread_local double* bufs[MAX_DEVICES] = {};
-	int dev = 0;
-	if (int rc = hip_check(hipGetDevice(&dev), "hipGetDevice"))
-		return rc;
-	if (dev < 0 || dev >= MAX_DEVICES)
-		return fail(TNL_LBM_ERR_ARG, "device ordinal beyond the reduction buffers' table");
-	if (! bufs[dev])
-		if (int rc = hip_check(hipMalloc(&bufs[dev], sizeof(double) * (RED_BLOCKS * RED_N + RED_N)), "hipMalloc reduce buffer"))
-			return rc;
-	*out = bufs[dev];
-	return TNL_LBM_OK;
-}
-
-// partial sums -> out (device) on `st`
-static int finish_reduction(double* partial, double* out_dev, hipStream_t st)
-{
-	hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, st, (const double*) partial, RED_BLOCKS, out_dev);
-	return hip_check(hipGetLastError(), "reduce launch");
-}
-
 static int reduction_args(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* SD, MacroArgs& M)
 {
 	if (int rc = validate(cfg, SD))
@@ -826,16 +887,8 @@ int tnl_lbm_d3q27_reduce_macro(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_da
 		return rc;
 	if (! out)
 		return fail(TNL_LBM_ERR_NULL, "output missing");
-	double* partial = nullptr;
-	if (int rc = partial_buffer(&partial))
-		return rc;
 	hipStream_t st = (hipStream_t) stream;
-	hipLaunchKernelGGL(k_reduce_macro, dim3(RED_BLOCKS), dim3(256), 0, st, M, partial);
-	if (int rc = finish_reduction(partial, partial + RED_BLOCKS * RED_N, st))
-		return rc;
-	if (int rc = hip_check(hipMemcpyAsync(out, partial + RED_BLOCKS * RED_N, sizeof(double) * RED_N, hipMemcpyDeviceToHost, st), "reduce copy"))
-		return rc;
-	return hip_check(hipStreamSynchronize(st), "reduce sync");
+	return reduce_to_host(st, out, RED_N, [&](double* partial, double* res) { return launch_reduce_macro(M, partial, res, st); });
 }
 
 int tnl_lbm_d3q27_reduce_macro_noalloc(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* SD, double* out_device,
@@ -847,17 +900,12 @@ int tnl_lbm_d3q27_reduce_macro_noalloc(const tnl_lbm_config* cfg, const tnl_lbm_
 	if (! out_device)
 		return fail(TNL_LBM_ERR_NULL, "device output missing");
 	// every one of the RED_BLOCKS workgroups writes its own partial row, so
-	// nothing in the scratch needs clearing; the grid never exceeds the rows
+	// nothing in the scratch needs clearing
 	static_assert(RED_BLOCKS <= SCRATCH_ROWS, "the reduction grid must fit the scratch");
-	const int blocks = RED_BLOCKS;
-	if (blocks > SCRATCH_ROWS)
-		return fail(TNL_LBM_ERR_DIMS, "reduction grid larger than the scratch (1024 partial rows)");
 	double* partial = nullptr;
 	if (int rc = scratch_address(&partial))
 		return rc;
-	hipStream_t st = (hipStream_t) stream;
-	hipLaunchKernelGGL(k_reduce_macro, dim3(blocks), dim3(256), 0, st, M, partial);
-	return finish_reduction(partial, out_device, st);
+	return launch_reduce_macro(M, partial, out_device, (hipStream_t) stream);
 }
 
 int tnl_lbm_d3q27_reduce_gradients(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* SD, uint32_t flags, double out[2],
@@ -873,21 +921,23 @@ int tnl_lbm_d3q27_reduce_gradients(const tnl_lbm_config* cfg, const tnl_lbm_d3q2
 	M.dist_z = (flags & TNL_LBM_FLAG_DISTRIBUTED_Z) != 0;
 	if ((M.dist_x && SD->ox < 1) || (M.dist_y && SD->oy < 1) || (M.dist_z && SD->oz < 1))
 		return fail(TNL_LBM_ERR_DIMS, "a distributed axis needs an overlap of at least one site");
-	double* partial = nullptr;
-	if (int rc = partial_buffer(&partial))
-		return rc;
 	hipStream_t st = (hipStream_t) stream;
-	hipLaunchKernelGGL(k_reduce_gradients, dim3(RED_BLOCKS), dim3(256), 0, st, M, partial);
-	if (int rc = finish_reduction(partial, partial + RED_BLOCKS * RED_N, st))
-		return rc;
-	double res[RED_N];
-	if (int rc = hip_check(hipMemcpyAsync(res, partial + RED_BLOCKS * RED_N, sizeof(double) * RED_N, hipMemcpyDeviceToHost, st), "reduce copy"))
-		return rc;
-	if (int rc = hip_check(hipStreamSynchronize(st), "reduce sync"))
-		return rc;
-	out[0] = res[0];
-	out[1] = res[1];
-	return TNL_LBM_OK;
+	return reduce_to_host(st, out, 2, [&](double* partial, double* res) {
+		const GradShape g = grad_shape(M);
+		auto go = [&](auto t) {
+			using T = decltype(t);
+			if ((uint64_t) M.Zs * (uint64_t) M.Ys * sizeof(T) <= (1ull << 32))
+				hipLaunchKernelGGL((k_reduce_gradients<T, uint32_t>), dim3(GRAD_BLOCKS), dim3(RED_THREADS), 0, st, M, g, partial);
+			else
+				hipLaunchKernelGGL((k_reduce_gradients<T, uint64_t>), dim3(GRAD_BLOCKS), dim3(RED_THREADS), 0, st, M, g, partial);
+		};
+		if (M.macro_f64)
+			go(double{});
+		else
+			go(float{});
+		hipLaunchKernelGGL((k_reduce_final<2, GRAD_BLOCKS>), dim3(1), dim3(1024), 0, st, (const double*) partial, res);
+		return hip_check(hipGetLastError(), "reduce launch");
+	});
 }
 
 }  // extern "C"

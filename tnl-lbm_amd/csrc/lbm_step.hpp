@@ -1863,26 +1863,33 @@ __global__ void k_transfer(void* df, double* buf, int64_t XYZ, int64_t nsites, c
 // FP64 reductions over the macro field: deterministic two-pass block sums
 constexpr int RED_N = 6;
 constexpr int RED_BLOCKS = 1024;
+constexpr unsigned RED_THREADS = 256;
 
-__device__ void block_sum(double* v, double (*sh)[RED_N])
+// v[0..N) summed over the block, in thread 0: shuffles within each wave, the
+// waves' sums through LDS (blocks of up to 16 whole waves)
+template <int N>
+__device__ void block_sum(double* v)
 {
-	const int t = threadIdx.x;
+	__shared__ double sh[16][N];
+	const unsigned t = threadIdx.x;
 #pragma unroll
-	for (int i = 0; i < RED_N; i++)
-		sh[t][i] = v[i];
+	for (int i = 0; i < N; i++)
+		for (int d = 32; d >= 1; d >>= 1)
+			v[i] += __shfl_xor(v[i], d);
+	if ((t & 63) == 0)
+#pragma unroll
+		for (int i = 0; i < N; i++)
+			sh[t >> 6][i] = v[i];
 	__syncthreads();
-	for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-		if (t < w)
+	if (t == 0)
+		for (unsigned w = 1; w < blockDim.x / 64; w++)
 #pragma unroll
-			for (int i = 0; i < RED_N; i++)
-				sh[t][i] += sh[t + w][i];
-		__syncthreads();
-	}
+			for (int i = 0; i < N; i++)
+				v[i] += sh[w][i];
 }
 
-static __global__ void __launch_bounds__(256) k_reduce_macro(const MacroArgs A, double* partial)
+static __global__ void __launch_bounds__(RED_THREADS) k_reduce_macro(const MacroArgs A, double* partial)
 {
-	__shared__ double sh[256][RED_N];
 	double v[RED_N] = {0, 0, 0, 0, 0, 0};
 	const int64_t N = A.X * A.Y * A.Z;
 	for (int64_t n = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; n < N; n += (int64_t) gridDim.x * blockDim.x) {
@@ -1905,11 +1912,11 @@ static __global__ void __launch_bounds__(256) k_reduce_macro(const MacroArgs A, 
 		v[4] += u2;
 		v[5] += 1.0;
 	}
-	block_sum(v, sh);
+	block_sum<RED_N>(v);
 	if (threadIdx.x == 0)
 #pragma unroll
 		for (int i = 0; i < RED_N; i++)
-			partial[blockIdx.x * RED_N + i] = sh[0][i];
+			partial[blockIdx.x * RED_N + i] = v[i];
 }
 
 // Velocity-gradient reductions of sim_4.cu:282-300: with the central
@@ -1918,59 +1925,120 @@ static __global__ void __launch_bounds__(256) k_reduce_macro(const MacroArgs A, 
 // overlap layer on one that is), per block:
 //   [0] sum rho |G|^2       (the enstrophy integrand of sim_4.cu:284-298)
 //   [1] sum rho |curl v|^2  (computeVorticity, sim_4.cu:62-82)
-// entries 2..5 of each partial row are zero.
-static __global__ void __launch_bounds__(256) k_reduce_gradients(const MacroArgs A, double* partial)
+//
+// A lane owns one (y, z) column of a segment of `len` x planes and walks it, the
+// velocities at x - 1 and x in registers, so that a plane is fetched once a
+// segment; the y and z neighbours of a plane are the columns of the same block
+// and of the next ones, found in L1 and (blocks of an XCD being consecutive) its
+// L2.  Item = (segment, 256 columns).  192^3 FP64:
+// 99 us with all 18 neighbours of a site loaded for it and its coordinates divided
+// out of its index, 66 to 83 us so (2.8 to 3.4 TB/s; the slower after a step that
+// leaves dirty lines in the last-level cache).  Bound: the latency of the loads.
+// as many blocks as run at once at 74 VGPRs, six waves per SIMD (at 64 VGPRs, eight
+// waves, it spills: 106 us against 79)
+constexpr int GRAD_BLOCKS = 1536;
+struct GradShape
 {
-	__shared__ double sh[256][RED_N];
-	double v[RED_N] = {0, 0, 0, 0, 0, 0};
-	const int64_t N = A.X * A.Y * A.Z;
-	auto at = [&](int id, int64_t x, int64_t y, int64_t z) -> double {
-		const int64_t s = (int64_t) id * A.XYZ + ((x + A.ox) * A.Zs + (z + A.oz)) * A.Ys + (y + A.oy);
-		return A.macro_f64 ? ((const double*) A.macro)[s] : (double) ((const float*) A.macro)[s];
-	};
-	for (int64_t n = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; n < N; n += (int64_t) gridDim.x * blockDim.x) {
-		const int64_t y = n % A.Y, t = n / A.Y, z = t % A.Z, x = t / A.Z;
-		const int64_t xp = (! A.dist_x && x == A.X - 1) ? 0 : x + 1, xm = (! A.dist_x && x == 0) ? A.X - 1 : x - 1;
-		const int64_t yp = (! A.dist_y && y == A.Y - 1) ? 0 : y + 1, ym = (! A.dist_y && y == 0) ? A.Y - 1 : y - 1;
-		const int64_t zp = (! A.dist_z && z == A.Z - 1) ? 0 : z + 1, zm = (! A.dist_z && z == 0) ? A.Z - 1 : z - 1;
-		double G[3][3];  // G[a][b] = d v_a / d x_b
-#pragma unroll
-		for (int a = 0; a < 3; a++) {
-			G[a][0] = 0.5 * (at(1 + a, xp, y, z) - at(1 + a, xm, y, z));
-			G[a][1] = 0.5 * (at(1 + a, x, yp, z) - at(1 + a, x, ym, z));
-			G[a][2] = 0.5 * (at(1 + a, x, y, zp) - at(1 + a, x, y, zm));
-		}
-		const double rho = at(0, x, y, z);
-		double g2 = 0;
-#pragma unroll
-		for (int a = 0; a < 3; a++)
-#pragma unroll
-			for (int b = 0; b < 3; b++)
-				g2 += G[a][b] * G[a][b];
-		const double wx = G[2][1] - G[1][2], wy = G[0][2] - G[2][0], wz = G[1][0] - G[0][1];
-		v[0] += rho * g2;
-		v[1] += rho * (wx * wx + wy * wy + wz * wz);
-	}
-	block_sum(v, sh);
-	if (threadIdx.x == 0)
-#pragma unroll
-		for (int i = 0; i < RED_N; i++)
-			partial[blockIdx.x * RED_N + i] = sh[0][i];
+	uint64_t tiles, items;
+	int64_t len;
+};
+inline GradShape grad_shape(const MacroArgs& A)
+{
+	GradShape g;
+	g.tiles = ((uint64_t) A.Y * (uint64_t) A.Z + RED_THREADS - 1) / RED_THREADS;
+	const int64_t most = g.tiles >= (uint64_t) GRAD_BLOCKS ? 1 : (int64_t) ((uint64_t) GRAD_BLOCKS / g.tiles);
+	const int64_t nseg = most < A.X ? most : A.X;
+	g.len = (A.X + nseg - 1) / nseg;
+	g.items = g.tiles * (uint64_t) ((A.X + g.len - 1) / g.len);
+	return g;
 }
 
-static __global__ void __launch_bounds__(256) k_reduce_final(const double* partial, int nparts, double* out)
+// Off: type of a byte offset within an x plane (32 bits where it holds at most
+// 4 GiB: scalar bases and one register per neighbour)
+template <typename T, typename Off>
+static __global__ void __launch_bounds__(RED_THREADS) k_reduce_gradients(const MacroArgs A, const GradShape S, double* partial)
 {
-	__shared__ double sh[256][RED_N];
-	double v[RED_N] = {0, 0, 0, 0, 0, 0};
-	for (int b = threadIdx.x; b < nparts; b += blockDim.x)
+	double v[2] = {0, 0};
+	const uint64_t plane = (uint64_t) A.Zs * (uint64_t) A.Ys;
+	// consecutive items on one XCD (GRAD_BLOCKS is a multiple of their number)
+	for (uint64_t L = (blockIdx.x % NXCD) * (gridDim.x / NXCD) + blockIdx.x / NXCD; L < S.items; L += gridDim.x) {
+		const uint64_t seg = L / S.tiles, i = (L % S.tiles) * RED_THREADS + threadIdx.x;
+		if (i >= (uint64_t) A.Y * (uint64_t) A.Z)
+			continue;
+		const int64_t z = (int64_t) (i / (uint64_t) A.Y), y = (int64_t) (i % (uint64_t) A.Y);
+		const int64_t yp = (! A.dist_y && y == A.Y - 1) ? 0 : y + 1, ym = (! A.dist_y && y == 0) ? A.Y - 1 : y - 1;
+		const int64_t zp = (! A.dist_z && z == A.Z - 1) ? 0 : z + 1, zm = (! A.dist_z && z == 0) ? A.Z - 1 : z - 1;
+		auto off = [&](int64_t zz, int64_t yy) { return (Off) (((zz + A.oz) * A.Ys + (yy + A.oy)) * (int64_t) sizeof(T)); };
+		const Off o = off(z, y), oyp = off(z, yp), oym = off(z, ym), ozp = off(zp, y), ozm = off(zm, y);
+		// field k of the x plane `base` sites into the array
+		auto get = [&](int k, uint64_t base, Off at) {
+			return *(const T*) ((const char*) ((const T*) A.macro + (k * A.XYZ + (int64_t) base)) + at);
+		};
+		const int64_t x0 = (int64_t) seg * S.len, x1 = x0 + S.len < A.X ? x0 + S.len : A.X;
+		const int64_t before = (! A.dist_x && x0 == 0) ? A.X - 1 : x0 - 1;
+		T vm[3], vc[3];
 #pragma unroll
-		for (int i = 0; i < RED_N; i++)
-			v[i] += partial[b * RED_N + i];
-	block_sum(v, sh);
+		for (int a = 0; a < 3; a++) {
+			vm[a] = get(1 + a, (uint64_t) (before + A.ox) * plane, o);
+			vc[a] = get(1 + a, (uint64_t) (x0 + A.ox) * plane, o);
+		}
+		for (int64_t x = x0; x < x1; x++) {
+			const int64_t xp = (! A.dist_x && x == A.X - 1) ? 0 : x + 1;
+			const uint64_t here = (uint64_t) (x + A.ox) * plane, next = (uint64_t) (xp + A.ox) * plane;
+			T n[3][5];
+#pragma unroll
+			for (int a = 0; a < 3; a++) {
+				n[a][0] = get(1 + a, next, o);
+				n[a][1] = get(1 + a, here, oyp);
+				n[a][2] = get(1 + a, here, oym);
+				n[a][3] = get(1 + a, here, ozp);
+				n[a][4] = get(1 + a, here, ozm);
+			}
+			const double rho = get(0, here, o);
+			// all 16 loads in flight before the first is used
+			__builtin_amdgcn_sched_barrier(0);
+			double G[3][3];  // G[a][b] = d v_a / d x_b
+#pragma unroll
+			for (int a = 0; a < 3; a++) {
+				G[a][0] = 0.5 * ((double) n[a][0] - (double) vm[a]);
+				G[a][1] = 0.5 * ((double) n[a][1] - (double) n[a][2]);
+				G[a][2] = 0.5 * ((double) n[a][3] - (double) n[a][4]);
+				vm[a] = vc[a];
+				vc[a] = n[a][0];
+			}
+			double g2 = 0;
+#pragma unroll
+			for (int a = 0; a < 3; a++)
+#pragma unroll
+				for (int b = 0; b < 3; b++)
+					g2 += G[a][b] * G[a][b];
+			const double wx = G[2][1] - G[1][2], wy = G[0][2] - G[2][0], wz = G[1][0] - G[0][1];
+			v[0] += rho * g2;
+			v[1] += rho * (wx * wx + wy * wy + wz * wz);
+		}
+	}
+	block_sum<2>(v);
+	if (threadIdx.x == 0) {
+		partial[blockIdx.x * 2] = v[0];
+		partial[blockIdx.x * 2 + 1] = v[1];
+	}
+}
+
+// the sums of ROWS blocks to `out` (device memory, or host memory mapped into
+// the device)
+template <int N, int ROWS>
+static __global__ void __launch_bounds__(1024) k_reduce_final(const double* partial, double* out)
+{
+	double v[N] = {};
+	for (int r = threadIdx.x; r < ROWS; r += 1024)
+#pragma unroll
+		for (int i = 0; i < N; i++)
+			v[i] += partial[r * N + i];
+	block_sum<N>(v);
 	if (threadIdx.x == 0)
 #pragma unroll
-		for (int i = 0; i < RED_N; i++)
-			out[i] = sh[0][i];
+		for (int i = 0; i < N; i++)
+			out[i] = v[i];
 }
 
 // ===========================================================================
