@@ -230,11 +230,25 @@ class CheckpointedRun:
     def _other(self, src):
         return self.pp[1] if src is self.pp[0] else self.pp[0]
 
+    def _record_segment(self, j, m):
+        """Segment j (m steps) again from its checkpoint, recording into `tape`."""
+        src, pp, fp32 = self.ckpt[j], self.pp, self.mode == "mixed"
+        if fp32:
+            self._refresh_fp32()
+            pp = self.pp32
+            src = pp[0]
+            src.copy_(self.ckpt[j])  # FP64 checkpoint -> FP32 state
+        for i in range(m):
+            dst = pp[1] if src is pp[0] else pp[0]
+            self._step(src, dst, self.tape[i], fp32=fp32)
+            src = dst
+
     # ---- the run ----------------------------------------------------------------
-    def forward(self, inflow: torch.Tensor, f0: torch.Tensor) -> torch.Tensor:
+    def forward(self, inflow: torch.Tensor, f0: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         """Runs T steps from f0 (flat storage layout) with the given inflow
         profile; returns the buffer holding the final state (valid until the
-        next call)."""
+        next call), or `out`, zeroed by the caller, which the last step then
+        writes (not in ``"tape"`` mode)."""
         try:
             self.generation += 1
             self.profile.copy_(inflow.reshape(3, self.lat.Z, self.lat.Y))
@@ -250,7 +264,10 @@ class CheckpointedRun:
             src = self.ckpt[0]
             for t in range(self.T):
                 nxt = t + 1
-                dst = self.ckpt[nxt // self.K] if nxt % self.K == 0 and nxt < self.T else self._other(src)
+                if nxt == self.T:
+                    dst = out if out is not None else self._other(src)
+                else:
+                    dst = self.ckpt[nxt // self.K] if nxt % self.K == 0 else self._other(src)
                 j = t // self.K
                 tape = self.rec[self.rec_offset[j] + t - j * self.K] if j >= self.rec_first else None
                 self._step(src, dst, tape)
@@ -259,65 +276,63 @@ class CheckpointedRun:
         finally:
             self.lat._bind()
 
-    def backward(self, lam_T: torch.Tensor, grad: torch.Tensor) -> torch.Tensor:
+    def backward(self, lam_T: torch.Tensor, grad: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         """lam_T = dL/d(final state); adds dL/d(inflow) to grad (3, Z, Y) float64
-        and returns dL/d(initial state) (a buffer valid until the next call).
-        Needs the recording of the last ``forward`` in ``"tape"`` mode."""
+        and returns dL/d(initial state) (a buffer valid until the next call),
+        or `out`, of the adjoint fields' type, which the last adjoint step
+        then writes.  Needs the recording of the last ``forward`` in
+        ``"tape"`` mode."""
         try:
             cur, other = self.lam
             cur.copy_(lam_T.reshape(-1))
             if self.mode == "tape":
                 for t in reversed(range(self.T)):
+                    if t == 0 and out is not None:
+                        other = out
                     self._adjoint(None, cur, other, grad, self.tape[t])
                     cur, other = other, cur
                 return cur
             for j in reversed(range(self.nseg)):
-                t0 = j * self.K
-                m = min(self.T, t0 + self.K) - t0
+                m = self._seg_len(j)
+                fp32 = self.mode == "mixed"
                 if j >= self.rec_first:
-                    for i in reversed(range(m)):
-                        self._adjoint(None, cur, other, grad, self.rec[self.rec_offset[j] + i])
-                        cur, other = other, cur
-                elif self.mode == "mixed":
-                    self._refresh_fp32()
-                    src = self.pp32[0]
-                    src.copy_(self.ckpt[j])  # FP64 checkpoint -> FP32 state
-                    for i in range(m):
-                        dst = self.pp32[1] if src is self.pp32[0] else self.pp32[0]
-                        self._step(src, dst, self.tape[i], fp32=True)
-                        src = dst
-                    for i in reversed(range(m)):
-                        self._adjoint(None, cur, other, grad, self.tape[i], fp32=True)
-                        cur, other = other, cur
+                    read = [(None, self.rec[self.rec_offset[j] + i]) for i in range(m)]
                 elif self.mode == "recompute":
                     states = [self.ckpt[j]] + self.seg[:m - 1]
                     for i in range(m - 1):
                         self._step(states[i], states[i + 1])
-                    for i in reversed(range(m)):
-                        self._adjoint(states[i], cur, other, grad)
-                        cur, other = other, cur
+                    read = [(f, None) for f in states]
                 else:
-                    src = self.ckpt[j]
-                    for i in range(m):
-                        dst = self._other(src)
-                        self._step(src, dst, self.tape[i])
-                        src = dst
-                    for i in reversed(range(m)):
-                        self._adjoint(None, cur, other, grad, self.tape[i])
-                        cur, other = other, cur
+                    self._record_segment(j, m)
+                    read = [(None, self.tape[i]) for i in range(m)]
+                for i in reversed(range(m)):
+                    if i == 0 and j == 0 and out is not None:
+                        other = out
+                    state, tape = read[i]
+                    self._adjoint(state, cur, other, grad, tape, fp32=fp32)
+                    cur, other = other, cur
             return cur
         finally:
             self.lat._bind()
 
 
+def _fresh(like: torch.Tensor, lat: D3Q27Lattice) -> torch.Tensor:
+    """A new tensor for a kernel that writes every stored site: zeros where
+    padding lies between the planes."""
+    return (torch.empty_like if lat.d.XYZ == lat.X * lat.Y * lat.Z else torch.zeros_like)(like)
+
+
 class _LatticeRun(torch.autograd.Function):
     @staticmethod
     def forward(ctx, inflow, f0, run: CheckpointedRun):
-        fT = run.forward(inflow.detach(), f0.detach())
+        # zeros, as the run's own buffers: a step leaves the slots of NOTHING sites
+        # and of the padding alone
+        own = torch.zeros_like(run.pp[0]) if run.mode != "tape" else None
+        fT = run.forward(inflow.detach(), f0.detach(), own)
         ctx.run = run
         ctx.generation = run.generation
         ctx.shapes = (inflow.shape, f0.shape, f0.dtype)
-        return fT.clone()
+        return fT.clone() if own is None else fT
 
     @staticmethod
     def backward(ctx, gF):
@@ -326,8 +341,10 @@ class _LatticeRun(torch.autograd.Function):
             raise RuntimeError("the CheckpointedRun was run forward again before this backward pass: its checkpoints "
                                "belong to the later run (use one CheckpointedRun per graph)")
         grad = torch.zeros(3, run.lat.Z, run.lat.Y, dtype=torch.float64, device=gF.device)
-        lam0 = run.backward(gF.to(run.lam[0].dtype).contiguous(), grad)
         inflow_shape, f0_shape, f0_dtype = ctx.shapes
+        # a tensor of the caller's own, where no conversion makes one
+        own = ctx.needs_input_grad[1] and f0_dtype == run.lam[0].dtype
+        lam0 = run.backward(gF, grad, _fresh(run.lam[0], run.lat) if own else None)
         return grad.reshape(inflow_shape), lam0.to(f0_dtype).reshape(f0_shape), None
 
 
@@ -352,7 +369,8 @@ class CoupledScalarRun:
     recomputed by plain D3Q27 steps that write their velocity (macro output
     into one buffer per step, the same velocity the coupled kernel hands to
     the D3Q7 update), and the D3Q7 adjoint steps (tnl_lbm_d3q7_adjoint_step)
-    run over it in reverse.  Memory: T/K flow states + K velocity fields,
+    run over it in reverse.  The coupled steps of the last segment write their
+    velocity there themselves, so that segment is not run again.  Memory: T/K flow states + K velocity fields,
     packed in 3K + 1 planes: step i of a segment writes its macro output (rho,
     vx, vy, vz) three planes below step i - 1's, so that only step i - 1's
     unused density plane is overwritten.  ``host_checkpoints`` keeps the flow
@@ -387,20 +405,25 @@ class CoupledScalarRun:
         self.lam = [torch.zeros(7 * n, dtype=cdt, device=dev) for _ in range(2)]
         self.out = torch.zeros(7 * n, dtype=torch.float64, device=dev)
         self.source = torch.zeros(n, dtype=mdt, device=dev)
+        self.held = None  # the segment whose velocities `vel` holds
         ade.source = self.source
         ade._bind()
 
     def _launch(self, rc):
         self.nse._check(rc)
 
-    def _coupled(self, fs, fd, gs, gd, stream=None):
+    def _coupled(self, fs, fd, gs, gd, ubuf=None, stream=None):
+        """One coupled step; `ubuf`: the planes its macro output goes to."""
         nse, ade = self.nse, self.ade
+        if ubuf is not None:
+            nse.d.macro = ubuf.data_ptr()
+            ade.d.macro = self.lam[0].data_ptr()  # phi, not needed: the adjoint fields are free in a forward pass
         nse.d.even_iter = ade.d.even_iter = 1
         nse.d.df[0], nse.d.df[1] = fs.data_ptr(), fd.data_ptr()
         ade.d.df[0], ade.d.df[1] = gs.data_ptr(), gd.data_ptr()
         self._launch(nse.lib.tnl_lbm_nse_ade_step(C.byref(nse.cfg), C.byref(nse.d), C.byref(ade.d),
-                                                  _abi.I64x3(0, 0, 0), _abi.I64x3(nse.X, nse.Y, nse.Z), 0,
-                                                  _stream_ptr(stream)))
+                                                  _abi.I64x3(0, 0, 0), _abi.I64x3(nse.X, nse.Y, nse.Z),
+                                                  0 if ubuf is None else _abi.FLAG_OUTPUT_MACRO, _stream_ptr(stream)))
 
     def _flow_step(self, fs, fd, ubuf, stream=None):
         nse = self.nse
@@ -423,24 +446,27 @@ class CoupledScalarRun:
                                                        _ptr(ubuf[nse.d.XYZ:]), _ptr(lam_next), _ptr(lam),
                                                        _ptr(grad), _stream_ptr(stream)))
 
-    def export(self, g: torch.Tensor) -> torch.Tensor:
+    def export(self, g: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         """A D3Q7 state (storage form) -> absolute populations, flat float64
-        (a buffer valid until the next call)."""
+        (a buffer valid until the next call, or `out`)."""
         ade = self.ade
+        out = self.out if out is None else out
         saved = ade.d.df[0]
         ade.d.df[0] = g.data_ptr()
         try:
-            ade._check(ade.lib.tnl_lbm_d3q7_export_f64(C.byref(ade.cfg), C.byref(ade.d), 0, _ptr(self.out),
+            ade._check(ade.lib.tnl_lbm_d3q7_export_f64(C.byref(ade.cfg), C.byref(ade.d), 0, _ptr(out),
                                                        _stream_ptr()))
         finally:
             ade.d.df[0] = saved
-        return self.out
+        return out
 
-    def forward(self, source: torch.Tensor, g0: torch.Tensor, f0: torch.Tensor) -> torch.Tensor:
+    def forward(self, source: torch.Tensor, g0: torch.Tensor, f0: torch.Tensor, keep: bool = True) -> torch.Tensor:
         """T coupled steps from (f0, g0) (flat storage layout) with the given
         source (flat XYZ in the lattice layout); returns the buffer holding
-        the final D3Q7 state."""
+        the final D3Q7 state.  keep=False: no backward pass will follow, keep
+        no velocities for it."""
         try:
+            self.held = None
             self.ade.refresh_rows()
             self.source.copy_(source.reshape(-1))
             self.ckpt[0].copy_(f0.reshape(-1))
@@ -455,10 +481,13 @@ class CoupledScalarRun:
                 other = self.pp[1] if fs is self.pp[0] else self.pp[0]
                 fd = self.ckpt[nxt // self.K] if at_ckpt and not self.host else other
                 gd = self.app[1] if gs is self.app[0] else self.app[0]
-                self._coupled(fs, fd, gs, gd)
+                j, i = divmod(t, self.K)
+                self._coupled(fs, fd, gs, gd, self._macro_slot(i) if keep and j == self.nseg - 1 else None)
                 if at_ckpt and self.host:
                     self.ckpt[nxt // self.K].copy_(fd)
                 fs, gs = fd, gd
+            if keep:
+                self.held = self.nseg - 1
             return gs
         finally:
             self.nse._bind()
@@ -475,15 +504,18 @@ class CoupledScalarRun:
             for j in reversed(range(self.nseg)):
                 t0 = j * self.K
                 m = min(self.T, t0 + self.K) - t0
-                if self.host:
-                    self.pp[0].copy_(self.ckpt[j])
-                    fs = self.pp[0]
-                else:
-                    fs = self.ckpt[j]
-                for i in range(m):
-                    fd = self.pp[1] if fs is self.pp[0] else self.pp[0]
-                    self._flow_step(fs, fd, self._macro_slot(i))
-                    fs = fd
+                if self.held != j:
+                    self.held = None
+                    if self.host:
+                        self.pp[0].copy_(self.ckpt[j])
+                        fs = self.pp[0]
+                    else:
+                        fs = self.ckpt[j]
+                    for i in range(m):
+                        fd = self.pp[1] if fs is self.pp[0] else self.pp[0]
+                        self._flow_step(fs, fd, self._macro_slot(i))
+                        fs = fd
+                    self.held = j
                 for i in reversed(range(m)):
                     self._adjoint(self._macro_slot(i), cur, other, grad)
                     cur, other = other, cur
@@ -496,16 +528,16 @@ class CoupledScalarRun:
 class _ScalarRun(torch.autograd.Function):
     @staticmethod
     def forward(ctx, source, run: CoupledScalarRun, g0, f0):
-        gT = run.forward(source.detach(), g0, f0)
+        gT = run.forward(source.detach(), g0, f0, ctx.needs_input_grad[0])
         ctx.run = run
         ctx.shape = source.shape
-        return run.export(gT).clone()
+        return run.export(gT, _fresh(run.out, run.nse))
 
     @staticmethod
     def backward(ctx, gG):
         run = ctx.run
         grad = torch.zeros(run.nse.d.XYZ, dtype=torch.float64, device=gG.device)
-        run.backward(gG.to(run.lam[0].dtype).contiguous(), grad)
+        run.backward(gG, grad)
         return grad.reshape(ctx.shape), None, None, None
 
 
@@ -520,5 +552,6 @@ def scalar_run(run: CoupledScalarRun, source: torch.Tensor, g0: torch.Tensor, f0
 def top_layer_variance(g: torch.Tensor, lat: D3Q27Lattice, layers: int) -> torch.Tensor:
     """Variance of phi = sum_q g_q over the top `layers` z-layers, in float64
     (g: flat 7*XYZ absolute populations)."""
-    phi = g.view(7, lat.d.XYZ)[:, :lat.nsites].sum(0).view(lat.X, lat.Z, lat.Y)[:, lat.Z - layers:, :]
+    # (the layers before the sum over q: one pass over them, not over the box)
+    phi = g.view(7, lat.d.XYZ)[:, :lat.nsites].view(7, lat.X, lat.Z, lat.Y)[:, :, lat.Z - layers:, :].sum(0)
     return ((phi - phi.mean()) ** 2).mean()
