@@ -459,6 +459,12 @@ int tnl_lbm_d3q27_step_record(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_dat
 int tnl_lbm_d3q7_adjoint_step(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* nse, const tnl_lbm_d3q7_data* ade,
                               const void* velocity, const void* lambda_next, void* lambda, double* grad_source,
                               void* stream);
+/* tnl_lbm_d3q27_step_record for F32 storage whose pulled populations come from
+ * an FP64 state (27*XYZ doubles in the layout of the populations, SD->df[0] is
+ * not read), each rounded to float as it is read: the step from the state's
+ * conversion to F32, without the conversion.  tape: float elements.          */
+int tnl_lbm_d3q27_step_record_from_f64(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* SD, const double* state,
+                                       void* tape, void* stream);
 int tnl_lbm_d3q27_adjoint_step_recorded(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* SD, const void* tape,
                                         int tape_f64, const void* lambda_next, void* lambda, double* grad_inflow,
                                         void* stream);

@@ -35,7 +35,7 @@ int record_for(const StepArgs& A0, unsigned threads, unsigned grid, hipStream_t 
 	// -124 (FP64) / -151 (FP32) VALU, ~4% on the C4 duct (kernel trace)
 	constexpr size_t E = sizeof(typename Storage<ST>::elem);
 	const bool nt = hint_streams(A, 54, E);
-	if (! narrow_slots(A.XYZ, E))
+	if (! narrow_slots(A.XYZ, sizeof(typename Pulled<ST>::elem)))
 		hipLaunchKernelGGL((k_general<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, TAPE>), dim3(grid), dim3(threads), 0, st, A);
 	else if (nt)
 		hipLaunchKernelGGL((k_general<ST, TNL_LBM_COLL_CUM, TNL_LBM_PATTERN_AB, TAPE, true, false, true>), dim3(grid), dim3(threads), 0, st, A);
@@ -94,6 +94,11 @@ int launch_record(const tnl_lbm_config* cfg, const StepArgs& A, int tape_kind, u
 		return tape_kind == 2 ? record_for<TNL_LBM_STORE_F64, 2>(A, threads, grid, st)
 							  : record_for<TNL_LBM_STORE_F64, 1>(A, threads, grid, st);
 	return record_for<TNL_LBM_STORE_F32, 1>(A, threads, grid, st);
+}
+
+int launch_record_from_f64(const StepArgs& A, unsigned threads, unsigned grid, hipStream_t st)
+{
+	return record_for<STORE_F32_FROM_F64, 1>(A, threads, grid, st);
 }
 
 }  // namespace lbm

@@ -1025,6 +1025,30 @@ int tnl_lbm_d3q27_step_record(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_dat
 	return launch_record(cfg, A, kind, threads, grid, (hipStream_t) stream);
 }
 
+int tnl_lbm_d3q27_step_record_from_f64(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* SD, const double* state,
+									   void* tape, void* stream)
+{
+	if (int rc = adjoint_config(cfg, SD))
+		return rc;
+	if (cfg->storage != TNL_LBM_STORE_F32)
+		return fail(TNL_LBM_ERR_UNSUPPORTED, "the recording step from an FP64 state writes F32 populations");
+	if (! state || ! tape)
+		return fail(TNL_LBM_ERR_NULL, "state or moment tape missing");
+	if (state == SD->df[1] || tape == state || tape == SD->df[1])
+		return fail(TNL_LBM_ERR_ARG, "the state, the tape and the populations must not alias");
+	tnl_lbm_d3q27_data D = *SD;
+	D.df[0] = (void*) state;
+	StepArgs A;
+	unsigned threads = 0, grid = 0;
+	const int64_t off[3] = {0, 0, 0}, end[3] = {SD->X, SD->Y, SD->Z};
+	if (int rc = make_step_args(cfg, &D, off, end, 0, A, threads, grid))
+		return rc;
+	if (grid == 0)
+		return TNL_LBM_OK;
+	A.tape = tape;
+	return launch_record_from_f64(A, threads, grid, (hipStream_t) stream);
+}
+
 int tnl_lbm_d3q27_adjoint_step_recorded(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* SD, const void* tape,
 										int tape_f64, const void* lambda_next, void* lambda, double* grad_inflow,
 										void* stream)

@@ -158,6 +158,30 @@ struct Storage<STORE_F32_F64MATH>
 	static LBM_DEV real ld(const elem* p, float = 1) { return (double) *p; }
 	static LBM_DEV void st(elem* p, real v, float = 1) { *p = (float) v; }
 };
+// The F32 form whose step pulls from FP64 populations, each rounded to float as
+// it is loaded: a form of the recording step only.
+constexpr int STORE_F32_FROM_F64 = 101;
+template <>
+struct Storage<STORE_F32_FROM_F64>
+{
+	using elem = float;
+	using real = float;
+	static constexpr bool dev = false;
+	static constexpr bool fixed = false;
+	static LBM_DEV real ld(const double* p, float = 1) { return (float) *p; }
+	static LBM_DEV void st(elem* p, real v, float = 1) { *p = v; }
+};
+// the element type that a step pulls
+template <int ST>
+struct Pulled
+{
+	using elem = typename Storage<ST>::elem;
+};
+template <>
+struct Pulled<STORE_F32_FROM_F64>
+{
+	using elem = double;
+};
 template <>
 struct Storage<TNL_LBM_STORE_F32_DEV>
 {

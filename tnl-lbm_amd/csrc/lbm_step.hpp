@@ -911,16 +911,17 @@ struct General
 	using S = Storage<ST>;
 	using real = typename S::real;
 	using elem = typename S::elem;
+	using pulled = typename Pulled<ST>::elem;
 	using P = Phys<ST>;
 	static constexpr bool AA = PATTERN == TNL_LBM_PATTERN_AA;
 	static constexpr int EQK = eq_kind_of(COLL);
 	static constexpr bool FAST = fast_collision<ST, COLL>;
 
-	static constexpr bool NT = NTG && ((LBM_NT_GENERAL >> ST) & 1);
-	static LBM_DEV real ldq(const elem* p, float sc, bool nt)
+	static constexpr bool NT = NTG && (ST == STORE_F32_FROM_F64 || ((LBM_NT_GENERAL >> ST % 32) & 1));
+	static LBM_DEV real ldq(const pulled* p, float sc, bool nt)
 	{
 		if (nt) {
-			const elem v = ld_nt(p);
+			const pulled v = ld_nt(p);
 			return S::ld(&v, sc);
 		}
 		return S::ld(p, sc);
@@ -1016,7 +1017,7 @@ struct General
 			add_site_force(A, s0, Fx, Fy, Fz);
 		real f[27];
 		real rho = 1, vx = 0, vy = 0, vz = 0;
-		const elem* __restrict__ cur = (const elem*) A.df0;
+		const pulled* __restrict__ cur = (const pulled*) A.df0;
 
 		if (gi != GEO_NOTHING) {
 			// pull location (bc.h:72-74); OUTFLOW_RIGHT pulls as if located at x-1

@@ -189,6 +189,7 @@ def _declare(lib, prefix: str):
         "d3q7_export_f64": [cfgp, d7p, C.c_int, _P],
         "d3q27_adjoint_step": [cfgp, d27p, _P, _P, _P],
         "d3q27_step_record": [cfgp, d27p, _P, C.c_int],
+        "d3q27_step_record_from_f64": [cfgp, d27p, _P, _P],
         "d3q27_adjoint_step_recorded": [cfgp, d27p, _P, C.c_int, _P, _P, _P],
         "d3q7_adjoint_step": [cfgp, d27p, d7p, _P, _P, _P, _P],
         "d3q27_halo_x": [cfgp, d27p, d27p, C.c_int],

@@ -210,6 +210,13 @@ class CheckpointedRun:
             lat._check(lat.lib.tnl_lbm_d3q27_step_record(C.byref(cfg), C.byref(d), _ptr(tape), int(self.tape_f64),
                                                          _stream_ptr(stream)))
 
+    def _record_from_f64(self, state: torch.Tensor, dst: torch.Tensor, tape: torch.Tensor, stream=None):
+        lat, d = self.lat, self.d32
+        d.even_iter = 1
+        d.df[0] = d.df[1] = dst.data_ptr()
+        lat._check(lat.lib.tnl_lbm_d3q27_step_record_from_f64(C.byref(self.cfg32), C.byref(d), _ptr(state), _ptr(tape),
+                                                              _stream_ptr(stream)))
+
     def _adjoint(self, state: torch.Tensor | None, lam_next: torch.Tensor, lam: torch.Tensor, grad: torch.Tensor,
                  tape: torch.Tensor | None = None, stream=None, fp32: bool = False):
         lat = self.lat
@@ -233,12 +240,17 @@ class CheckpointedRun:
     def _record_segment(self, j, m):
         """Segment j (m steps) again from its checkpoint, recording into `tape`."""
         src, pp, fp32 = self.ckpt[j], self.pp, self.mode == "mixed"
+        first = 0
         if fp32:
             self._refresh_fp32()
             pp = self.pp32
-            src = pp[0]
-            src.copy_(self.ckpt[j])  # FP64 checkpoint -> FP32 state
-        for i in range(m):
+            if src.is_cuda:
+                # the first step rounds the FP64 checkpoint to FP32 as it pulls
+                self._record_from_f64(src, pp[1], self.tape[0])
+                src, first = pp[1], 1
+            else:
+                src = pp[0].copy_(src)
+        for i in range(first, m):
             dst = pp[1] if src is pp[0] else pp[0]
             self._step(src, dst, self.tape[i], fp32=fp32)
             src = dst
