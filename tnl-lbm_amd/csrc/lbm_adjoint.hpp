@@ -332,6 +332,37 @@ LBM_DEV uint32_t irregular_pulls(bool per, bool right, int32_t x, int32_t y, int
 	return m;
 }
 
+// rank of q among the directions with its c_y
+constexpr int y_rank(int q)
+{
+	int k = 0;
+	for (int r = 0; r < q; r++)
+		k += CY[r] == CY[q];
+	return k;
+}
+
+// Wall sites of the y faces.  A y face is strided in memory, so the second pass
+// touches a cache line for every one of a wall's nine irregular pulls, reading and
+// adding (with them 32 us in a 256x96x96 duct, float fields, without 16; the first
+// pass 145 and 134).  The slots meant are those
+// that the site one row in owns, and it is the next lane: the wall hands its nine
+// values to that lane through LDS, and the second pass leaves the wall out.  That
+// is done where the wall's pulls are irregular in y alone, the site one row in is
+// an ordinary one, and both are in one wave.
+LBM_DEV bool inner_xz(const StepArgs& A, int64_t x, int64_t z)
+{
+	return A.Y >= 3 && x > 0 && x < A.X - 1 && z > 0 && z < A.Z - 1;
+}
+LBM_DEV bool collides(int16_t gi)
+{
+	return gi == GEO_FLUID || gi == GEO_PERIODIC;
+}
+// whether the wall (x, y, z) hands them over; lane: its lane in the first pass
+LBM_DEV bool wall_gives(const StepArgs& A, int64_t x, int64_t y, int64_t z, uint32_t lane, int16_t before, int16_t after)
+{
+	return inner_xz(A, x, z) && ((y == 0 && lane < 63 && collides(after)) || (y == A.Y - 1 && lane > 0 && collides(before)));
+}
+
 // SPECIAL = false: every site, plain stores to the slots it owns under the
 // periodic wrap (0 for slots whose true reader is elsewhere).  SPECIAL = true:
 // the face sites only, atomic adds of those contributions to their true
@@ -345,7 +376,7 @@ LBM_DEV uint32_t irregular_pulls(bool per, bool right, int32_t x, int32_t y, int
 // Bound: HBM, then FP64 issue (about 500 FP64 instructions a site).  Four
 // waves per SIMD (at most 128 VGPRs; from an FP64 state, whose 27 pulled values
 // meet the 27 of lambda, three): 256x96x96 duct, float fields and recording,
-// 164 -> 145 us (4.2 TB/s) against the sweep that recomputed the chain's
+// 164 -> 145 us (134 with the walls handed over, 4.5 TB/s) against the sweep that recomputed the chain's
 // intermediate populations at 256 VGPRs and two waves.
 template <int ST, bool SPECIAL, int TAPE = 0, bool P32 = false>
 __global__ void __launch_bounds__(256, (TAPE == 0 && ST == TNL_LBM_STORE_F64) ? 3 : 4) k_adjoint_ab(const StepArgs A, const AdjPtrs P)
@@ -382,6 +413,12 @@ __global__ void __launch_bounds__(256, (TAPE == 0 && ST == TNL_LBM_STORE_F64) ? 
 		// bounce-back: mu_q = lam_next[opp(q)], read only for the irregular directions
 		// (the face sites are one per cache line here); inflow: mu = 0
 		if (gi == GEO_WALL) {
+			if ((y == 0 || y == A.Y - 1) && inner_xz(A, x, z)) {
+				const uint32_t lane = ((A.lin ? (uint32_t) z * (uint32_t) A.Y : 0u) + (uint32_t) y) & 63u;
+				const int16_t in = A.map[y == 0 ? s0 + 1 : s0 - 1];
+				if (wall_gives(A, x, y, z, lane, in, in))
+					return;
+			}
 			const Nb NX = neighbours<false>(x, A.X, 0, false, false);
 			const Nb NY = neighbours<false>(y, A.Y, 0, false, false);
 			const Nb NZ = neighbours<false>(z, A.Z, 0, false, false);
@@ -400,6 +437,25 @@ __global__ void __launch_bounds__(256, (TAPE == 0 && ST == TNL_LBM_STORE_F64) ? 
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		lam[q] = (lreal) S::ld(slot_at(Ln, q, x, y, z));
+	// what the walls of the y faces hand to the next lane (wall_gives)
+	__shared__ lreal given[SPECIAL ? 1 : 9][SPECIAL ? 1 : 256];
+	bool from_before = false, from_after = false;
+	if constexpr (! SPECIAL) {
+		const uint32_t lane = threadIdx.x & 63u;
+		const int16_t before = (int16_t) __shfl_up((int) gi, 1), after = (int16_t) __shfl_down((int) gi, 1);
+		const bool inner = inner_xz(A, x, z) && collides(gi);
+		from_before = inner && y == 1 && lane > 0 && before == GEO_WALL;
+		from_after = inner && y == A.Y - 2 && lane < 63 && after == GEO_WALL;
+		if (gi == GEO_WALL && wall_gives(A, x, y, z, lane, before, after)) {
+#pragma unroll
+			for (int q = 0; q < 27; q++)
+				if (CY[q] != 0 && (CY[q] > 0) == (y == 0))
+					given[y_rank(q)][threadIdx.x] = lam[opp(q)];
+		}
+		// (one wave: its LDS accesses are in order; the compiler must keep them so)
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+	}
 	// raw moments of the pulled populations: from the state, or recorded by the
 	// forward step (read at every site, used where the forward step wrote them)
 	Nb PX, NY, NZ;
@@ -444,8 +500,24 @@ __global__ void __launch_bounds__(256, (TAPE == 0 && ST == TNL_LBM_STORE_F64) ? 
 	if ((gi == GEO_FLUID || gi == GEO_PERIODIC || gi == GEO_OUTFLOW_RIGHT) && ! unsupported) {
 		real l[D::NMOM];
 		D::vjp_m(m, lam, (real) A.fx, (real) A.fy, (real) A.fz, (real) A.omega1, gi == GEO_OUTFLOW_RIGHT, l);
-		if (! SPECIAL && irregular == 0)
-			D::for_each_mu(l, [&](int q, real v) { S::st(slot_at(L, q, WX[-CX[q]], WY[-CY[q]], WZ[-CZ[q]]), v); });
+		if (! SPECIAL && irregular == 0) {
+			real wb[9], wa[9];
+#pragma unroll
+			for (int k = 0; k < 9; k++)
+				wb[k] = wa[k] = 0;
+			if (from_before)
+#pragma unroll
+				for (int k = 0; k < 9; k++)
+					wb[k] = (real) given[k][threadIdx.x - 1];
+			if (from_after)
+#pragma unroll
+				for (int k = 0; k < 9; k++)
+					wa[k] = (real) given[k][threadIdx.x + 1];
+			D::for_each_mu(l, [&](int q, real v) {
+				const real w = CY[q] > 0 ? v + wb[y_rank(q)] : CY[q] < 0 ? v + wa[y_rank(q)] : v;
+				S::st(slot_at(L, q, WX[-CX[q]], WY[-CY[q]], WZ[-CZ[q]]), w);
+			});
+		}
 		else
 			D::for_each_mu(l, put);
 	}
