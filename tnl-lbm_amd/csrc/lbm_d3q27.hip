@@ -8,9 +8,10 @@
 //  * a block spans one (x, z) row segment, so the row offsets of the site
 //    and of its x/z neighbours are wave-uniform and live in scalar
 //    registers; only the y index (and its +-1 neighbours) is per lane;
-//  * the 1-D grid is remapped so that consecutive row segments land on the
-//    same XCD (workgroups are dispatched round-robin over the 8 XCDs), which
-//    keeps the cache lines shared by y-neighbouring waves in one L2;
+//  * the 1-D grid is remapped (workgroups are dispatched round-robin over the 8
+//    XCDs) so that groups of consecutive row segments land on one XCD, which
+//    keeps the cache lines shared by y-neighbouring waves in one L2, while the
+//    XCDs work side by side on one range of each population plane;
 //  * the pure-periodic A-A path reads no geometry map at all; the general
 //    path reads the int16 map and applies D3Q27_BC_All (d3q27/bc.h:61-422).
 #include <hip/hip_runtime.h>
@@ -531,8 +532,7 @@ static int make_step_args(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* S
 	if (nb >= (1ull << 31))
 		return fail(TNL_LBM_ERR_DIMS, "lattice box too large for one launch");
 	A.nblocks = (uint32_t) nb;
-	const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
-	A.per_xcd = padded / NXCD;
+	const uint32_t padded = padded_blocks(A);
 	A.even = SD->even_iter ? 1 : 0;
 	A.out_macro = (flags & TNL_LBM_FLAG_OUTPUT_MACRO) ? 1 : 0;
 	A.macro_f64 = cfg->macro_real == TNL_LBM_REAL_F64;

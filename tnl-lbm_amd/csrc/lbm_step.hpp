@@ -50,7 +50,7 @@ struct StepArgs
 	int32_t nx, ny, nz;
 	uint32_t nyb;      // y segments per row (linear mapping: blocks per x plane)
 	uint32_t nblocks;  // logical blocks
-	uint32_t per_xcd;  // padded blocks / 8
+	uint32_t group;    // log2 of the consecutive blocks of one XCD (logical_block)
 	int32_t lin;       // linear y-z mapping (see linearize)
 	// the even A-A step over one contiguous range of stored sites (flat_range)
 	int32_t flat;
@@ -97,6 +97,33 @@ LBM_DEV bool plain_scalar(int16_t ga)
 
 constexpr int NXCD = 8;
 
+// Workgroups go to the XCDs in turn.  Groups of 2^A.group consecutive logical
+// blocks belong to one XCD, so that its L2 serves the lines that neighbouring
+// waves share, and the groups go to the XCDs in turn, so that all of them work
+// on one range of each population plane.  With an eighth of the grid for each XCD
+// the step streamed through 8 ranges of 27 (A-B: 54) planes at once, on most
+// sizes at 5 to 20% less bandwidth.  Steps in one process on one buffer, an
+// eighth each / groups of 1 / 8 / 32 / 256 blocks: 48x320x320 FP64 slab 964 / 803 /
+// 794 / 789 / 817 us; 256x96x96 mixed gradient 15.1 / 12.5 / 12.3 / 12.3 / 12.5 ms;
+// 301x417x333 F32_DEV box 4359 / - / 3498 / 3477 / 3480 us; 512^3 FP64 box 18.95 /
+// 22.9 / 19.05 / 18.90 / 18.81 ms (singly, the XCDs fetch each other's lines).
+LBM_DEV uint32_t logical_block(const StepArgs& A)
+{
+	const uint32_t k = blockIdx.x / NXCD;
+	return (((k >> A.group) * NXCD + blockIdx.x % NXCD) << A.group) + (k & ((1u << A.group) - 1u));
+}
+// The grid for A.nblocks logical blocks.  Smaller groups where there would be
+// fewer than 16 for each XCD: the last ones keep one XCD busy alone (128x64x64,
+// groups of 1024: 208 us a pair of steps, of 32: 90).
+inline uint32_t padded_blocks(StepArgs& A, uint32_t group = 5)
+{
+	while (group > 0 && ((uint64_t) NXCD << group) * 16 > A.nblocks)
+		group--;
+	A.group = group;
+	const uint32_t whole = (uint32_t) NXCD << group;
+	return (A.nblocks + whole - 1) / whole * whole;
+}
+
 // one x plane of a population array of `elem`-byte elements takes 32-bit offsets
 inline bool narrow_planes(const StepArgs& A, size_t elem)
 {
@@ -142,8 +169,7 @@ LBM_DEV double inflow_component(const StepArgs& A, int k, int64_t i)
 template <bool LIN = true, bool LIST = false>
 LBM_DEV bool block_coords(const StepArgs& A, int64_t& x, int64_t& z, int64_t& y)
 {
-	const uint32_t b = blockIdx.x;
-	const uint32_t L = (b % NXCD) * A.per_xcd + b / NXCD;
+	const uint32_t L = logical_block(A);
 	if (L >= A.nblocks)
 		return false;
 	if constexpr (LIST) {
@@ -191,8 +217,7 @@ LBM_DEV bool block_coords(const StepArgs& A, int64_t& x, int64_t& z, int64_t& y)
 template <bool LIN>
 LBM_DEV bool box_coords(const StepArgs& A, int64_t& x, int64_t& z, int64_t& y)
 {
-	const uint32_t b = blockIdx.x;
-	const uint32_t L = (b % NXCD) * A.per_xcd + b / NXCD;
+	const uint32_t L = logical_block(A);
 	if (L >= A.nblocks)
 		return false;
 	if constexpr (LIN) {
@@ -452,8 +477,7 @@ LBM_DEV char* sptr(char* p)
 // whether a wave's accesses cover whole lines.  `per` sites per lane.
 LBM_DEV bool even_site(const StepArgs& A, uint32_t per, uint64_t& row, uint32_t& yl)
 {
-	const uint32_t b = blockIdx.x;
-	const uint32_t L = (b % NXCD) * A.per_xcd + b / NXCD;
+	const uint32_t L = logical_block(A);
 	if (L >= A.nblocks)
 		return false;
 	if (A.flat) {
@@ -2057,8 +2081,7 @@ inline void linearize(StepArgs& A, unsigned& threads, unsigned& grid)
 	const uint64_t plane = (uint64_t) A.ny * (uint64_t) A.nz;
 	A.nyb = (uint32_t) ((plane + threads - 1) / threads);
 	A.nblocks = A.nyb * (uint32_t) A.nx;  // no larger than the row mapping's count
-	const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
-	A.per_xcd = padded / NXCD;
+	const uint32_t padded = padded_blocks(A);
 	A.lin = 1;
 	grid = padded;
 }
@@ -2082,8 +2105,7 @@ inline void list_shape(StepArgs& A, const uint32_t* rows, uint32_t nrows, unsign
 		A.nyb = 1;
 		A.nblocks = (uint32_t) (((uint64_t) nrows * (uint64_t) A.ny + threads - 1) / threads);
 	}
-	const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
-	A.per_xcd = padded / NXCD;
+	const uint32_t padded = padded_blocks(A);
 	grid = padded;
 }
 
@@ -2130,8 +2152,8 @@ inline bool even_shape(StepArgs& A, uint32_t per, unsigned most, unsigned& threa
 		A.nblocks = A.nyb * (uint32_t) A.nz * (uint32_t) A.nx;  // no more blocks than one lane per site needs
 		whole = planes && (uint64_t) A.Ys * elem % 128 == 0 && (uint64_t) (A.oy + A.offy) * elem % 128 == 0;
 	}
-	const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
-	A.per_xcd = padded / NXCD;
+	// (2-byte forms, 512^3: groups of 32 blocks 1 to 2% slower than of 256)
+	const uint32_t padded = padded_blocks(A, elem == 2 ? 8 : 5);
 	grid = padded;
 	return whole;
 }
@@ -2186,8 +2208,7 @@ void odd_launch(const StepArgs& A0, unsigned threads, unsigned grid, hipStream_t
 			threads /= 2;
 		A.nyb = (uint32_t) ((plane + threads - 1) / threads);
 		A.nblocks = A.nyb * (uint32_t) A.nx;
-		const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
-		A.per_xcd = padded / NXCD;
+		const uint32_t padded = padded_blocks(A);
 		hipLaunchKernelGGL((k_aa_odd<ST, COLL, NTO, true>), dim3(padded), dim3(threads), 0, st, A);
 		return;
 	}
@@ -2195,8 +2216,7 @@ void odd_launch(const StepArgs& A0, unsigned threads, unsigned grid, hipStream_t
 		threads = LBM_TPB_FP32;
 		A.nyb = (uint32_t) A.ny / LBM_TPB_FP32;
 		A.nblocks = A.nyb * (uint32_t) A.nz * (uint32_t) A.nx;  // fewer blocks than at 256
-		grid = (A.nblocks + NXCD - 1) / NXCD * NXCD;
-		A.per_xcd = grid / NXCD;
+		grid = padded_blocks(A);
 	}
 	hipLaunchKernelGGL((k_aa_odd<ST, COLL, NTO, false>), dim3(grid), dim3(threads), 0, st, A);
 }
@@ -2248,8 +2268,7 @@ void lean_shape(const StepArgs& A0, uint64_t planes, size_t elem, Go&& go)
 		A.nyb = (uint32_t) A.ny / threads;
 		A.nblocks = A.nyb * (uint32_t) A.nz * (uint32_t) A.nx;
 	}
-	const uint32_t padded = (A.nblocks + NXCD - 1) / NXCD * NXCD;
-	A.per_xcd = padded / NXCD;
+	const uint32_t padded = padded_blocks(A);
 	go(A, threads, padded, lin);
 }
 
