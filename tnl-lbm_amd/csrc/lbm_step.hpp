@@ -1286,10 +1286,9 @@ struct AdeIn
 	typename Storage<ST>::real D, S;
 };
 
-// src(q): pointer to the stored population q pulled here, qs(q) its storage
-// direction, nt(q) whether to hint
-template <int ST, bool LEAN, typename Src>
-LBM_DEV void ade_load(const StepArgs& A, const AdeArgs& B, int64_t s0, int16_t gi, Src&& src, AdeIn<ST>& in)
+// src(k, ...): the k-th load, population from(k) pulled here
+template <int ST, bool LEAN, typename From, typename Src>
+LBM_DEV void ade_load(const StepArgs& A, const AdeArgs& B, int64_t s0, int16_t gi, From from, Src&& src, AdeIn<ST>& in)
 {
 	using K = Ade7<ST>;
 	using real = typename K::real;
@@ -1303,8 +1302,8 @@ LBM_DEV void ade_load(const StepArgs& A, const AdeArgs& B, int64_t s0, int16_t g
 	const real pr = (real) B.phi_ref, isc = (real) 1 / (real) B.scale;
 	if (LEAN || gi != A_NOTHING) {
 #pragma unroll
-		for (int q = 0; q < 7; q++)
-			in.f[q] = src(q, pr, isc);
+		for (int k = 0; k < 7; k++)
+			in.f[from(k)] = src(k, pr, isc);
 	}
 }
 
@@ -1417,7 +1416,7 @@ __global__ void __launch_bounds__(256) k_nse_ade(const StepArgs A, const AdeArgs
 		PX.p = PX.o = NX.m;
 	AdeIn<ST> in;
 	const elem* cur = (const elem*) B.df0;
-	ade_load<ST, false>(A, B, s0, ga,
+	ade_load<ST, false>(A, B, s0, ga, [](int q) { return q; },
 				 [&](int q, real pr, real isc) {
 					 if (AA && B.even)
 						 return ade_get<ST>(slot0<O32>(cur, q, A, s0), q, pr, isc, NT);
@@ -1492,15 +1491,32 @@ struct Stencil
 		asm volatile("" : "+v"(s));
 		return s;
 	}
-	// slot of direction q: pb is the byte stride between directions
+	// slot of the direction whose array `base` is
 	template <typename E>
-	LBM_DEV E* slot(E* base, uint64_t pb, const StepArgs& A, int q, int cx, int cy, int cz) const
+	LBM_DEV E* slot(E* base, const StepArgs& A, int cx, int cy, int cz) const
 	{
 		if constexpr (LIN)
-			return at((E*) sptr<true>((char*) base + ((uint64_t) q * pb + xoff[1 + cx] * sizeof(E))), zr[1 + cz] + ys[1 + cy]);
+			return at((E*) sptr<true>((char*) base + xoff[1 + cx] * sizeof(E)), zr[1 + cz] + ys[1 + cy]);
 		else
-			return at((E*) sptr<true>((char*) base + ((uint64_t) q * pb + (xoff[1 + cx] + (uint64_t) (zs[1 + cz] * (uint32_t) A.Ys)) * sizeof(E))),
-					  ys[1 + cy]);
+			return at((E*) sptr<true>((char*) base + (xoff[1 + cx] + (uint64_t) (zs[1 + cz] * (uint32_t) A.Ys)) * sizeof(E)), ys[1 + cy]);
+	}
+};
+
+// The arrays of the directions in turn: two scalar additions each, where the
+// multiples of the stride, formed afresh for every access so as not to stay live,
+// took six: 548 -> 378 scalar instructions a wave, coupled 256^3 F16 1009 -> 986 us for
+// two steps, equal where HBM alone bounds the step.
+template <typename E>
+struct Planes
+{
+	char* p;
+	uint64_t pb;
+	LBM_DEV Planes(const void* base, uint64_t stride) : p((char*) base), pb(stride) {}
+	LBM_DEV E* next()
+	{
+		E* r = (E*) p;
+		p = sptr<true>(p + pb);
+		return r;
 	}
 };
 
@@ -1571,46 +1587,41 @@ LBM_DEV void lean_site(const StepArgs& A, const AdeArgs& B)
 			N.zs[1] = (uint32_t) NZ.o;
 			N.zs[2] = (uint32_t) NZ.p;
 		}
-		// the slot of population q pulled here, and pushed
-		auto src = [&](const elem* base, int q) {
+		// Array k holds what population from(k) pulls here and population to(k)
+		// pushes; their slots in it.
+		constexpr auto from = [](int k) { return MODE == LEAN_ODD ? opp(k) : k; };
+		constexpr auto to = [](int k) { return MODE == LEAN_EVEN ? opp(k) : k; };
+		auto src = [&](const elem* base, int k) {
 			if constexpr (MODE == LEAN_EVEN)
-				return N.slot(base, pb, A, q, 0, 0, 0);
+				return N.slot(base, A, 0, 0, 0);
 			else
-				return N.slot(base, pb, A, MODE == LEAN_ODD ? opp(q) : q, -CX[q], -CY[q], -CZ[q]);
+				return N.slot(base, A, -CX[from(k)], -CY[from(k)], -CZ[from(k)]);
 		};
-		auto dst = [&](elem* base, uint64_t pbo, int q) {
+		auto dst = [&](elem* base, int k) {
 			if constexpr (MODE == LEAN_ODD)
-				return N.slot(base, pbo, A, q, CX[q], CY[q], CZ[q]);
+				return N.slot(base, A, CX[k], CY[k], CZ[k]);
 			else
-				return N.slot(base, pbo, A, MODE == LEAN_EVEN ? opp(q) : q, 0, 0, 0);
+				return N.slot(base, A, 0, 0, 0);
 		};
 		AdeIn<ST> in;
 		N.local();
 		if constexpr (ADE) {
-			const elem* acur = (const elem*) here((char*) B.df0);
-			ade_load<ST, true>(A, B, N.own(A), ga,
-							   [&](int q, real pr, real isc) {
-								   return ade_get<ST>(src(acur, q), MODE == LEAN_ODD ? opp(q) : q, pr, isc,
-													  NT && (MODE == LEAN_EVEN || CY[q] == 0));
+			Planes<const elem> acur(here((char*) B.df0), pb);
+			ade_load<ST, true>(A, B, N.own(A), ga, from,
+							   [&](int k, real pr, real isc) {
+								   return ade_get<ST>(src(acur.next(), k), k, pr, isc, NT && (MODE == LEAN_EVEN || CY[k] == 0));
 							   },
 							   in);
 			N.local();
 		}
 		real f[27];
-		const elem* cur = (const elem*) here((char*) A.df0);
+		Planes<const elem> cur(here((char*) A.df0), pb);
 #pragma unroll
-		for (int q = 0; q < 27; q++) {
-			const elem* p = src(cur, q);
-			const elem v = NT && (MODE == LEAN_EVEN || CY[q] == 0) ? ld_nt(p) : *p;
-			f[q] = S::ld(&v, A.cls_sc[ncls(q)]);
+		for (int k = 0; k < 27; k++) {
+			const elem* p = src(cur.next(), k);
+			const elem v = NT && (MODE == LEAN_EVEN || CY[k] == 0) ? ld_nt(p) : *p;
+			f[from(k)] = S::ld(&v, A.cls_sc[ncls(k)]);
 		}
-		auto put = [&](elem* out, uint64_t pbo, int q, elem e) {
-			elem* p = dst(out, pbo, q);
-			if (NT && (MODE != LEAN_ODD || CY[q] == 0))
-				st_nt(p, e);
-			else
-				*p = e;
-		};
 		real rho = 1, vx = 0, vy = 0, vz = 0;
 		real Fx = (real) here(A.fx), Fy = (real) here(A.fy), Fz = (real) here(A.fz);
 		if (A.force)
@@ -1619,22 +1630,30 @@ LBM_DEV void lean_site(const StepArgs& A, const AdeArgs& B)
 			bounce_back<ST, COLL>(f);
 		if (! wall)
 			collide_site<ST, COLL>(f, A, Fx, Fy, Fz, rho, vx, vy, vz);
-		elem* out = (elem*) after<true>((char*) (AA ? A.df0 : A.df1), f[26]);
-		const uint64_t pbo = here(A.plane_bytes);
+		Planes<elem> out(after<true>((char*) (AA ? A.df0 : A.df1), f[26]), here(A.plane_bytes));
 		N.local();
-		encode_all<ST, COLL>(f, A, [&](int q, elem e) { put(out, pbo, q, e); });
+		real o[27];
+#pragma unroll
+		for (int k = 0; k < 27; k++)
+			o[k] = f[to(k)];
+		encode_all<ST, COLL>(o, A, [&](int k, elem e) {
+			elem* p = dst(out.next(), k);
+			if (NT && (MODE != LEAN_ODD || CY[k] == 0))
+				st_nt(p, e);
+			else
+				*p = e;
+		});
 		if (A.out_macro)
 			write_macro(A, N.own(A), rho, vx, vy, vz);
 		if constexpr (ADE) {
 			real g[7];
 			const real phi = ade_update<ST, true>(B, in, vx, vy, vz, g);
-			elem* aout = (elem*) after<true>((char*) (AA ? B.df0 : B.df1), g[6]);
 			const real pr = (real) B.phi_ref, sc = (real) B.scale;
-			const uint64_t pbo = here(A.plane_bytes);
+			Planes<elem> aout(after<true>((char*) (AA ? B.df0 : B.df1), g[6]), here(A.plane_bytes));
 			N.local();
 #pragma unroll
-			for (int q = 0; q < 7; q++)
-				ade_put<ST>(dst(aout, pbo, q), MODE == LEAN_EVEN ? opp(q) : q, g[q], pr, sc, NT && (MODE != LEAN_ODD || CY[q] == 0));
+			for (int k = 0; k < 7; k++)
+				ade_put<ST>(dst(aout.next(), k), k, g[to(k)], pr, sc, NT && (MODE != LEAN_ODD || CY[k] == 0));
 			write_phi<ST>(A, B, N.own(A), phi);
 		}
 	};
