@@ -468,6 +468,24 @@ LBM_DEV char* sptr(char* p)
 	return p;
 }
 
+// The arrays of the directions in turn: two scalar additions each, where the
+// multiples of the stride, formed afresh for every access so as not to stay live,
+// took six: 548 -> 378 scalar instructions a wave, coupled 256^3 F16 1009 -> 986 us for
+// two steps, equal where HBM alone bounds the step.
+template <typename E, bool PIN = true>
+struct Planes
+{
+	char* p;
+	uint64_t pb;
+	LBM_DEV Planes(const void* base, uint64_t stride) : p((char*) base), pb(stride) {}
+	LBM_DEV E* next()
+	{
+		E* r = (E*) p;
+		p = sptr<PIN>(p + pb);
+		return r;
+	}
+};
+
 // Site of a lane of the even step: the stored offset of its block's row or
 // range (wave-uniform) and its own offset from there.  The even step moves
 // nothing between sites, so where the launch covers whole rows and columns of
@@ -628,17 +646,25 @@ k_aa_odd(const StepArgs A)
 		xrow[k] = (uint64_t) (xs[k] * A.Zs * A.Ys) * E;
 		zrow[k] = (uint32_t) zs[k] * (uint32_t) A.Ys * E;
 	}
-	auto slot_of = [&](char* base, int q, int cx, int cy, int cz) {
+	auto slot_of = [&](char* plane, int cx, int cy, int cz) {
 		if constexpr (LIN)
-			return (elem*) (sptr<PIN_ODD>(base + ((uint64_t) q * pb + xrow[1 + cx])) + (zrow[1 + cz] + ys[1 + cy]));
+			return (elem*) (sptr<PIN_ODD>(plane + xrow[1 + cx]) + (zrow[1 + cz] + ys[1 + cy]));
 		else {
 			const uint64_t row = (uint64_t) ((xs[1 + cx] * A.Zs + zs[1 + cz]) * A.Ys) * E;
-			return (elem*) (sptr<PIN_ODD>(base + ((uint64_t) q * pb + row)) + ys[1 + cy]);
+			return (elem*) (sptr<PIN_ODD>(plane + row) + ys[1 + cy]);
 		}
 	};
+	// The 2-byte forms in rows take the arrays in order: where the memory serves
+	// the allocation fast their issue bounds the step (512^3 F16 4986 -> 4835 us for
+	// both steps, 512x256x384 I16 1905 -> 1866); on slower allocations both orders
+	// are within 0.5% (BF16 256^3 1%).  The wider forms, which HBM bounds alone, and
+	// the linear mapping keep the pairs' order, up to 0.7% faster there.
+	constexpr bool WALK = ! LIN && E == 2;
+	Planes<char, PIN_ODD> in(df, pb);
 #pragma unroll
-	for (int q = 0; q < 27; q++) {
-		const elem* p = slot_of(df, opp(q), -CX[q], -CY[q], -CZ[q]);
+	for (int k = 0; k < 27; k++) {
+		const int q = WALK ? opp(k) : k;
+		const elem* p = slot_of(WALK ? in.next() : df + (uint64_t) opp(q) * pb, -CX[q], -CY[q], -CZ[q]);
 		if (NT_ODD && CY[q] == 0) {
 			const elem v = ld_nt(p);
 			f[q] = S::ld(&v, A.cls_sc[ncls(q)]);
@@ -648,13 +674,13 @@ k_aa_odd(const StepArgs A)
 	}
 	real rho, vx, vy, vz;
 	collide_site<ST, COLL>(f, A, rho, vx, vy, vz);
-	char* out = after<PIN_ODD>(df, f[26]);
-	auto dst = [&](int q) { return slot_of(out, q, CX[q], CY[q], CZ[q]); };
+	Planes<char, PIN_ODD> out(after<PIN_ODD>(df, f[26]), pb);
 	encode_all<ST, COLL>(f, A, [&](int q, elem v) {
+		elem* p = slot_of(WALK ? out.next() : out.p + (uint64_t) q * pb, CX[q], CY[q], CZ[q]);
 		if (NT_ODD && CY[q] == 0)
-			st_nt(dst(q), v);
+			st_nt(p, v);
 		else
-			*dst(q) = v;
+			*p = v;
 	});
 	if (A.out_macro)
 		write_macro(A, (xs[1] * A.Zs + zs[1]) * A.Ys + yl, rho, vx, vy, vz);
@@ -1499,24 +1525,6 @@ struct Stencil
 			return at((E*) sptr<true>((char*) base + xoff[1 + cx] * sizeof(E)), zr[1 + cz] + ys[1 + cy]);
 		else
 			return at((E*) sptr<true>((char*) base + (xoff[1 + cx] + (uint64_t) (zs[1 + cz] * (uint32_t) A.Ys)) * sizeof(E)), ys[1 + cy]);
-	}
-};
-
-// The arrays of the directions in turn: two scalar additions each, where the
-// multiples of the stride, formed afresh for every access so as not to stay live,
-// took six: 548 -> 378 scalar instructions a wave, coupled 256^3 F16 1009 -> 986 us for
-// two steps, equal where HBM alone bounds the step.
-template <typename E>
-struct Planes
-{
-	char* p;
-	uint64_t pb;
-	LBM_DEV Planes(const void* base, uint64_t stride) : p((char*) base), pb(stride) {}
-	LBM_DEV E* next()
-	{
-		E* r = (E*) p;
-		p = sptr<true>(p + pb);
-		return r;
 	}
 };
 
