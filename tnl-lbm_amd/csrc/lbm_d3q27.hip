@@ -532,8 +532,8 @@ static int make_step_args(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* S
 	if (nb >= (1ull << 31))
 		return fail(TNL_LBM_ERR_DIMS, "lattice box too large for one launch");
 	A.nblocks = (uint32_t) nb;
-	const uint32_t padded = padded_blocks(A);
 	A.even = SD->even_iter ? 1 : 0;
+	const uint32_t padded = padded_blocks(A);
 	A.out_macro = (flags & TNL_LBM_FLAG_OUTPUT_MACRO) ? 1 : 0;
 	A.macro_f64 = cfg->macro_real == TNL_LBM_REAL_F64;
 	A.dist_x = (flags & TNL_LBM_FLAG_DISTRIBUTED_X) != 0;

@@ -51,6 +51,7 @@ struct StepArgs
 	uint32_t nyb;      // y segments per row (linear mapping: blocks per x plane)
 	uint32_t nblocks;  // logical blocks
 	uint32_t group;    // log2 of the consecutive blocks of one XCD (logical_block)
+	int32_t backwards;  // the blocks in falling order
 	int32_t lin;       // linear y-z mapping (see linearize)
 	// the even A-A step over one contiguous range of stored sites (flat_range)
 	int32_t flat;
@@ -110,13 +111,46 @@ constexpr int NXCD = 8;
 LBM_DEV uint32_t logical_block(const StepArgs& A)
 {
 	const uint32_t k = blockIdx.x / NXCD;
-	return (((k >> A.group) * NXCD + blockIdx.x % NXCD) << A.group) + (k & ((1u << A.group) - 1u));
+	const uint32_t L = (((k >> A.group) * NXCD + blockIdx.x % NXCD) << A.group) + (k & ((1u << A.group) - 1u));
+	return A.backwards && L < A.nblocks ? A.nblocks - 1u - L : L;
+}
+// bytes of the step's population arrays
+inline uint64_t population_bytes(const StepArgs& A)
+{
+	return (A.df1 ? 54u : 27u) * A.plane_bytes;
+}
+constexpr uint64_t L2_BYTES = 32ull << 20;    // of all XCDs
+constexpr uint64_t LLC_BYTES = 256ull << 20;  // last-level cache
+// Whether steps that run in alternating order find enough of the arrays in the
+// last-level cache: five times its size at most.
+inline bool alternating(uint64_t bytes)
+{
+	return bytes <= 5 * LLC_BYTES;
 }
 // The grid for A.nblocks logical blocks.  Smaller groups where there would be
 // fewer than 16 for each XCD: the last ones keep one XCD busy alone (128x64x64,
 // groups of 1024: 208 us a pair of steps, of 32: 90).
+//
+// Where the arrays fit the L2 caches, an eighth of the grid to each XCD instead,
+// in one order: its L2 then still holds what it stepped before (48^3 FP64 18 us a
+// pair of steps, in groups 21; 65x55x58 BF16 16 and 21).
+//
+// Where they do not, but are no more than some times the last-level cache, odd
+// steps run through the blocks backwards: they begin where the step before ended,
+// with what that cache still holds, while in one order each step evicts what it
+// would need next.  One process and buffer, without / with: 189x233x43 FP64 A-A duct
+// 370 / 302 us, 262x85x95 FP64 coupled 561 / 477, 301x187x129 F16 channel 398 / 362,
+// 243x205x157 F32_DEV box 682 / 625, 150x90x96 FP64 A-B duct 220 / 201.
 inline uint32_t padded_blocks(StepArgs& A, uint32_t group = 5)
 {
+	if (population_bytes(A) <= L2_BYTES) {
+		A.backwards = 0;
+		A.group = 0;
+		while (((uint64_t) NXCD << A.group) < A.nblocks)
+			A.group++;
+		return (uint32_t) NXCD << A.group;
+	}
+	A.backwards = ! A.even && alternating(population_bytes(A));
 	while (group > 0 && ((uint64_t) NXCD << group) * 16 > A.nblocks)
 		group--;
 	A.group = group;
@@ -2136,12 +2170,14 @@ inline void list_shape(StepArgs& A, const uint32_t* rows, uint32_t nrows, unsign
 	grid = padded;
 }
 
-// Whether the populations fit the 256 MiB last-level cache, where one step
-// finds what the step before it wrote; nontemporal accesses give that up
-// (300x50x300 F16, 243 MB: 204 us for the two steps with them, 153 without).
+// Whether a step finds a part of `planes` population planes in the last-level
+// cache, where the step before it left them; nontemporal accesses give that up
+// (300x50x300 F16, 243 MB: 204 us for the two steps with them, 153 without; with
+// alternating order 128^3 FP64, 453 MB, 312 and 293; 48x320x320 FP64 slab, 1.1 GB,
+// 811 and 791; 192^3 FP64, 1.5 GB, equal; 256^3 F32, 1.8 GB, 1286 and 1316).
 inline bool cache_resident(const StepArgs& A, uint64_t planes = 27)
 {
-	return planes * A.plane_bytes <= (256ull << 20);
+	return alternating(planes * A.plane_bytes);
 }
 // Whether a step over `planes` population planes in all hints the streams that
 // no other wave touches: rows and planes start on lines, and the arrays exceed

@@ -48,6 +48,12 @@ def density_velocity(f: torch.Tensor, force=(0.0, 0.0, 0.0)):
     return rho, (j + 0.5 * F) / rho
 
 
+def _turn(d):
+    """The parity of the next A-B step: it decides only whether the step runs
+    through the lattice backwards, which alternates from step to step."""
+    d.even_iter = 0 if d.even_iter else 1
+
+
 MODES = ("recompute", "segment", "tape", "hybrid", "mixed")
 
 
@@ -201,7 +207,7 @@ class CheckpointedRun:
               fp32: bool = False):
         lat = self.lat
         cfg, d = (self.cfg32, self.d32) if fp32 else (lat.cfg, lat.d)
-        d.even_iter = 1
+        _turn(d)
         d.df[0], d.df[1] = src.data_ptr(), dst.data_ptr()
         if tape is None:
             lat._check(lat.lib.tnl_lbm_d3q27_step(C.byref(cfg), C.byref(d), _abi.I64x3(0, 0, 0),
@@ -212,7 +218,7 @@ class CheckpointedRun:
 
     def _record_from_f64(self, state: torch.Tensor, dst: torch.Tensor, tape: torch.Tensor, stream=None):
         lat, d = self.lat, self.d32
-        d.even_iter = 1
+        _turn(d)
         d.df[0] = d.df[1] = dst.data_ptr()
         lat._check(lat.lib.tnl_lbm_d3q27_step_record_from_f64(C.byref(self.cfg32), C.byref(d), _ptr(state), _ptr(tape),
                                                               _stream_ptr(stream)))
@@ -221,6 +227,7 @@ class CheckpointedRun:
                  tape: torch.Tensor | None = None, stream=None, fp32: bool = False):
         lat = self.lat
         cfg, d = (self.cfg32, self.d32) if fp32 else (lat.cfg, lat.d)
+        _turn(d)
         if tape is None:
             d.df[0], d.df[1] = state.data_ptr(), None
             lat._check(lat.lib.tnl_lbm_d3q27_adjoint_step(C.byref(cfg), C.byref(d), _ptr(lam_next), _ptr(lam),
@@ -430,7 +437,8 @@ class CoupledScalarRun:
         if ubuf is not None:
             nse.d.macro = ubuf.data_ptr()
             ade.d.macro = self.lam[0].data_ptr()  # phi, not needed: the adjoint fields are free in a forward pass
-        nse.d.even_iter = ade.d.even_iter = 1
+        _turn(nse.d)
+        ade.d.even_iter = nse.d.even_iter
         nse.d.df[0], nse.d.df[1] = fs.data_ptr(), fd.data_ptr()
         ade.d.df[0], ade.d.df[1] = gs.data_ptr(), gd.data_ptr()
         self._launch(nse.lib.tnl_lbm_nse_ade_step(C.byref(nse.cfg), C.byref(nse.d), C.byref(ade.d),
@@ -439,7 +447,7 @@ class CoupledScalarRun:
 
     def _flow_step(self, fs, fd, ubuf, stream=None):
         nse = self.nse
-        nse.d.even_iter = 1
+        _turn(nse.d)
         nse.d.df[0], nse.d.df[1] = fs.data_ptr(), fd.data_ptr()
         nse.d.macro = ubuf.data_ptr()
         self._launch(nse.lib.tnl_lbm_d3q27_step(C.byref(nse.cfg), C.byref(nse.d), _abi.I64x3(0, 0, 0),
