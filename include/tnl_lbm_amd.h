@@ -176,7 +176,9 @@ typedef struct tnl_lbm_d3q27_data {
 	int64_t X, Y, Z;      /* local sizes without overlaps (LBM_Data::X/Y/Z) */
 	int64_t ox, oy, oz;   /* overlaps (indexer overlaps; 0 on one GPU)      */
 	int64_t XYZ;          /* population stride; >= (X+2ox)(Y+2oy)(Z+2oz)    */
-	int32_t even_iter;    /* A-A parity, LBM::updateKernelData (lbm.hpp:311) */
+	int32_t even_iter;    /* A-A parity, LBM::updateKernelData (lbm.hpp:311); A-B: the
+	                       * results do not depend on it, steps that alternate it find
+	                       * more of the arrays in the cache */
 	int32_t inflow_profile_real; /* enum tnl_lbm_real: element type of inflow_profile
 	                                (F64 = 0, the default; F32 for TraitsSP's dreal) */
 	double lbm_viscosity; /* LBM_Data::lbmViscosity                          */

@@ -986,7 +986,7 @@ LBM_DEV E* slot0(E* base, int q, const StepArgs& A, int64_t s)
 // NTG: nontemporal hints on the A-B streams no other wave touches in this step
 // (the site's own slots, and the pulls with c_y = 0; the +-1 shifted rows share
 // cache lines with the neighbouring wave), where rows start on lines and the
-// arrays exceed the last-level cache (hint_streams): 256^3 F16 +2%, F32 +3%;
+// last-level cache holds too little of the arrays (hint_streams): 256^3 F16 +2%, F32 +3%;
 // rows off the lines 301x187x129 F16 282 us with them and 187 without, arrays
 // within the cache 128x64x64 FP64 48.6 and 41.
 template <int ST, int COLL, int PATTERN, int TAPE = 0, bool O32 = false, bool LISTED = false, bool NTG = false>
@@ -2180,8 +2180,8 @@ inline bool cache_resident(const StepArgs& A, uint64_t planes = 27)
 	return alternating(planes * A.plane_bytes);
 }
 // Whether a step over `planes` population planes in all hints the streams that
-// no other wave touches: rows and planes start on lines, and the arrays exceed
-// the last-level cache.
+// no other wave touches: rows and planes start on lines, and the last-level cache
+// holds too little of the arrays.
 inline bool hint_streams(const StepArgs& A, uint64_t planes, size_t elem)
 {
 	return ! cache_resident(A, planes) && A.plane_bytes % 128 == 0 && (uintptr_t) A.df0 % 128 == 0
@@ -2192,7 +2192,7 @@ inline bool hint_streams(const StepArgs& A, uint64_t planes, size_t elem)
 // range where the box covers whole rows and columns of a lattice without y and
 // z overlaps, else rows.  Returns whether to use nontemporal hints: where every
 // wave's accesses cover whole lines (the planes and each wave's first site
-// start on a 128-byte line) and the populations exceed the last-level cache.
+// start on a 128-byte line) and the last-level cache holds too little of the arrays.
 inline bool even_shape(StepArgs& A, uint32_t per, unsigned most, unsigned& threads, unsigned& grid, size_t elem)
 {
 	const bool planes = A.plane_bytes % 128 == 0 && (uintptr_t) A.df0 % 128 == 0 && ! cache_resident(A);
