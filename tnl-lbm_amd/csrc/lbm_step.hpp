@@ -558,15 +558,20 @@ LBM_DEV bool even_site(const StepArgs& A, uint32_t per, uint64_t& row, uint32_t&
 // and the store swaps them back.  Waves of walls alone leave theirs; in other
 // waves the walls store what they loaded, since a gap would leave partial lines.
 
+// (no map: a box with a force field alone, every site PERIODIC)
+LBM_DEV int16_t code_at(const StepArgs& A, int64_t s)
+{
+	return A.map ? A.map[s] : (int16_t) GEO_PERIODIC;
+}
 // whether the site collides (a wall keeps its populations)
 LBM_DEV bool even_active(const StepArgs& A, int64_t s)
 {
-	const int16_t gi = A.map[s];
+	const int16_t gi = code_at(A, s);
 	return gi == GEO_FLUID || gi == GEO_PERIODIC;
 }
 LBM_DEV void wall_macro(const StepArgs& A, int64_t s, bool f64)
 {
-	if (A.out_macro && A.map[s] == GEO_WALL) {
+	if (A.out_macro && code_at(A, s) == GEO_WALL) {
 		if (f64)
 			write_macro(A, s, 1.0, 0.0, 0.0, 0.0);
 		else
@@ -591,7 +596,7 @@ k_aa_even(const StepArgs A)
 		return;
 	bool wall = false;
 	if constexpr (MAP) {
-		const int16_t gi = A.map[(int64_t) first + yl];
+		const int16_t gi = code_at(A, (int64_t) first + yl);
 		wall = gi == GEO_WALL;
 		const bool moves = gi == GEO_FLUID || gi == GEO_PERIODIC;
 		const uint64_t any = __ballot(moves);
