@@ -253,11 +253,14 @@ uint32_t tnl_lbm_abi_version(void);
 const char* tnl_lbm_last_error(void);
 
 /* No counterpart in the reference: a diagnostic switch.  Where a population
- * array holds at most 4 GiB, the map kernel (2-byte forms), the coupled
- * kernel (2-byte forms), the recording step and the FP64 adjoint address
- * each slot as a per-direction base plus a 32-bit offset; on = 1 makes every
- * launch of this process take the 64-bit form (same results, bit for bit),
- * on = 0 restores the default.  Returns the previous setting.              */
+ * array holds at most 4 GiB, the map kernel and the coupled kernel with every
+ * boundary code (2-byte forms) and the recording step address each slot as a
+ * per-direction base plus a 32-bit offset, and the D3Q27 adjoint step does
+ * where one x plane of the array holds at most 4 GiB; on = 1 makes every
+ * launch of these kernels in this process take the 64-bit form (same results,
+ * bit for bit), on = 0 restores the default.  Which kernels a step takes does
+ * not depend on it: those without a 64-bit form keep theirs.  Returns the
+ * previous setting.                                                         */
 int tnl_lbm_set_wide_addressing(int on);
 
 /* No counterpart in the reference: classification of the interior (x, z)

@@ -158,10 +158,16 @@ inline uint32_t padded_blocks(StepArgs& A, uint32_t group = 5)
 	return (A.nblocks + whole - 1) / whole * whole;
 }
 
-// one x plane of a population array of `elem`-byte elements takes 32-bit offsets
+// One x plane of a population array of `elem`-byte elements takes 32-bit offsets.
+// plane_fits alone decides for the kernels that have no other form (lean, linear odd
+// step): the addressing switch chooses between the forms of one kernel only.
+inline bool plane_fits(const StepArgs& A, size_t elem)
+{
+	return (uint64_t) A.Ys * (uint64_t) A.Zs * elem <= (1ull << 32);
+}
 inline bool narrow_planes(const StepArgs& A, size_t elem)
 {
-	return narrow_slots_allowed() && (uint64_t) A.Ys * (uint64_t) A.Zs * elem <= (1ull << 32);
+	return narrow_slots_allowed() && plane_fits(A, elem);
 }
 
 // per-site force of MACRO::computeForcing (kernels.h:103): added to the
@@ -2269,7 +2275,7 @@ template <int ST, int COLL, bool NTO>
 void odd_launch(const StepArgs& A0, unsigned threads, unsigned grid, hipStream_t st)
 {
 	StepArgs A = A0;
-	if (A.ny % (int32_t) threads && (uint64_t) A.Ys * (uint64_t) A.Zs * sizeof(typename Storage<ST>::elem) <= (1ull << 32)) {
+	if (A.ny % (int32_t) threads && plane_fits(A, sizeof(typename Storage<ST>::elem))) {
 		threads = 256;
 		const uint64_t plane = (uint64_t) A.ny * (uint64_t) A.nz;
 		while (threads > 64 && plane * (uint64_t) A.nx < (uint64_t) threads * 2048)
@@ -2312,7 +2318,7 @@ int launch_periodic(const StepArgs& A, unsigned threads, unsigned grid, hipStrea
 inline bool lean_split(const StepArgs& A, size_t elem)
 {
 	const int64_t rows = A.list_count[0] + A.list_count[1] + A.list_count[2];
-	return A.lists && narrow_planes(A, elem) && rows == A.X * A.Z && A.list_count[0] * 8 <= rows;
+	return A.lists && plane_fits(A, elem) && rows == A.X * A.Z && A.list_count[0] * 8 <= rows;
 }
 
 // Launch shape of a lean kernel: rows of whole blocks with hints, else the
