@@ -210,11 +210,14 @@ typedef struct tnl_lbm_d3q27_data {
 	/* Row lists of this map (no counterpart in the reference; NULL = none):
 	 * the output of tnl_lbm_classify_rows(SD, NULL, ...).  A step over the
 	 * whole box (offset 0, end = X, Y, Z) of the default cumulant then takes
-	 * its FLUID, PERIODIC and WALL sites through kernels without the other
-	 * boundary codes, and the other sites of the class 0 rows through the
-	 * kernel with every code (where those rows are at most an eighth of all;
-	 * the A-B steps of F64 and F32: where there are none).  The lists must
-	 * describe the current map: classify again after changing it.            */
+	 * the other sites of the class 0 rows through the kernel with every
+	 * boundary code, and its FLUID, PERIODIC and WALL sites through kernels
+	 * without the other codes (where the class 0 rows are at most an eighth of
+	 * all, in A-A steps of the deviation forms and coupled ones a quarter; the
+	 * A-B steps of F64 and F32: where there are none).  Where they are more,
+	 * those A-A steps launch the class 0 rows, then the others, and the other
+	 * steps take no lists.  The lists must describe the current map: classify
+	 * again after changing it.                                               */
 	const uint32_t* rows;
 	int64_t row_count[3];
 } tnl_lbm_d3q27_data;

@@ -648,7 +648,16 @@ int tnl_lbm_nse_ade_step(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* ns
 			return hip_check(hipGetLastError(), "nse_ade launch");
 		};
 		// the lean kernels step both lattices in one parity
-		if (lean_split(A, E) && (ab || B.even == A.even)) {
+		const bool ordered = in_order(A, true, cfg->pattern);
+		if (lean_split(A, E, ordered) && (ab || B.even == A.even)) {
+			if (A.list_count[0] > 0) {
+				StepArgs C = A;
+				C.others = 1;
+				unsigned t = threads, g = grid;
+				list_shape(C, A.lists, (uint32_t) A.list_count[0], t, g);
+				if (int rc = general(std::true_type{}, C, t, g))
+					return rc;
+			}
 			lean_shape(A, ab ? 68 : 34, E, [&](const StepArgs& C, unsigned t, unsigned g, bool lin) {
 				auto mode = [&](auto mc) {
 					constexpr int MODE = decltype(mc)::value;
@@ -664,15 +673,10 @@ int tnl_lbm_nse_ade_step(const tnl_lbm_config* cfg, const tnl_lbm_d3q27_data* ns
 				else
 					mode(std::integral_constant<int, LEAN_ODD>{});
 			});
-			if (int rc = hip_check(hipGetLastError(), "nse_ade launch"))
-				return rc;
-			if (A.list_count[0] == 0)
-				return (int) TNL_LBM_OK;
-			StepArgs C = A;
-			unsigned t = threads, g = grid;
-			list_shape(C, A.lists, (uint32_t) A.list_count[0], t, g);
-			return general(std::true_type{}, C, t, g);
+			return hip_check(hipGetLastError(), "nse_ade launch");
 		}
+		if (ordered && lists_cover(A))
+			return in_turn(A, [&](const StepArgs& C, unsigned t, unsigned g) { return general(std::true_type{}, C, t, g); });
 		StepArgs C = A;
 		unsigned t = threads, g = grid;
 		linearize(C, t, g);

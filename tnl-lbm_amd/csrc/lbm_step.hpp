@@ -76,6 +76,7 @@ struct StepArgs
 	// after another), or null
 	const uint32_t* lists;
 	int64_t list_count[3];
+	int32_t others;  // listed launches: the sites of other codes than the plain ones only
 };
 
 enum : int16_t
@@ -787,18 +788,19 @@ struct PairCodec
 // high halves still hold site s + 1's inputs, so one packed array serves
 // both sites (binary16 writes a half and keeps the other in one
 // instruction).
+// (MAP: a site that does not collide, `lo` or `hi` false, writes no macros here)
 template <int ST, int COLL, bool MAP = false>
-LBM_DEV void collide_pair(uint32_t* w, const StepArgs& A, int64_t s)
+LBM_DEV void collide_pair(uint32_t* w, const StepArgs& A, int64_t s, bool lo = true, bool hi = true)
 {
 	using C = PairCodec<ST, COLL>;
 	float f[27];
 	float rho, vx, vy, vz;
-	auto site = [&](int64_t i) {
+	auto site = [&](int64_t i, bool on) {
 		float Fx = (float) A.fx, Fy = (float) A.fy, Fz = (float) A.fz;
 		if (MAP && A.force)
 			add_site_force(A, i, Fx, Fy, Fz);
 		collide_site<ST, COLL>(f, A, Fx, Fy, Fz, rho, vx, vy, vz);
-		if (A.out_macro)
+		if (A.out_macro && (! MAP || on))
 			write_macro(A, i, rho, vx, vy, vz);
 	};
 	if constexpr (C::PACK2) {
@@ -810,14 +812,14 @@ LBM_DEV void collide_pair(uint32_t* w, const StepArgs& A, int64_t s)
 #pragma unroll
 		for (int q = 0; q < 27; q++)
 			f[q] = C::get(w[q] & 0xffffu, q, A);
-		site(s);
+		site(s, lo);
 #pragma unroll
 		for (int q = 0; q < 27; q++)
 			a[q] = C::scaled(f[q], q, A);
 #pragma unroll
 		for (int q = 0; q < 27; q++)
 			f[q] = C::get(w[q] >> 16, q, A);
-		site(s + 1);
+		site(s + 1, hi);
 #pragma unroll
 		for (int q = 0; q < 27; q++)
 			w[q] = C::pack2(a[q], C::scaled(f[q], q, A));
@@ -826,14 +828,14 @@ LBM_DEV void collide_pair(uint32_t* w, const StepArgs& A, int64_t s)
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		f[q] = C::get(w[q] & 0xffffu, q, A);
-	site(s);
+	site(s, lo);
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		w[q] = (w[q] & 0xffff0000u) | C::put(f[q], q, A);
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		f[q] = C::get(w[q] >> 16, q, A);
-	site(s + 1);
+	site(s + 1, hi);
 #pragma unroll
 	for (int q = 0; q < 27; q++)
 		w[q] = (w[q] & 0xffffu) | (C::put(f[q], q, A) << 16);
@@ -869,7 +871,7 @@ __global__ void __launch_bounds__(256) k_aa_even_pair(const StepArgs A)
 		const uint32_t* p = (const uint32_t*) (sptr<PIN>(df + ((uint64_t) q * pb + row)) + yb);
 		w[q] = NT ? __builtin_nontemporal_load(p) : *p;
 	}
-	collide_pair<ST, COLL, MAP>(w, A, (int64_t) (row / 2) + yl);
+	collide_pair<ST, COLL, MAP>(w, A, (int64_t) (row / 2) + yl, lo, hi);
 	if constexpr (MAP) {
 		if (! (lo && hi)) {
 			// one plain site of the pair: its half only
@@ -991,8 +993,8 @@ LBM_DEV E* slot0(E* base, int q, const StepArgs& A, int64_t s)
 // access is one scalar-base load or store, in place of a 64-bit address per
 // lane and access.
 //
-// LISTED: the launch covers rows that hold other codes than the plain ones, and
-// steps their other sites only: the plain ones belong to the lean kernels.
+// LISTED: the launch covers a list of rows; with A.others it steps their sites of
+// other codes only, the plain ones belonging to the lean kernels.
 //
 // NTG: nontemporal hints on the A-B streams no other wave touches in this step
 // (the site's own slots, and the pulls with c_y = 0; the +-1 shifted rows share
@@ -1101,7 +1103,7 @@ struct General
 	{
 		const int64_t s0 = sidx(A, x + A.ox, y + A.oy, z + A.oz);
 		const int16_t gi = A.map ? __builtin_nontemporal_load(A.map + s0) : (int16_t) GEO_PERIODIC;
-		if (LISTED && plain(gi))
+		if (LISTED && A.others && plain(gi))
 			return;
 		const bool per = gi == GEO_PERIODIC;
 		NX = neighbours<AA>(x, A.X, A.ox, A.dist_x, per);
@@ -1475,7 +1477,7 @@ __global__ void __launch_bounds__(256) k_nse_ade(const StepArgs A, const AdeArgs
 	const int64_t s0 = ((x + A.ox) * A.Zs + (z + A.oz)) * A.Ys + (y + A.oy);
 	const int16_t gn = A.map ? A.map[s0] : (int16_t) GEO_PERIODIC;
 	const int16_t ga = B.map ? B.map[s0] : (int16_t) A_PERIODIC;
-	if (LISTED && plain(gn) && plain_scalar(ga))
+	if (LISTED && A.others && plain(gn) && plain_scalar(ga))
 		return;
 	// neighbours as General::site forms them (periodic wrap for PERIODIC-coded sites)
 	const bool per = gn == GEO_PERIODIC;
@@ -1521,7 +1523,7 @@ __global__ void __launch_bounds__(256) k_nse_ade(const StepArgs A, const AdeArgs
 // Lean kernels: the plain sites (FLUID, PERIODIC, WALL) of a box with a
 // geometry map, flow alone (A-A odd step, A-B step) or coupled (all three).
 // The sites of any other code are skipped; a launch of the general kernels
-// over the rows that hold them (LISTED) steps those.
+// over the rows that hold them (LISTED) steps those before.
 //
 // A kernel's registers are the maximum over all of its paths, so the rarely
 // taken boundary codes cost every site of the general kernels their occupancy
@@ -2311,14 +2313,49 @@ int launch_periodic(const StepArgs& A, unsigned threads, unsigned grid, hipStrea
 	return hip_check(hipGetLastError(), "step launch");
 }
 
+inline bool lists_cover(const StepArgs& A)
+{
+	return A.lists && A.list_count[0] + A.list_count[1] + A.list_count[2] == A.X * A.Z;
+}
+
+// In place, a site whose code pulls from another site's slots (OUTFLOW_RIGHT, and
+// OUTFLOW_RIGHT_INTERP, from column x - 1) reads them as they were before the step
+// if the rows that hold other codes are stepped first: in one launch the two sites
+// race, and after it such a site reads the step's results.  So the A-A steps of the
+// deviation forms and the coupled ones step those rows first, with the lean kernels
+// or without (in_turn).  (F64 and F32 without them in one launch.)
+inline bool in_order(const StepArgs& A, bool dev_or_coupled, int pattern)
+{
+	return dev_or_coupled && pattern == TNL_LBM_PATTERN_AA && A.list_count[0] > 0 && A.list_count[0] < A.X * A.Z;
+}
+
 // Whether a full-box launch with row lists takes the lean kernels: x planes
 // within 32-bit offsets, and few rows with other codes (each of those is read
 // again by the general kernel; from an eighth of the rows on, that launch costs
-// what the lean one saves)
-inline bool lean_split(const StepArgs& A, size_t elem)
+// what the lean one saves).  Steps that keep the order need two launches
+// anyhow: up to a quarter.  A-A F16 128x128 rows, flow / coupled, us for two
+// steps, lean and in turn: 64 planes, a fifth of the rows 74 / 89 and 78 / 111,
+// half 91 / 108 and 81 / 109 (in one launch, out of order, 68 / 93 and 68 / 97).
+inline bool lean_split(const StepArgs& A, size_t elem, bool ordered)
 {
-	const int64_t rows = A.list_count[0] + A.list_count[1] + A.list_count[2];
-	return A.lists && plane_fits(A, elem) && rows == A.X * A.Z && A.list_count[0] * 8 <= rows;
+	return lists_cover(A) && plane_fits(A, elem) && A.list_count[0] * (ordered ? 4 : 8) <= A.X * A.Z;
+}
+
+// The rows that hold other codes in one launch of the general kernel, then the rest
+// in another.  go(shape, threads, grid) makes a launch.
+template <typename Go>
+int in_turn(const StepArgs& A, Go&& go)
+{
+	const int64_t first = A.list_count[0];
+	const int64_t rest = A.X * A.Z - first;
+	for (int k = 0; k < 2; k++) {
+		StepArgs B = A;
+		unsigned threads = 0, grid = 0;
+		list_shape(B, A.lists + (k ? first : 0), (uint32_t) (k ? rest : first), threads, grid);
+		if (int rc = go(B, threads, grid))
+			return rc;
+	}
+	return 0;
 }
 
 // Launch shape of a lean kernel: rows of whole blocks with hints, else the
@@ -2392,26 +2429,34 @@ int launch_step(const tnl_lbm_config* cfg, const StepArgs& A, unsigned threads, 
 	// the map-free periodic kernels take the homogeneous force only
 	if (! A.map && ! A.force && cfg->pattern == TNL_LBM_PATTERN_AA)
 		return launch_periodic<ST, COLL>(A, threads, grid, st);
-	// The lean kernels for the plain sites, then the rows that hold others.
+	// The rows that hold other codes (in_order says why first), then the lean
+	// kernels for the plain sites.
 	// The A-B steps of FP64 and F32 take them where there are none such: their
 	// map kernel is bound by HBM, and the second launch costs more than it gains.
 	if constexpr (COLL == TNL_LBM_COLL_CUM) {
-		if (lean_split(A, sizeof(typename Storage<ST>::elem)) && (Storage<ST>::dev || cfg->pattern == TNL_LBM_PATTERN_AA || A.list_count[0] == 0)) {
+		const bool ordered = in_order(A, Storage<ST>::dev, cfg->pattern);
+		if (lean_split(A, sizeof(typename Storage<ST>::elem), ordered) && (Storage<ST>::dev || cfg->pattern == TNL_LBM_PATTERN_AA || A.list_count[0] == 0)) {
+			if (A.list_count[0] > 0) {
+				StepArgs B = A;
+				B.others = 1;
+				list_shape(B, A.lists, (uint32_t) A.list_count[0], threads, grid);
+				launch_general<ST, COLL, true>(cfg->pattern, B, threads, grid, st);
+				if (int rc = hip_check(hipGetLastError(), "step launch"))
+					return rc;
+			}
 			if (cfg->pattern == TNL_LBM_PATTERN_AB)
 				lean_launch<ST, LEAN_AB>(A, st);
 			else if (! A.even)
 				lean_launch<ST, LEAN_ODD>(A, st);
-			else if (int rc = even_launch<ST, COLL, true>(A, st))
-				return rc;
-			if (int rc = hip_check(hipGetLastError(), "step launch"))
-				return rc;
-			if (A.list_count[0] > 0) {
-				StepArgs B = A;
-				list_shape(B, A.lists, (uint32_t) A.list_count[0], threads, grid);
-				launch_general<ST, COLL, true>(cfg->pattern, B, threads, grid, st);
-			}
+			else
+				return even_launch<ST, COLL, true>(A, st);
 			return hip_check(hipGetLastError(), "step launch");
 		}
+		if (ordered && lists_cover(A))
+			return in_turn(A, [&](const StepArgs& B, unsigned t, unsigned g) {
+				launch_general<ST, COLL, true>(cfg->pattern, B, t, g, st);
+				return hip_check(hipGetLastError(), "step launch");
+			});
 	}
 	StepArgs B = A;
 	linearize(B, threads, grid);
