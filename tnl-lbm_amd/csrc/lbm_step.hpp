@@ -50,7 +50,7 @@ struct StepArgs
 	int32_t nx, ny, nz;
 	uint32_t nyb;      // y segments per row (linear mapping: blocks per x plane)
 	uint32_t nblocks;  // logical blocks
-	uint32_t group;    // log2 of the consecutive blocks of one XCD (logical_block)
+	uint32_t group, span;  // which logical blocks belong to one XCD (block_of)
 	int32_t backwards;  // the blocks in falling order
 	int32_t lin;       // linear y-z mapping (see linearize)
 	// the even A-A step over one contiguous range of stored sites (flat_range)
@@ -109,10 +109,16 @@ constexpr int NXCD = 8;
 // 794 / 789 / 817 us; 256x96x96 mixed gradient 15.1 / 12.5 / 12.3 / 12.3 / 12.5 ms;
 // 301x417x333 F32_DEV box 4359 / - / 3498 / 3477 / 3480 us; 512^3 FP64 box 18.95 /
 // 22.9 / 19.05 / 18.90 / 18.81 ms (singly, the XCDs fetch each other's lines).
+// (block_of: groups of 2^group blocks with span = 2^group; one run of `span` blocks
+// for each XCD with group = 31)
+__host__ __device__ __forceinline__ uint32_t block_of(uint32_t b, uint32_t group, uint32_t span)
+{
+	const uint32_t k = b / NXCD;
+	return ((k >> group) * NXCD + b % NXCD) * span + (k & ((1u << group) - 1u));
+}
 LBM_DEV uint32_t logical_block(const StepArgs& A)
 {
-	const uint32_t k = blockIdx.x / NXCD;
-	const uint32_t L = (((k >> A.group) * NXCD + blockIdx.x % NXCD) << A.group) + (k & ((1u << A.group) - 1u));
+	const uint32_t L = block_of(blockIdx.x, A.group, A.span);
 	return A.backwards && L < A.nblocks ? A.nblocks - 1u - L : L;
 }
 // bytes of the step's population arrays
@@ -134,7 +140,9 @@ inline bool alternating(uint64_t bytes)
 //
 // Where the arrays fit the L2 caches, an eighth of the grid to each XCD instead,
 // in one order: its L2 then still holds what it stepped before (48^3 FP64 18 us a
-// pair of steps, in groups 21; 65x55x58 BF16 16 and 21).
+// pair of steps, in groups 21; 65x55x58 BF16 16 and 21).  Runs of the same length
+// for all XCDs: with powers of two, some of them idle (48x61x53 FP64 coupled A-A 57
+// us and 45, 30x300x30 F16 32 and 26).
 //
 // Where they do not, but are no more than some times the last-level cache, odd
 // steps run through the blocks backwards: they begin where the step before ended,
@@ -146,15 +154,15 @@ inline uint32_t padded_blocks(StepArgs& A, uint32_t group = 5)
 {
 	if (population_bytes(A) <= L2_BYTES) {
 		A.backwards = 0;
-		A.group = 0;
-		while (((uint64_t) NXCD << A.group) < A.nblocks)
-			A.group++;
-		return (uint32_t) NXCD << A.group;
+		A.group = 31;
+		A.span = (A.nblocks + NXCD - 1) / NXCD;
+		return NXCD * A.span;
 	}
 	A.backwards = ! A.even && alternating(population_bytes(A));
 	while (group > 0 && ((uint64_t) NXCD << group) * 16 > A.nblocks)
 		group--;
 	A.group = group;
+	A.span = 1u << group;
 	const uint32_t whole = (uint32_t) NXCD << group;
 	return (A.nblocks + whole - 1) / whole * whole;
 }
