@@ -212,12 +212,12 @@ typedef struct tnl_lbm_d3q27_data {
 	 * whole box (offset 0, end = X, Y, Z) of the default cumulant then takes
 	 * the other sites of the class 0 rows through the kernel with every
 	 * boundary code, and its FLUID, PERIODIC and WALL sites through kernels
-	 * without the other codes (where the class 0 rows are at most an eighth of
-	 * all, in A-A steps of the deviation forms and coupled ones a quarter; the
-	 * A-B steps of F64 and F32: where there are none).  Where they are more,
-	 * those A-A steps launch the class 0 rows, then the others, and the other
-	 * steps take no lists.  The lists must describe the current map: classify
-	 * again after changing it.                                               */
+	 * without the other codes (deviation forms and coupled steps: where the
+	 * class 0 rows are at most an eighth of all, a quarter in A-A steps; flow
+	 * steps of F64 and F32: where there are none).  Where they are more, the
+	 * A-A steps of the former launch the class 0 rows, then the others, and
+	 * other steps take no lists.  The lists must describe the current map:
+	 * classify again after changing it.                                      */
 	const uint32_t* rows;
 	int64_t row_count[3];
 } tnl_lbm_d3q27_data;

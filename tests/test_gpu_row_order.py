@@ -1,4 +1,4 @@
-"""The A-A steps over row lists run the rows that hold other codes first: a site whose
+"""The A-A steps over row lists (deviation forms, coupled) run the rows that hold other codes first: a site whose
 code pulls from another site's slots (OUTFLOW_RIGHT of either lattice) reads them as
 they were before the step.  Against launches over sub-boxes, which take no lists: the
 outlet's plane, then the rest.  Tolerance as for the row lists: 16 epsilons of an
@@ -36,8 +36,7 @@ def outlet_first(lat, step):
     step(end=(lat.X - 1, lat.Y, lat.Z))
 
 
-@pytest.mark.parametrize("shape,storage", [(s, f) for s in SPARSE for f in ("f64", "f32", "f32dev", "f16dev", "bf16dev", "i16dev")]
-                         + [(s, f) for s in DENSE for f in ("f32dev", "f16dev", "bf16dev", "i16dev")])
+@pytest.mark.parametrize("shape,storage", [(s, f) for s in SPARSE + DENSE for f in ("f32dev", "f16dev", "bf16dev", "i16dev")])
 def test_step(storage, shape):
     X, Y, Z = shape
     geo = channel(X, Y, Z, GEO)

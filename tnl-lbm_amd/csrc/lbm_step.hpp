@@ -2331,7 +2331,7 @@ inline bool lists_cover(const StepArgs& A)
 // if the rows that hold other codes are stepped first: in one launch the two sites
 // race, and after it such a site reads the step's results.  So the A-A steps of the
 // deviation forms and the coupled ones step those rows first, with the lean kernels
-// or without (in_turn).  (F64 and F32 without them in one launch.)
+// or without (in_turn).  (FP64 and F32 flow steps go through one launch.)
 inline bool in_order(const StepArgs& A, bool dev_or_coupled, int pattern)
 {
 	return dev_or_coupled && pattern == TNL_LBM_PATTERN_AA && A.list_count[0] > 0 && A.list_count[0] < A.X * A.Z;
@@ -2439,18 +2439,23 @@ int launch_step(const tnl_lbm_config* cfg, const StepArgs& A, unsigned threads, 
 		return launch_periodic<ST, COLL>(A, threads, grid, st);
 	// The rows that hold other codes (in_order says why first), then the lean
 	// kernels for the plain sites.
-	// The A-B steps of FP64 and F32 take them where there are none such: their
-	// map kernel is bound by HBM, and the second launch costs more than it gains.
+	// FP64 and F32 take them where there are no such rows: their map kernel is bound
+	// by HBM, and the second launch costs more than it gains (A-A ducts, two steps,
+	// with it / in one launch: FP64 24^3 28 / 22 us, 64^3 56 / 51, 160x128x128 396 /
+	// 386; F32 24^3 26 / 19, 200x131x128 272 / 256).
 	if constexpr (COLL == TNL_LBM_COLL_CUM) {
-		const bool ordered = in_order(A, Storage<ST>::dev, cfg->pattern);
-		if (lean_split(A, sizeof(typename Storage<ST>::elem), ordered) && (Storage<ST>::dev || cfg->pattern == TNL_LBM_PATTERN_AA || A.list_count[0] == 0)) {
-			if (A.list_count[0] > 0) {
-				StepArgs B = A;
-				B.others = 1;
-				list_shape(B, A.lists, (uint32_t) A.list_count[0], threads, grid);
-				launch_general<ST, COLL, true>(cfg->pattern, B, threads, grid, st);
-				if (int rc = hip_check(hipGetLastError(), "step launch"))
-					return rc;
+		constexpr bool DEV = Storage<ST>::dev;
+		const bool ordered = in_order(A, DEV, cfg->pattern);
+		if (lean_split(A, sizeof(typename Storage<ST>::elem), ordered) && (DEV || A.list_count[0] == 0)) {
+			if constexpr (DEV) {
+				if (A.list_count[0] > 0) {
+					StepArgs B = A;
+					B.others = 1;
+					list_shape(B, A.lists, (uint32_t) A.list_count[0], threads, grid);
+					launch_general<ST, COLL, true>(cfg->pattern, B, threads, grid, st);
+					if (int rc = hip_check(hipGetLastError(), "step launch"))
+						return rc;
+				}
 			}
 			if (cfg->pattern == TNL_LBM_PATTERN_AB)
 				lean_launch<ST, LEAN_AB>(A, st);
@@ -2460,11 +2465,13 @@ int launch_step(const tnl_lbm_config* cfg, const StepArgs& A, unsigned threads, 
 				return even_launch<ST, COLL, true>(A, st);
 			return hip_check(hipGetLastError(), "step launch");
 		}
-		if (ordered && lists_cover(A))
-			return in_turn(A, [&](const StepArgs& B, unsigned t, unsigned g) {
-				launch_general<ST, COLL, true>(cfg->pattern, B, t, g, st);
-				return hip_check(hipGetLastError(), "step launch");
-			});
+		if constexpr (DEV) {
+			if (ordered && lists_cover(A))
+				return in_turn(A, [&](const StepArgs& B, unsigned t, unsigned g) {
+					launch_general<ST, COLL, true>(cfg->pattern, B, t, g, st);
+					return hip_check(hipGetLastError(), "step launch");
+				});
+		}
 	}
 	StepArgs B = A;
 	linearize(B, threads, grid);
