@@ -21,7 +21,7 @@ bool narrow_slots_allowed() { return true; }
 int main()
 {
 	using namespace lbm;
-	// arrays within the L2 caches, within some times the last-level cache, beyond it
+	// arrays within half the last-level cache, within some times it, beyond
 	const uint64_t bytes[] = {1ull << 20, 20ull << 20, 300ull << 20, 4000ull << 20};
 	const uint32_t counts[] = {1, 7, 8, 9, 63, 64, 65, 128, 129, 1023, 1025, 2448, 2544, 4095, 4096, 4097, 20000, 32769, 131073};
 	int bad = 0;

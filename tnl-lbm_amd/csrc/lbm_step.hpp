@@ -126,7 +126,6 @@ inline uint64_t population_bytes(const StepArgs& A)
 {
 	return (A.df1 ? 54u : 27u) * A.plane_bytes;
 }
-constexpr uint64_t L2_BYTES = 32ull << 20;    // of all XCDs
 constexpr uint64_t LLC_BYTES = 256ull << 20;  // last-level cache
 // Whether steps that run in alternating order find enough of the arrays in the
 // last-level cache: five times its size at most.
@@ -138,11 +137,14 @@ inline bool alternating(uint64_t bytes)
 // fewer than 16 for each XCD: the last ones keep one XCD busy alone (128x64x64,
 // groups of 1024: 208 us a pair of steps, of 32: 90).
 //
-// Where the arrays fit the L2 caches, an eighth of the grid to each XCD instead,
-// in one order: its L2 then still holds what it stepped before (48^3 FP64 18 us a
-// pair of steps, in groups 21; 65x55x58 BF16 16 and 21).  Runs of the same length
-// for all XCDs: with powers of two, some of them idle (48x61x53 FP64 coupled A-A 57
-// us and 45, 30x300x30 F16 32 and 26).
+// Where the arrays fit half the last-level cache, an eighth of the grid to each XCD
+// instead, in one order: its L2 then still holds (a part of) what it stepped before,
+// and no range of memory is short of bandwidth.  A pair of steps, eighths / groups:
+// 48^3 FP64 25 / 30 us; F16 70^3 28 / 34; beyond the L2 caches' 32 MB F32 A-B duct
+// 50x60x55 (36 MB) 26.5 / 32, F32 box 70^3 (37) 31 / 35, FP64 A-B 61x77x53 (108)
+// 43.6 / 45.4; from there to the cache's size equal.  Runs of the same length for all
+// XCDs: with powers of two, some of them idle (48x61x53 FP64 coupled A-A 57 us and
+// 45, 30x300x30 F16 32 and 26).
 //
 // Where they do not, but are no more than some times the last-level cache, odd
 // steps run through the blocks backwards: they begin where the step before ended,
@@ -152,7 +154,7 @@ inline bool alternating(uint64_t bytes)
 // 243x205x157 F32_DEV box 682 / 625, 150x90x96 FP64 A-B duct 220 / 201.
 inline uint32_t padded_blocks(StepArgs& A, uint32_t group = 5)
 {
-	if (population_bytes(A) <= L2_BYTES) {
+	if (population_bytes(A) <= LLC_BYTES / 2) {
 		A.backwards = 0;
 		A.group = 31;
 		A.span = (A.nblocks + NXCD - 1) / NXCD;
