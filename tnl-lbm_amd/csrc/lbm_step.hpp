@@ -133,6 +133,17 @@ inline bool alternating(uint64_t bytes)
 {
 	return bytes <= 5 * LLC_BYTES;
 }
+// A-B arrays with planes of exactly 8 or 16 MiB (128^3 FP32 and FP64, 256^2 x 64 and
+// 128 F16): the same range of all 54 planes meets in the same memory channels, so a
+// step whose XCDs work side by side on one range waits for those.  An eighth of the
+// grid to each XCD and hints instead.  Two steps, side by side / so: 128^3 FP64 354 /
+// 337 us, MRT 365 / 339, FP32 187 / 180; 64x256x256 F16 197 / 181; coupled 128^3 FP64
+// 460 / 439.  (32 MiB planes 658 / 687, 12 and 20 MiB 266 / 285 and 436 / 474, 15.875
+// MiB 377 / 427, 4 MiB within the cache.)
+inline bool planes_meet(const StepArgs& A)
+{
+	return A.df1 && (A.plane_bytes == 8ull << 20 || A.plane_bytes == 16ull << 20);
+}
 // The grid for A.nblocks logical blocks.  Smaller groups where there would be
 // fewer than 16 for each XCD: the last ones keep one XCD busy alone (128x64x64,
 // groups of 1024: 208 us a pair of steps, of 32: 90).
@@ -154,7 +165,7 @@ inline bool alternating(uint64_t bytes)
 // 243x205x157 F32_DEV box 682 / 625, 150x90x96 FP64 A-B duct 220 / 201.
 inline uint32_t padded_blocks(StepArgs& A, uint32_t group = 5)
 {
-	if (population_bytes(A) <= LLC_BYTES / 2) {
+	if (population_bytes(A) <= LLC_BYTES / 2 || planes_meet(A)) {
 		A.backwards = 0;
 		A.group = 31;
 		A.span = (A.nblocks + NXCD - 1) / NXCD;
@@ -2200,7 +2211,7 @@ inline void list_shape(StepArgs& A, const uint32_t* rows, uint32_t nrows, unsign
 // 811 and 791; 192^3 FP64, 1.5 GB, equal; 256^3 F32, 1.8 GB, 1286 and 1316).
 inline bool cache_resident(const StepArgs& A, uint64_t planes = 27)
 {
-	return alternating(planes * A.plane_bytes);
+	return alternating(planes * A.plane_bytes) && ! planes_meet(A);
 }
 // Whether a step over `planes` population planes in all hints the streams that
 // no other wave touches: rows and planes start on lines, and the last-level cache
