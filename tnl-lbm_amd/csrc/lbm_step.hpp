@@ -721,11 +721,13 @@ k_aa_odd(const StepArgs A)
 			return (elem*) (sptr<PIN_ODD>(plane + row) + ys[1 + cy]);
 		}
 	};
-	// The 2-byte forms in rows take the arrays in order: where the memory serves
-	// the allocation fast their issue bounds the step (512^3 F16 4986 -> 4835 us for
-	// both steps, 512x256x384 I16 1905 -> 1866); on slower allocations both orders
-	// are within 0.5% (BF16 256^3 1%).  The wider forms, which HBM bounds alone, and
-	// the linear mapping keep the pairs' order, up to 0.7% faster there.
+	// The 2-byte forms in rows take the arrays in order: where the last-level cache or
+	// a fast allocation serves them, their issue bounds the step (one odd step, pairs'
+	// order / this: 256x256x64 F16 82 / 76 us, 256x256x100 134 / 129, 1024x512x512 I16
+	// 5050 / 4990; 512^3 F16, both steps, 4986 / 4835); on slower allocations of large
+	// boxes it is up to 1.2% slower (200x512x300 F16 628 / 635, 512^3 2870 / 2895).  The
+	// wider forms, which HBM bounds alone, and the linear mapping keep the pairs'
+	// order, up to 0.7% faster there.
 	constexpr bool WALK = ! LIN && E == 2;
 	Planes<char, PIN_ODD> in(df, pb);
 #pragma unroll
@@ -2249,8 +2251,13 @@ inline bool even_shape(StepArgs& A, uint32_t per, unsigned most, unsigned& threa
 		A.nblocks = A.nyb * (uint32_t) A.nz * (uint32_t) A.nx;  // no more blocks than one lane per site needs
 		whole = planes && (uint64_t) A.Ys * elem % 128 == 0 && (uint64_t) (A.oy + A.offy) * elem % 128 == 0;
 	}
-	// (2-byte forms, 512^3: groups of 32 blocks 1 to 2% slower than of 256)
-	const uint32_t padded = padded_blocks(A, elem == 2 ? 8 : 5);
+	// Groups of 256 blocks for the 2-byte forms on planes of a power of two from 128 MiB
+	// on, which meet in the same channels: groups of 32 / 256, us, 512^3 F16 2532 / 2419,
+	// I16 2440 / 2289, 512x512x256 F16 1222 / 1165, 1024x512x512 I16 4811 / 4605.  Other
+	// sizes are equal or slower so: 512x256x256 F16 585 / 598, 450x448x448 1722 / 1824,
+	// 640x320x320 1362 / 1397, 301x187x129 159 / 159.
+	const bool pow2 = A.plane_bytes >= 128ull << 20 && (A.plane_bytes & (A.plane_bytes - 1)) == 0;
+	const uint32_t padded = padded_blocks(A, elem == 2 && pow2 ? 8 : 5);
 	grid = padded;
 	return whole;
 }
