@@ -299,7 +299,7 @@ static int launch_reduce_macro(const MacroArgs& M, double* partial, double* out,
 // blockIdx.y is the copy, blockIdx.x an 8 KB piece of its plane, moved in units
 // of U.  Bound: HBM and the launch; the runtime's device copy took about 5 us for
 // each of the 18 planes, one after another (FP64 320^2 planes, 0.8 MB: 90 us an
-// exchange as copies, HALO_US us as this kernel).
+// exchange as copies, 19 us as this kernel).
 constexpr int HALO_COPIES = 18;
 struct HaloArgs
 {

@@ -985,26 +985,24 @@ LBM_DEV void raw_moments10(const real* f, real* m)
 }
 
 // Slot q of the site at storage coordinates (xs, ys, zs), and of site s:
-// with O32, the array of direction q as a wave-uniform base plus a 32-bit
-// per-lane byte offset formed in 32-bit arithmetic; else a 64-bit address
-// per lane. PIN keeps the base in scalar registers (one scalar-base access
-// each); it needs the call to sit where the compiler can prove the base
-// uniform, which the adjoint's branchy body does not allow.
-template <bool O32, bool PIN = true, typename E>
+// with O32, the array of direction q as a wave-uniform base, pinned in scalar
+// registers, plus a 32-bit per-lane byte offset formed in 32-bit arithmetic;
+// else a 64-bit address per lane.
+template <bool O32, typename E>
 LBM_DEV E* slot(E* base, int q, const StepArgs& A, int64_t xs, int64_t ys, int64_t zs)
 {
 	if constexpr (O32) {
 		const uint32_t i = ((uint32_t) xs * (uint32_t) A.Zs + (uint32_t) zs) * (uint32_t) A.Ys + (uint32_t) ys;
-		return at((E*) sptr<PIN>((char*) (base + q * A.XYZ)), i);
+		return at((E*) sptr<true>((char*) (base + q * A.XYZ)), i);
 	}
 	else
 		return base + q * A.XYZ + (xs * A.Zs + zs) * A.Ys + ys;
 }
-template <bool O32, bool PIN = true, typename E>
+template <bool O32, typename E>
 LBM_DEV E* slot0(E* base, int q, const StepArgs& A, int64_t s)
 {
 	if constexpr (O32)
-		return at((E*) sptr<PIN>((char*) (base + q * A.XYZ)), (uint32_t) s);
+		return at((E*) sptr<true>((char*) (base + q * A.XYZ)), (uint32_t) s);
 	else
 		return base + q * A.XYZ + s;
 }
@@ -2169,7 +2167,7 @@ static __global__ void __launch_bounds__(1024) k_reduce_final(const double* part
 // Kernels that compute every lane's coordinates (k_general, k_nse_ade, the
 // adjoint) can take the y-z plane of one x as one linear range, so that a row
 // length that is not a multiple of the block (Y = 96, say) still fills every
-// wave.  The map-free periodic kernel keeps whole rows per block.
+// wave.  (k_aa_odd and k_lean choose between the two mappings at compile time.)
 inline void linearize(StepArgs& A, unsigned& threads, unsigned& grid)
 {
 	if (A.nx == 0 || A.ny % (int32_t) threads == 0)
@@ -2211,6 +2209,11 @@ inline void list_shape(StepArgs& A, const uint32_t* rows, uint32_t nrows, unsign
 // (300x50x300 F16, 243 MB: 204 us for the two steps with them, 153 without; with
 // alternating order 128^3 FP64, 453 MB, 312 and 293; 48x320x320 FP64 slab, 1.1 GB,
 // 811 and 791; 192^3 FP64, 1.5 GB, equal; 256^3 F32, 1.8 GB, 1286 and 1316).
+// The rule takes a lattice to step alone.  Where other work between its steps takes
+// the cache, it costs what it gains and more: two lattices stepped in turn, two steps
+// of each, with hints / without: 128^3 F32 331 / 372 us, FP64 668 / 742, 160^3 FP64
+// 1344 / 1402, 256x256x100 F16 542 / 595, 256x256x200 F16 1090 / 1148 (alone 152 / 141,
+// 318 / 297, 653 / 621, 257 / 248, 528 / 501; in turn by two steps as alone).
 inline bool cache_resident(const StepArgs& A, uint64_t planes = 27)
 {
 	return alternating(planes * A.plane_bytes) && ! planes_meet(A);

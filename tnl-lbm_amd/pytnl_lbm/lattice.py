@@ -98,9 +98,11 @@ class D3Q27Lattice:
                  XYZ: int | None = None, store_range: float = 1.0, store_range_class=None, overlap=(0, 0, 0),
                  row_lists: bool = True, placement: str = "auto", placement_tries: int = 6):
         """row_lists: classify the map's rows (tnl_lbm_classify_rows) so that
-        whole-box steps run the rows of FLUID/PERIODIC (and WALL) sites
-        through lean kernels; False steps every row through the kernel with
-        all boundary codes (same results, bit for bit).
+        whole-box steps take the FLUID, PERIODIC and WALL sites through lean
+        kernels (tnl_lbm_d3q27_data.rows says where); False steps every site
+        through the kernel with all boundary codes (the same operations; the
+        compiler fuses them differently, so a step agrees to a few epsilons
+        of each array's scale, one unit of a stored 2-byte value).
 
         placement: "first" keeps the first population buffer allocated;
         "probe" times candidate buffers and keeps the fastest (up to
