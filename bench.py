@@ -605,8 +605,8 @@ def main():
     tau = 0.5015 if st == "f64" else 0.505
     head = bench_case(N, st, args.steps, args.warmup, tau=tau, store_range=0.5 if st == "i16dev" else 1.0,
                       placement=args.placement)
-    kernel = (f"k_aa_even_pair<{st.upper()},CUM> (even) / k_aa_periodic<{st.upper()},CUM> (odd)"
-              if st in ("f16dev", "bf16dev", "i16dev") else f"k_aa_periodic<{st.upper()},CUM> (even/odd)")
+    kernel = (f"k_aa_even_pair<{st.upper()},CUM> (even) / k_aa_odd<{st.upper()},CUM> (odd)"
+              if st in ("f16dev", "bf16dev", "i16dev") else f"k_aa_even<{st.upper()},CUM> (even) / k_aa_odd<{st.upper()},CUM> (odd)")
     workload = f"D3Q27 cumulant A-A {st.upper()}, {N}^3 periodic box, tau={tau}"
     out = {
         "metric": METRIC,
